@@ -577,6 +577,37 @@ int moc_sparse_dq_combine(int dtype, const void* dq_part, const int32_t* edge_u,
 /* dw f32 [E]: mode 0 sum of dst rows; modes 2/3 sum of dlog rows / w (0 where the clamp is active). */
 int moc_sparse_dw(const float* src, const float* w, const int32_t* edge_u, int mode, int rpe, int64_t E, float* dw,
                   hipStream_t stream);
+/* Per-head block choices (the FSA entry points' block_indices [B, Tq, HK, S]) as one problem:
+ * every (token, kv head) pair is a token' = token * HK + hk with G = HQ / HK query rows (q
+ * [ntok'][G][64], the same memory as [ntok][HQ][64]), every (batch, block, kv head) a plan id
+ * (b * nblk + block) * HK + hk, so one plan and one launch serve all heads
+ * (kernels-final/kernel_v4.py:213-257 sorts on the same combined key).  K / V (and dK / dV)
+ * [Bk][Tk][HK][64]; a block is KT keys, 64 or (bf16) 128, nblk = ceil(Tk / KT), the last one of a
+ * batch possibly half; edge e = token' * S + slot, rows e * G + r.  bf16 units with many rows run
+ * pipelined kernels that keep K / V operands in registers and may split a unit's rows over
+ * workgroups (f32 partials in the workspace, summed in a fixed order). */
+/* KT for these arguments (ntok = ntok'; S slots of block_size keys; mode as moc_sparse_combine), or
+ * 0 when the packed form does not apply (too many ids for the plan or rows for its indices; a
+ * per-block softmax over other blocks than 64 and 128 keys). */
+int moc_sparse_packed_block(int dtype, int64_t ntok, int G, int64_t S, int64_t Bk, int64_t Tk, int HK, int block_size,
+                            int mode, float scale);
+/* out i32 [ntok * HK * S]: plan ids of idx [ntok][heads][S] (4- or 8-byte ids, heads >= HK); -1
+ * for a choice outside [0, nblk).  per_batch: K / V per batch row of tok_per_batch tokens. */
+int moc_sparse_pack_ids(const void* idx, int idx_bytes, int64_t ntok, int64_t tok_per_batch, int heads, int HK, int S,
+                        int64_t nblk, int per_batch, int32_t* out, hipStream_t stream);
+/* moc_sparse_fwd / moc_sparse_bwd over a packed plan (o_part, lse_part, lse_row, delta_row, w,
+ * dq_part, dlog as there with ntok', HQ = rpe = G; moc_sparse_combine, _bwd_prep, _dq_combine and
+ * _dw take the same).  dk / dv blocks no edge touched are left as they are. */
+int moc_sparse_packed_fwd(int dtype, const void* q, int64_t ntok, int G, const void* k, const void* v, int64_t Bk,
+                          int64_t Tk, int HK, int KT, const int32_t* uniq, const int32_t* n_uniq,
+                          const int32_t* csr_off, const int32_t* csr_edge, int64_t max_u, int S, float scale,
+                          void* o_part, float* lse_part, hipStream_t stream);
+size_t moc_sparse_packed_bwd_workspace(int dtype, int64_t ntok, int G, int S, int KT, int64_t max_u, float scale);
+int moc_sparse_packed_bwd(int dtype, const void* q, const void* dout, int64_t ntok, int G, const void* k, const void* v,
+                          int64_t Bk, int64_t Tk, int HK, int KT, const int32_t* uniq, const int32_t* n_uniq,
+                          const int32_t* csr_off, const int32_t* csr_edge, int64_t max_u, int S, int mode,
+                          const float* lse_row, float* delta_row, const float* w, float scale, void* dk, void* dv,
+                          void* dq_part, float* dlog, void* workspace, size_t workspace_bytes, hipStream_t stream);
 /* Zeros the (chapter, kv head) blocks of dK / dV (element (t, dh) at c*cs + hk*hs + t*rs + dh,
  * heads hk0 .. hk0+nhk-1, C chapters) whose chapter is not among the plan's uniq[0 .. n_uniq):
  * moc_sparse_bwd writes every block it touches whole, so this replaces zero-initialising the

@@ -103,6 +103,13 @@ _SIGS = {
                             _I, _I, _I, _I, _P, _P, _P, _F, _P, _P, _I64, _I64, _I64, _P, _P, _P, _P]),
     "moc_sparse_dq_combine": (_I, [_I, _P, _P, _I, _I, _I64, _I, _I, _P, _P]),
     "moc_sparse_dw": (_I, [_P, _P, _P, _I, _I, _I64, _P, _P]),
+    "moc_sparse_packed_block": (_I, [_I, _I64, _I, _I64, _I64, _I64, _I, _I, _I, _F]),
+    "moc_sparse_pack_ids": (_I, [_P, _I, _I64, _I64, _I, _I, _I, _I64, _I, _P, _P]),
+    "moc_sparse_packed_fwd": (_I, [_I, _P, _I64, _I, _P, _P, _I64, _I64, _I, _I, _P, _P, _P, _P, _I64, _I, _F, _P, _P,
+                                   _P]),
+    "moc_sparse_packed_bwd_workspace": (_SZ, [_I, _I64, _I, _I, _I, _I64, _F]),
+    "moc_sparse_packed_bwd": (_I, [_I, _P, _P, _I64, _I, _P, _P, _I64, _I64, _I, _I, _P, _P, _P, _P, _I64, _I, _I, _P,
+                                   _P, _P, _F, _P, _P, _P, _P, _P, _SZ, _P]),
     "moc_sparse_zero_untouched": (_I, [_I, _P, _P, _I64, _I64, _I64, _I64, _I, _I, _P, _P, _I64, _P, _P]),
     "moc_decode_partial": (_I, [_I, _P, _I64, _I, _P, _P, _I, _I, _I, _P, _P, _P, _P, _I64, _P, _I, _F, _P, _P, _P,
                                 _P]),

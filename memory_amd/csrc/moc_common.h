@@ -350,7 +350,15 @@ int sparse_fwd_launch(int dtype, const void* q, int HQ, const void* k, const voi
                       int64_t rs, int HK, const int32_t* uniq, const int32_t* n_uniq, const int32_t* csr_off,
                       const int32_t* csr_edge, int64_t max_u, int S, int hk0, int nhk, int hq_off, int rpe,
                       float scale, const float* omega, void* o_part, float* lse_part, hipStream_t stream,
-                      const char* who, const int32_t* row_tab = nullptr);
+                      const char* who, const int32_t* row_tab = nullptr, int kvdiv = 1);
+// Its backward, arguments as moc_sparse_bwd.  kvdiv (both): > 1 for a plan over packed (chapter, kv
+// head) ids, id = chapter * kvdiv + kv head, run with HK = nhk = 1 and hk0 = 0.
+int sparse_bwd_launch(int dtype, const void* q, const void* dout, int64_t ntok, int HQ, const void* k, const void* v,
+                      int64_t cs, int64_t hs, int64_t rs, int HK, int Dh, const int32_t* uniq, const int32_t* n_uniq,
+                      const int32_t* csr_off, const int32_t* csr_edge, int64_t max_u, int S, int hk0, int nhk,
+                      int hq_off, int rpe, int mode, const float* lse_row, float* delta_row, const float* w,
+                      float scale, void* dk, void* dv, int64_t ocs, int64_t ohs, int64_t ors, void* dq_part,
+                      float* dlog, const int32_t* row_tab, hipStream_t stream, const char* who, int kvdiv);
 
 // out[i] = inv * sum_j part[j * n + i] for i < n, j < nsplit, summed in a fixed order
 // (router.hip's split-row reduction); returns a MOC_ status.

@@ -56,6 +56,14 @@ __device__ __forceinline__ void sp_load_tile(char* dst, const T* base, int64_t r
   }
 }
 
+// Element offset of a plan id's (chapter, kv head) block at strides (cs, hs).  Plans over packed
+// (chapter, kv head) ids (id = chapter * kvdiv + kv head; the launch then has one kv head of its
+// own, hk = 0) unpack the id here; kvdiv = 1 leaves id = chapter.
+__device__ __forceinline__ int64_t sp_kv_base(int gid, int hk, int kvdiv, int64_t cs, int64_t hs) {
+  const int c = gid / kvdiv;
+  return (int64_t)c * cs + (int64_t)(hk + gid - c * kvdiv) * hs;
+}
+
 // ------------------------------------------------------------------ forward
 // Partial rows (per (edge, row) outputs and dQ contributions) are kept in the data type of the
 // call: bf16 for bf16 inputs (half the bytes of the round trip through HBM), f32 for f32.
@@ -77,7 +85,8 @@ __global__ __launch_bounds__(64 * SpCfg<T>::NW) void sparse_fwd_kernel(
     const T* __restrict__ q, int HQ, const T* __restrict__ k, const T* __restrict__ v, int64_t cs, int64_t hs,
     int64_t rs, int HK, const int32_t* __restrict__ uniq, const int32_t* __restrict__ n_uniq,
     const int32_t* __restrict__ csr_off, const int32_t* __restrict__ csr_edge, int S, int hk0, int hq_off, int rpe,
-    float scale_log2, T* __restrict__ o_part, float* __restrict__ lse_part, const float* __restrict__ omega) {
+    float scale_log2, T* __restrict__ o_part, float* __restrict__ lse_part, const float* __restrict__ omega,
+    int kvdiv) {
   typedef typename Frag<T>::type F8;
   constexpr int NW = SpCfg<T>::NW, NT = 64 * NW;
   using Tile = SwzTile<T, 64>;
@@ -88,9 +97,9 @@ __global__ __launch_bounds__(64 * SpCfg<T>::NW) void sparse_fwd_kernel(
   if (u >= n_uniq[0]) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int g = lane >> 4, c16 = lane & 15;
-  const int gid = uniq[u];
-  sp_load_tile<T, NT>(sK, k + gid * cs + hk * hs, rs, tid, false);
-  sp_load_tile<T, NT>(sVt, v + gid * cs + hk * hs, rs, tid, true);
+  const int64_t kv0 = sp_kv_base(uniq[u], hk, kvdiv, cs, hs);
+  sp_load_tile<T, NT>(sK, k + kv0, rs, tid, false);
+  sp_load_tile<T, NT>(sVt, v + kv0, rs, tid, true);
   __syncthreads();
   const int G = HQ / HK;
   const int p0 = csr_off[u], p1 = csr_off[u + 1];
@@ -389,6 +398,86 @@ __global__ __launch_bounds__(64 * kCombWaves) void sparse_combine_small_kernel(
   sp_row_store(out + ((int64_t)tok * HQ + hq_off + r) * kSpDh, acc, inv, lane);
 }
 
+// The combine for at most kCombFew slots: a row of 64 dims is LPR lanes of 16 bytes each, and those
+// lanes read every slot's id, lse, weight and partial row before using any; no value crosses lanes
+// (a wave holds 64 / LPR rows, where the kernels above spend a wave and several cross-lane rounds on
+// each).  A skipped slot's row was never written: its value is dropped by a select.  Bound: HBM;
+// 262,144 rows of 8 slots (268 MB): 182 -> 75 us, dQ 101 -> 71.  With 16 slots in two chunks the
+// one-wave-per-row kernel is the faster one (52.6 against 58.4 us at 98,304 rows).
+constexpr int kCombFew = 8;
+
+// token and row-in-token of a flat row (32-bit division where the rows allow it)
+__device__ __forceinline__ void sp_split_row(int64_t row, int rpe, int64_t& tok, int& r) {
+  if (row < (int64_t)1 << 31) {
+    const uint32_t t = (uint32_t)row / (uint32_t)rpe;
+    tok = t;
+    r = (int)((uint32_t)row - t * (uint32_t)rpe);
+  } else {
+    tok = row / rpe;
+    r = (int)(row % rpe);
+  }
+}
+
+// every lane: its 16 bytes of the row (chunk ch)
+template <typename T>
+__device__ __forceinline__ void sp_chunk_store(T* __restrict__ row, const float (&acc)[SpRow16<T>::EPL], float scale,
+                                               int ch) {
+  typename SpRow16<T>::V o;
+#pragma unroll
+  for (int x = 0; x < SpRow16<T>::EPL; ++x) o[x] = from_f<T>(acc[x] * scale);
+  *reinterpret_cast<typename SpRow16<T>::V*>(row + SpRow16<T>::EPL * ch) = o;
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void sparse_combine_few_kernel(
+    const T* __restrict__ o_part, const float* __restrict__ lse_part, const int32_t* __restrict__ edge_u,
+    const float* __restrict__ w, int mode, int S, int rpe, int64_t ntok, int HQ, int hq_off, T* __restrict__ out,
+    float* __restrict__ lse_joint) {
+  using R = SpRow16<T>;
+  typedef typename R::V V;
+  const int64_t row = ((int64_t)blockIdx.x * 256 + threadIdx.x) / R::LPR;
+  const int ch = threadIdx.x % R::LPR;
+  if (row >= ntok * rpe) return;
+  int64_t tok;
+  int r;
+  sp_split_row(row, rpe, tok, r);
+  V v[kCombFew];
+  float lg[kCombFew];
+  bool ok[kCombFew];
+#pragma unroll
+  for (int i = 0; i < kCombFew; ++i) {
+    const bool in = i < S;
+    const int64_t e = tok * S + i;
+    v[i] = in ? *reinterpret_cast<const V*>(o_part + (e * rpe + r) * kSpDh + R::EPL * ch) : V{};
+    const int eu = in ? edge_u[e] : -1;
+    const float lp = in && mode != 0 ? lse_part[e * rpe + r] : 0.f;
+    const float we = in && w ? w[e] : 1.f;
+    ok[i] = in && eu >= 0;
+    lg[i] = !ok[i] ? -INFINITY : mode == 0 ? we : lp + sp_logw(mode, we);
+  }
+  float M = -INFINITY;
+#pragma unroll
+  for (int i = 0; i < kCombFew; ++i) M = fmaxf(M, lg[i]);
+  float den = 0.f, acc[R::EPL];
+#pragma unroll
+  for (int x = 0; x < R::EPL; ++x) acc[x] = 0.f;
+#pragma unroll
+  for (int i = 0; i < kCombFew; ++i) {
+    const float a = !ok[i] ? 0.f : mode == 0 ? lg[i] : M > -INFINITY ? exp2f(lg[i] - M) : 0.f;
+    den += a;
+    if (a != 0.f) {
+#pragma unroll
+      for (int x = 0; x < R::EPL; ++x) acc[x] += a * (float)v[i][x];
+    }
+  }
+  float inv = 1.f;
+  if (mode != 0) {
+    inv = den > 0.f ? 1.f / den : 0.f;
+    if (ch == 0) lse_joint[row] = den > 0.f ? M + log2f(den) : INFINITY;
+  }
+  sp_chunk_store(out + (tok * HQ + hq_off + r) * kSpDh, acc, inv, ch);
+}
+
 // ----------------------------------------------------------------- backward
 // mode 0: dwe[e*rpe + r] = dO_row . o_part[e, r]      (dL/dw_s partial per head)
 // else:   delta[row]     = dO_row . out_row
@@ -441,7 +530,7 @@ __global__ __launch_bounds__(64 * SpCfg<T>::NW, 1) void sparse_bwd_kernel(
     const int32_t* __restrict__ csr_off, const int32_t* __restrict__ csr_edge, int S, int hk0, int hq_off, int rpe,
     int mode, const float* __restrict__ lse_row, float* __restrict__ delta_row, const float* __restrict__ w,
     float scale_log2, float scale, T* __restrict__ dk, T* __restrict__ dv, int64_t ocs, int64_t ohs, int64_t ors,
-    T* __restrict__ dq_part, float* __restrict__ dlog) {
+    T* __restrict__ dq_part, float* __restrict__ dlog, int kvdiv) {
   typedef typename Frag<T>::type F8;
   constexpr int NW = SpCfg<T>::NW, NT = 64 * NW;
   using Tile = SwzTile<T, 64>;   // [key][dim] and [dim][key] tiles
@@ -458,9 +547,10 @@ __global__ __launch_bounds__(64 * SpCfg<T>::NW, 1) void sparse_bwd_kernel(
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int g = lane >> 4, c16 = lane & 15;
   const int gid = uniq[u];
-  sp_load_tile<T, NT>(sK, k + gid * cs + hk * hs, rs, tid, false);
-  sp_load_tile<T, NT>(sKt, k + gid * cs + hk * hs, rs, tid, true);
-  sp_load_tile<T, NT>(sV, v + gid * cs + hk * hs, rs, tid, false);
+  const int64_t kv0 = sp_kv_base(gid, hk, kvdiv, cs, hs);
+  sp_load_tile<T, NT>(sK, k + kv0, rs, tid, false);
+  sp_load_tile<T, NT>(sKt, k + kv0, rs, tid, true);
+  sp_load_tile<T, NT>(sV, v + kv0, rs, tid, false);
   __syncthreads();
   T* sQt = reinterpret_cast<T*>(sW[wave][0]);
   T* sDt = reinterpret_cast<T*>(sW[wave][1]);
@@ -693,8 +783,9 @@ __global__ __launch_bounds__(64 * SpCfg<T>::NW, 1) void sparse_bwd_kernel(
   // ---- cross-wave reduction of dK / dV and strided store
   __syncthreads();
   float* buf = reinterpret_cast<float*>(&sW[0][0][0]);  // NW * 3 * TB/2 bytes >= 16 KB
-  T* dkb = dk + gid * ocs + hk * ohs;
-  T* dvb = dv + gid * ocs + hk * ohs;
+  const int64_t ob = sp_kv_base(gid, hk, kvdiv, ocs, ohs);
+  T* dkb = dk + ob;
+  T* dvb = dv + ob;
   auto reduce_store = [&](f32x4 (&acc)[4][4], T* dst) {
     for (int src = 1; src < NW; ++src) {
       if (wave == src) {
@@ -750,6 +841,41 @@ __global__ __launch_bounds__(64 * kCombWaves) void sparse_dq_combine_kernel(cons
   }
   sp_groups_sum<T>(acc);
   sp_row_store(dq + ((int64_t)tok * HQ + hq_off + r) * kSpDh, acc, 1.f, lane);
+}
+
+// The same for at most kCombFew slots, lanes as in sparse_combine_few_kernel.
+template <typename T>
+__global__ __launch_bounds__(256) void sparse_dq_combine_few_kernel(const T* __restrict__ dq_part,
+                                                                    const int32_t* __restrict__ edge_u, int S, int rpe,
+                                                                    int64_t ntok, int HQ, int hq_off,
+                                                                    T* __restrict__ dq) {
+  using R = SpRow16<T>;
+  typedef typename R::V V;
+  const int64_t row = ((int64_t)blockIdx.x * 256 + threadIdx.x) / R::LPR;
+  const int ch = threadIdx.x % R::LPR;
+  if (row >= ntok * rpe) return;
+  int64_t tok;
+  int r;
+  sp_split_row(row, rpe, tok, r);
+  V v[kCombFew];
+  int eu[kCombFew];
+#pragma unroll
+  for (int i = 0; i < kCombFew; ++i) {
+    const bool in = i < S;
+    const int64_t e = tok * S + i;
+    v[i] = in ? *reinterpret_cast<const V*>(dq_part + (e * rpe + r) * kSpDh + R::EPL * ch) : V{};
+    eu[i] = in ? edge_u[e] : -1;
+  }
+  float acc[R::EPL];
+#pragma unroll
+  for (int x = 0; x < R::EPL; ++x) acc[x] = 0.f;
+#pragma unroll
+  for (int i = 0; i < kCombFew; ++i)
+    if (eu[i] >= 0) {
+#pragma unroll
+      for (int x = 0; x < R::EPL; ++x) acc[x] += (float)v[i][x];
+    }
+  sp_chunk_store(dq + (tok * HQ + hq_off + r) * kSpDh, acc, 1.f, ch);
 }
 
 // dw[e] for an edge e = token * S + s, summed over its rpe rows:
@@ -832,7 +958,7 @@ __global__ __launch_bounds__(64 * kUnitWaves) void sparse_fwd_unit_kernel(
     int64_t hs, int64_t rs, int HK, const int32_t* __restrict__ uniq, const int32_t* __restrict__ n_uniq,
     const int32_t* __restrict__ csr_off, const int32_t* __restrict__ csr_edge, int64_t max_u, int S, int hk0,
     int nhk, int hq_off, int rpe, float scale_log2, bf16* __restrict__ o_part, float* __restrict__ lse_part,
-    const float* __restrict__ omega, const int32_t* __restrict__ row_tab) {
+    const float* __restrict__ omega, const int32_t* __restrict__ row_tab, int kvdiv) {
   using Tile = SwzTile<bf16, 64>;
   __shared__ __attribute__((aligned(1024))) char sVall[kUnitWaves][64 * 64 * 2];
   const int G = HQ / HK;
@@ -848,7 +974,7 @@ __global__ __launch_bounds__(64 * kUnitWaves) void sparse_fwd_unit_kernel(
   }
   if (!unit_setup(ur, uniq, n_uniq, csr_off, hk0, nhk, G, max_u)) return;
   char* sV = sVall[threadIdx.x >> 6];
-  const int64_t kv0 = (int64_t)ur.gid * cs + (int64_t)ur.hk * hs;
+  const int64_t kv0 = sp_kv_base(ur.gid, ur.hk, kvdiv, cs, hs);
   {
     // DMA instruction i fills LDS rows 8 i .. 8 i + 7: lane l -> row 8 i + l / 8, physical chunk
     // l % 8 = logical chunk (l % 8) ^ (row & 7) of Tile::off
@@ -961,7 +1087,7 @@ __global__ __launch_bounds__(64 * kBwdWaves) void sparse_bwd_unit_kernel(
     int64_t max_u, int S, int hk0, int nhk, int hq_off, int rpe, int mode, const float* __restrict__ lse_row,
     float* __restrict__ delta_row, const float* __restrict__ w, float scale_log2, float scale, bf16* __restrict__ dk,
     bf16* __restrict__ dv, int64_t ocs, int64_t ohs, int64_t ors, bf16* __restrict__ dq_part,
-    float* __restrict__ dlog, const int32_t* __restrict__ row_tab, uint32_t qbytes) {
+    float* __restrict__ dlog, const int32_t* __restrict__ row_tab, uint32_t qbytes, int kvdiv) {
   using Tile = SwzTile<bf16, 64>;
   constexpr int kKB = 64 * 64 * 2, kRB = 32 * 64 * 2;
   __shared__ __attribute__((aligned(1024))) char sK[kKB];   // K [key][dim]
@@ -1021,7 +1147,7 @@ __global__ __launch_bounds__(64 * kBwdWaves) void sparse_bwd_unit_kernel(
   const int p0 = __builtin_amdgcn_readfirstlane(cur.p0);
   const int nrows = (__builtin_amdgcn_readfirstlane(cur.p1) - p0) * G;
   const int tab_d[2] = {cur.d0, cur.d1}, tab_c = cur.c;
-  const int64_t kv0 = (int64_t)gid * cs + (int64_t)hk * hs;
+  const int64_t kv0 = sp_kv_base(gid, hk, kvdiv, cs, hs);
   __syncthreads();   // the previous unit's dK / dV rows (staged in sK / sV) have been read back
   {
     // K and V tiles -> LDS (K the B operand of S and, transposed, of dQ; V the B operand of dPu):
@@ -1287,8 +1413,9 @@ __global__ __launch_bounds__(64 * kBwdWaves) void sparse_bwd_unit_kernel(
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  bf16* dkb = dk + (int64_t)gid * ocs + (int64_t)hk * ohs;
-  bf16* dvb = dv + (int64_t)gid * ocs + (int64_t)hk * ohs;
+  const int64_t ob = sp_kv_base(gid, hk, kvdiv, ocs, ohs);
+  bf16* dkb = dk + ob;
+  bf16* dvb = dv + ob;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int key = key0 + 8 * i + (lane >> 3), ch = lane & 7;
@@ -1365,7 +1492,7 @@ int moc::sparse_fwd_launch(int dtype, const void* q, int HQ, const void* k, cons
                            int64_t rs, int HK, const int32_t* uniq, const int32_t* n_uniq, const int32_t* csr_off,
                            const int32_t* csr_edge, int64_t max_u, int S, int hk0, int nhk, int hq_off, int rpe,
                            float scale, const float* omega, void* o_part, float* lse_part, hipStream_t stream,
-                           const char* who, const int32_t* row_tab) {
+                           const char* who, const int32_t* row_tab, int kvdiv) {
   const float sl2 = scale * 1.4426950408889634f;
   if (dtype == MOC_BF16) {
     MOC_REQUIRE(unit_kv_aligned(q, k, v, cs, hs, rs) && ((uintptr_t)o_part & 15) == 0, MOC_ERR_ARG,
@@ -1374,17 +1501,62 @@ int moc::sparse_fwd_launch(int dtype, const void* q, int HQ, const void* k, cons
     hipLaunchKernelGGL(sparse_fwd_unit_kernel, dim3((unsigned)((units + kUnitWaves - 1) / kUnitWaves)),
                        dim3(64 * kUnitWaves), 0, stream, (const bf16*)q, HQ, (const bf16*)k, (const bf16*)v, cs, hs,
                        rs, HK, uniq, n_uniq, csr_off, csr_edge, max_u, S, hk0, nhk, hq_off, rpe, sl2, (bf16*)o_part,
-                       lse_part, omega, row_tab);
+                       lse_part, omega, row_tab, kvdiv);
     return check_launch("sparse_fwd_unit_kernel");
   }
   if (dtype == MOC_F32) {
     dim3 grid((unsigned)max_u, (unsigned)nhk);
     hipLaunchKernelGGL(sparse_fwd_kernel<float>, grid, dim3(sp_threads<float>()), 0, stream, (const float*)q, HQ,
                        (const float*)k, (const float*)v, cs, hs, rs, HK, uniq, n_uniq, csr_off, csr_edge, S, hk0,
-                       hq_off, rpe, sl2, (float*)o_part, lse_part, omega);
+                       hq_off, rpe, sl2, (float*)o_part, lse_part, omega, kvdiv);
     return check_launch("sparse_fwd_kernel");
   }
   return set_error(MOC_ERR_UNSUPPORTED, "%s: dtype %d", who, dtype);
+}
+
+int moc::sparse_bwd_launch(int dtype, const void* q, const void* dout, int64_t ntok, int HQ, const void* k,
+                           const void* v, int64_t cs, int64_t hs, int64_t rs, int HK, int Dh, const int32_t* uniq,
+                           const int32_t* n_uniq, const int32_t* csr_off, const int32_t* csr_edge, int64_t max_u, int S,
+                           int hk0, int nhk, int hq_off, int rpe, int mode, const float* lse_row, float* delta_row,
+                           const float* w, float scale, void* dk, void* dv, int64_t ocs, int64_t ohs, int64_t ors,
+                           void* dq_part, float* dlog, const int32_t* row_tab, hipStream_t stream, const char* who,
+                           int kvdiv) {
+  MOC_REQUIRE(q && dout && k && v && uniq && n_uniq && csr_off && csr_edge && lse_row && delta_row && dk && dv &&
+                  dq_part,
+              MOC_ERR_ARG, "%s: null pointer", who);
+  MOC_REQUIRE(Dh == kSpDh, MOC_ERR_UNSUPPORTED, "%s: head_dim %d (needs 64)", who, Dh);
+  MOC_REQUIRE(mode >= 0 && mode <= 3 && (mode == 1 || w), MOC_ERR_ARG, "%s: mode %d / weights", who, mode);
+  MOC_REQUIRE(HQ > 0 && HK > 0 && HQ % HK == 0 && nhk > 0 && hk0 >= 0 && hk0 + nhk <= HK && S > 0, MOC_ERR_ARG,
+              "%s: bad heads", who);
+  if (max_u == 0 || ntok == 0) return MOC_OK;
+  dim3 grid((unsigned)max_u, (unsigned)nhk);
+  const float sl2 = scale * 1.4426950408889634f;
+  if (dtype == MOC_BF16) {
+    MOC_REQUIRE(unit_kv_aligned(q, k, v, cs, hs, rs) && ((uintptr_t)dout & 15) == 0 && ((uintptr_t)dq_part & 15) == 0 &&
+                    ((uintptr_t)dk & 15) == 0 && ((uintptr_t)dv & 15) == 0 && ocs % 8 == 0 && ohs % 8 == 0 &&
+                    ors % 8 == 0,
+                MOC_ERR_ARG,
+                "%s: bf16 needs 16-byte aligned q/dout/k/v/dq_part/dk/dv and strides that are multiples of 8", who);
+    // q / dout rows are moved by bounded buffer loads (rows past a unit read zeros from offsets
+    // past the buffer)
+    const int64_t qbytes = ntok * HQ * kSpDh * 2;
+    MOC_REQUIRE(qbytes < ((int64_t)1 << 32) - 16, MOC_ERR_UNSUPPORTED,
+                "%s: q / dout of %lld bytes (bf16 needs < 4 GiB)", who, (long long)qbytes);
+    const int64_t units = max_u * nhk;
+    const int64_t wgs = min(units, (int64_t)kBwdPerCU * sp_cus());
+    hipLaunchKernelGGL(sparse_bwd_unit_kernel, dim3((unsigned)wgs), dim3(64 * kBwdWaves), 0, stream, (const bf16*)q, (const bf16*)dout, HQ, (const bf16*)k,
+                       (const bf16*)v, cs, hs, rs, HK, uniq, n_uniq, csr_off, csr_edge, max_u, S, hk0, nhk, hq_off,
+                       rpe, mode, lse_row, delta_row, w, sl2, scale, (bf16*)dk, (bf16*)dv, ocs, ohs, ors,
+                       (bf16*)dq_part, dlog, row_tab, (uint32_t)qbytes, kvdiv);
+    return check_launch("sparse_bwd_unit_kernel");
+  } else if (dtype == MOC_F32)
+    hipLaunchKernelGGL(sparse_bwd_kernel<float>, grid, dim3(sp_threads<float>()), 0, stream, (const float*)q,
+                       (const float*)dout, HQ, (const float*)k, (const float*)v, cs, hs, rs, HK, uniq, n_uniq,
+                       csr_off, csr_edge, S, hk0, hq_off, rpe, mode, lse_row, delta_row, w, sl2, scale, (float*)dk,
+                       (float*)dv, ocs, ohs, ors, (float*)dq_part, dlog, kvdiv);
+  else
+    return set_error(MOC_ERR_UNSUPPORTED, "%s: dtype %d", who, dtype);
+  return check_launch("sparse_bwd_kernel");
 }
 
 extern "C" {
@@ -1419,13 +1591,22 @@ int moc_sparse_combine(int dtype, const void* o_part, const float* lse_part, con
   // few rows (decode): latency-bound, every load of a row in one round; many rows (token
   // routing over a batch): throughput-bound, the lighter streaming kernel keeps more rows resident
   const bool small = S <= 4 * kCombSmallPerGroup && rows <= 16384;
+  const bool few = S <= kCombFew;   // LPR lanes per row (8 for bf16, 16 for f32) instead of a wave
+  if (few) {
+    const int64_t per = dtype == MOC_F32 ? 16 : 32;
+    grid = dim3((unsigned)((rows + per - 1) / per));
+  }
 #define SC(KERN, TT)                                                                                                  \
   hipLaunchKernelGGL(KERN<TT>, grid, dim3(64 * kCombWaves), 0, stream, (const TT*)o_part, lse_part, edge_u, w, mode, S, \
                      rpe, ntok, HQ, hq_off, (TT*)out, lse_joint)
   if (dtype == MOC_BF16) {
-    if (small) SC(sparse_combine_small_kernel, bf16); else SC(sparse_combine_kernel, bf16);
+    if (few) SC(sparse_combine_few_kernel, bf16);
+    else if (small) SC(sparse_combine_small_kernel, bf16);
+    else SC(sparse_combine_kernel, bf16);
   } else if (dtype == MOC_F32) {
-    if (small) SC(sparse_combine_small_kernel, float); else SC(sparse_combine_kernel, float);
+    if (few) SC(sparse_combine_few_kernel, float);
+    else if (small) SC(sparse_combine_small_kernel, float);
+    else SC(sparse_combine_kernel, float);
   } else {
     return set_error(MOC_ERR_UNSUPPORTED, "moc_sparse_combine: dtype %d", dtype);
   }
@@ -1456,43 +1637,9 @@ int moc_sparse_bwd(int dtype, const void* q, const void* dout, int64_t ntok, int
                    int hq_off, int rpe, int mode, const float* lse_row, float* delta_row, const float* w,
                    float scale, void* dk, void* dv, int64_t ocs, int64_t ohs, int64_t ors, void* dq_part,
                    float* dlog, const int32_t* row_tab, hipStream_t stream) {
-  MOC_REQUIRE(q && dout && k && v && uniq && n_uniq && csr_off && csr_edge && lse_row && delta_row && dk && dv &&
-                  dq_part,
-              MOC_ERR_ARG, "moc_sparse_bwd: null pointer");
-  MOC_REQUIRE(Dh == kSpDh, MOC_ERR_UNSUPPORTED, "moc_sparse_bwd: head_dim %d (needs 64)", Dh);
-  MOC_REQUIRE(mode >= 0 && mode <= 3 && (mode == 1 || w), MOC_ERR_ARG, "moc_sparse_bwd: mode %d / weights", mode);
-  MOC_REQUIRE(HQ > 0 && HK > 0 && HQ % HK == 0 && nhk > 0 && hk0 >= 0 && hk0 + nhk <= HK && S > 0, MOC_ERR_ARG,
-              "moc_sparse_bwd: bad heads");
-  if (max_u == 0 || ntok == 0) return MOC_OK;
-  dim3 grid((unsigned)max_u, (unsigned)nhk);
-  const float sl2 = scale * 1.4426950408889634f;
-  if (dtype == MOC_BF16) {
-    MOC_REQUIRE(unit_kv_aligned(q, k, v, cs, hs, rs) && ((uintptr_t)dout & 15) == 0 && ((uintptr_t)dq_part & 15) == 0 &&
-                    ((uintptr_t)dk & 15) == 0 && ((uintptr_t)dv & 15) == 0 && ocs % 8 == 0 && ohs % 8 == 0 &&
-                    ors % 8 == 0,
-                MOC_ERR_ARG,
-                "moc_sparse_bwd: bf16 needs 16-byte aligned q/dout/k/v/dq_part/dk/dv and strides that are "
-                "multiples of 8");
-    // q / dout rows are moved by bounded buffer loads (rows past a unit read zeros from offsets
-    // past the buffer)
-    const int64_t qbytes = ntok * HQ * kSpDh * 2;
-    MOC_REQUIRE(qbytes < ((int64_t)1 << 32) - 16, MOC_ERR_UNSUPPORTED,
-                "moc_sparse_bwd: q / dout of %lld bytes (bf16 needs < 4 GiB)", (long long)qbytes);
-    const int64_t units = max_u * nhk;
-    const int64_t wgs = min(units, (int64_t)kBwdPerCU * sp_cus());
-    hipLaunchKernelGGL(sparse_bwd_unit_kernel, dim3((unsigned)wgs), dim3(64 * kBwdWaves), 0, stream, (const bf16*)q, (const bf16*)dout, HQ, (const bf16*)k,
-                       (const bf16*)v, cs, hs, rs, HK, uniq, n_uniq, csr_off, csr_edge, max_u, S, hk0, nhk, hq_off,
-                       rpe, mode, lse_row, delta_row, w, sl2, scale, (bf16*)dk, (bf16*)dv, ocs, ohs, ors,
-                       (bf16*)dq_part, dlog, row_tab, (uint32_t)qbytes);
-    return check_launch("sparse_bwd_unit_kernel");
-  } else if (dtype == MOC_F32)
-    hipLaunchKernelGGL(sparse_bwd_kernel<float>, grid, dim3(sp_threads<float>()), 0, stream, (const float*)q,
-                       (const float*)dout, HQ, (const float*)k, (const float*)v, cs, hs, rs, HK, uniq, n_uniq,
-                       csr_off, csr_edge, S, hk0, hq_off, rpe, mode, lse_row, delta_row, w, sl2, scale, (float*)dk,
-                       (float*)dv, ocs, ohs, ors, (float*)dq_part, dlog);
-  else
-    return set_error(MOC_ERR_UNSUPPORTED, "moc_sparse_bwd: dtype %d", dtype);
-  return check_launch("sparse_bwd_kernel");
+  return moc::sparse_bwd_launch(dtype, q, dout, ntok, HQ, k, v, cs, hs, rs, HK, Dh, uniq, n_uniq, csr_off, csr_edge,
+                                max_u, S, hk0, nhk, hq_off, rpe, mode, lse_row, delta_row, w, scale, dk, dv, ocs, ohs,
+                                ors, dq_part, dlog, row_tab, stream, "moc_sparse_bwd", 1);
 }
 
 int moc_sparse_dq_combine(int dtype, const void* dq_part, const int32_t* edge_u, int S, int rpe, int64_t ntok,
@@ -1502,15 +1649,19 @@ int moc_sparse_dq_combine(int dtype, const void* dq_part, const int32_t* edge_u,
               "moc_sparse_dq_combine: dq_part and dq must be 16-byte aligned");
   const int64_t rows = ntok * rpe;
   if (rows == 0) return MOC_OK;
-  dim3 grid((unsigned)((rows + kCombWaves - 1) / kCombWaves));
-  if (dtype == MOC_BF16)
-    hipLaunchKernelGGL(sparse_dq_combine_kernel<bf16>, grid, dim3(64 * kCombWaves), 0, stream, (const bf16*)dq_part, edge_u, S, rpe, ntok, HQ,
-                       hq_off, (bf16*)dq);
-  else if (dtype == MOC_F32)
-    hipLaunchKernelGGL(sparse_dq_combine_kernel<float>, grid, dim3(64 * kCombWaves), 0, stream, (const float*)dq_part, edge_u, S, rpe, ntok, HQ,
-                       hq_off, (float*)dq);
-  else
-    return set_error(MOC_ERR_UNSUPPORTED, "moc_sparse_dq_combine: dtype %d", dtype);
+  MOC_REQUIRE(dtype == MOC_BF16 || dtype == MOC_F32, MOC_ERR_UNSUPPORTED, "moc_sparse_dq_combine: dtype %d", dtype);
+  const bool few = S <= kCombFew;
+  const int64_t per = !few ? kCombWaves : dtype == MOC_F32 ? 16 : 32;   // rows per workgroup
+  dim3 grid((unsigned)((rows + per - 1) / per));
+#define SD(KERN, TT)                                                                                             \
+  hipLaunchKernelGGL(KERN<TT>, grid, dim3(64 * kCombWaves), 0, stream, (const TT*)dq_part, edge_u, S, rpe, ntok, \
+                     HQ, hq_off, (TT*)dq)
+  if (dtype == MOC_BF16) {
+    if (few) SD(sparse_dq_combine_few_kernel, bf16); else SD(sparse_dq_combine_kernel, bf16);
+  } else {
+    if (few) SD(sparse_dq_combine_few_kernel, float); else SD(sparse_dq_combine_kernel, float);
+  }
+#undef SD
   return check_launch("sparse_dq_combine_kernel");
 }
 

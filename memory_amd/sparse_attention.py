@@ -227,6 +227,103 @@ class _FSAFunction(torch.autograd.Function):
         return dq, dk, dv, dw, None, None, None
 
 
+class _PackedFSA(torch.autograd.Function):
+    """Sparse attention over per-head block choices as one problem (include/moc.h, the packed
+    entry points): every (token, kv head) is a token of G query rows, every (batch, block of kt
+    keys, kv head) an id of one plan, so all heads share each launch.
+
+    idx (B, Tq, >= HK, S) int32 / int64 block ids of kt keys; w (B, Tq, HK, S), (B, Tq, S) or None."""
+
+    @staticmethod
+    def forward(ctx, q, k, v, w, idx, mode, scale, kt):
+        B, Tq, HQ, D = q.shape
+        Bk, Tk, HK = k.shape[:3]
+        G, S = HQ // HK, idx.shape[-1]
+        ntok, nblk = B * Tq * HK, -(-Tk // kt)
+        dev, dt = q.device, L.dtype_code(q.dtype)
+        st = stream_ptr(dev)
+        q, k, v = q.contiguous(), k.to(q.dtype).contiguous(), v.to(q.dtype).contiguous()
+        idx = idx.contiguous()
+        ids = torch.empty(ntok * S, device=dev, dtype=torch.int32)
+        call("moc_sparse_pack_ids", ptr(idx), idx.element_size(), B * Tq, Tq, idx.shape[2], HK, S, nblk,
+             1 if Bk > 1 else 0, ptr(ids), st)
+        plan = ops.chapter_plan(ids, Bk * nblk * HK)
+        wf = None
+        if w is not None:
+            wf = w.float() if w.dim() == 4 else w.float().unsqueeze(2).expand(B, Tq, HK, S)
+            wf = wf.contiguous()
+        o_part = torch.empty(ntok * S * G, D, device=dev, dtype=q.dtype)
+        lse_part = torch.empty(ntok * S * G, device=dev, dtype=torch.float32)
+        call("moc_sparse_packed_fwd", dt, ptr(q), ntok, G, ptr(k), ptr(v), Bk, Tk, HK, kt, ptr(plan.uniq),
+             ptr(plan.n_uniq), ptr(plan.csr_off), ptr(plan.csr_edge), plan.max_u, S, scale, ptr(o_part), ptr(lse_part),
+             st)
+        out = torch.empty_like(q)
+        lse_joint = None if mode == 0 else torch.empty(ntok * G, device=dev, dtype=torch.float32)
+        call("moc_sparse_combine", dt, ptr(o_part), ptr(lse_part), ptr(plan.edge_u), ptr(wf), mode, S, G, ntok, G, 0,
+             ptr(out), ptr(lse_joint), st)
+        ctx.save_for_backward(q, k, v, out, wf, lse_part if mode == 0 else lse_joint)
+        ctx.plan, ctx.cfg = plan, (mode, scale, kt, S, None if w is None else w.dim(), None if w is None else w.dtype)
+        return out
+
+    @staticmethod
+    def backward(ctx, dout):
+        q, k, v, out, wf, lrow = ctx.saved_tensors
+        mode, scale, kt, S, wdim, wdt = ctx.cfg
+        plan = ctx.plan
+        B, Tq, HQ, D = q.shape
+        Bk, Tk, HK = k.shape[:3]
+        G, ntok = HQ // HK, B * Tq * HK
+        dev, dt = q.device, L.dtype_code(q.dtype)
+        st = stream_ptr(dev)
+        dout = dout.to(q.dtype).contiguous()
+        dk, dv = torch.zeros_like(k), torch.zeros_like(v)
+        if mode == 0:
+            drow = torch.empty(ntok * S * G, device=dev, dtype=torch.float32)
+        else:
+            drow = torch.empty(ntok * G, device=dev, dtype=torch.float32)
+            call("moc_sparse_bwd_prep", dt, ptr(dout), ptr(out), None, ptr(plan.edge_u), mode, S, G, ntok, G, 0,
+                 ptr(drow), st)
+        dq_part = torch.empty(ntok * S * G, D, device=dev, dtype=q.dtype)
+        dlog = torch.empty(ntok * S * G, device=dev, dtype=torch.float32) if mode in (2, 3) else None
+        ws_bytes = L.query("moc_sparse_packed_bwd_workspace", dt, ntok, G, S, kt, plan.max_u, scale)
+        ws = torch.empty(ws_bytes, device=dev, dtype=torch.uint8) if ws_bytes else None
+        call("moc_sparse_packed_bwd", dt, ptr(q), ptr(dout), ntok, G, ptr(k), ptr(v), Bk, Tk, HK, kt, ptr(plan.uniq),
+             ptr(plan.n_uniq), ptr(plan.csr_off), ptr(plan.csr_edge), plan.max_u, S, mode, ptr(lrow), ptr(drow), ptr(wf),
+             scale, ptr(dk), ptr(dv), ptr(dq_part), ptr(dlog), ptr(ws), ws_bytes, st)
+        dq = torch.empty_like(q)
+        call("moc_sparse_dq_combine", dt, ptr(dq_part), ptr(plan.edge_u), S, G, ntok, G, 0, ptr(dq), st)
+        dw = None
+        if mode != 1:
+            dw = torch.empty(B, Tq, HK, S, device=dev, dtype=torch.float32)
+            call("moc_sparse_dw", ptr(drow if mode == 0 else dlog), ptr(wf), ptr(plan.edge_u), mode, G, ntok * S,
+                 ptr(dw), st)
+            if wdim == 3:    # the weights of a token serve every kv head
+                dw = dw.sum(2)
+            dw = dw.to(wdt)
+        return dq, dk, dv, dw, None, None, None, None
+
+
+def _packed_block(q, k, v, w, idx, mode: int, scale: float, block_size: int) -> int:
+    """Keys per unit (64 or 128) when the call runs as one packed problem, else 0: the segments of
+    _FSAFunction, one per kv head, which also report what a call has wrong."""
+    if not (q.is_cuda and q.dim() == 4 and k.dim() == 4 and idx.dim() == 4 and k.shape == v.shape
+            and q.dtype in (torch.float32, torch.bfloat16)):
+        return 0
+    B, Tq, HQ, D = q.shape
+    Bk, Tk, HK, Dk = k.shape
+    if not (D == Dk == 64 and HK > 0 and HQ % HK == 0 and Tk % BLOCK == 0 and Bk in (1, B) and k.is_cuda and v.is_cuda
+            and idx.is_cuda and idx.shape[:2] == (B, Tq) and idx.shape[2] >= HK and idx.shape[3] > 0
+            and idx.dtype in (torch.int32, torch.int64) and idx.numel() > 0):
+        return 0
+    if w is None:
+        if mode != 1:
+            return 0
+    elif not (w.is_cuda and tuple(w.shape) in ((B, Tq, HK, idx.shape[3]), (B, Tq, idx.shape[3]))):
+        return 0
+    return int(L.query("moc_sparse_packed_block", L.dtype_code(q.dtype), B * Tq * HK, HQ // HK, idx.shape[3], Bk, Tk, HK,
+                       int(block_size), mode, float(scale)))
+
+
 def _check_common(cu_seqlens_q, cu_seqlens_k, disable_causal_mask, block_size):
     if (cu_seqlens_q is None) != (cu_seqlens_k is None):
         raise ValueError("cu_seqlens_q and cu_seqlens_k are given together")
@@ -246,17 +343,22 @@ def _fsa(q, k, v, w, idx, mode: int, scale: float, block_size: int):
     over the blocks, the block weight's gradient the sum of its sub-blocks' (autograd of the
     repeat), and a block reaching past the keys has its missing sub-blocks skipped as out of range
     (the reference masks those keys).  fp16 inputs run the fp32 kernels (exact widening), the
-    output rounded back to fp16."""
-    m = int(block_size) // BLOCK
+    output rounded back to fp16.  Per-head choices run as one packed problem (_PackedFSA), whose
+    units may take 128 keys of a block at once."""
+    half = q.dtype == torch.float16
+    if half:
+        q, k, v = q.float(), k.float(), v.float()
+    kt = _packed_block(q, k, v, w, idx, mode, scale, block_size)
+    m = int(block_size) // (kt or BLOCK)
     if m > 1:
         sub = torch.arange(m, device=idx.device, dtype=idx.dtype)
         idx = (idx.unsqueeze(-1) * m + sub).flatten(-2)    # negative ids stay negative
         if w is not None:
             w = w.repeat_interleave(m, dim=-1)
-    half = q.dtype == torch.float16
-    if half:
-        q, k, v = q.float(), k.float(), v.float()
-    out = _FSAFunction.apply(q, k, v, w, idx, mode, scale)
+    if kt:
+        out = _PackedFSA.apply(q, k, v, w, idx, mode, float(scale), kt)
+    else:
+        out = _FSAFunction.apply(q, k, v, w, idx, mode, scale)
     return out.to(torch.float16) if half else out
 
 
@@ -351,7 +453,7 @@ def FSA_topk_sparse_attention_weighted_bthd(q_bthd, k_bthd, v_bthd, block_indice
             term = o.float() * ws.float()
             out = term if out is None else out + term
         return out.to(q_bthd.dtype).reshape(q_bthd.shape)
-    if m == 1:
+    if m == 1 or _packed_block(q_bthd, k_bthd, v_bthd, w, idx, 0, scale, block_size):
         return _fsa(q_bthd, k_bthd, v_bthd, w, idx, 0, scale, block_size)
     out = None
     for sl in range(idx.shape[-1]):

@@ -1,0 +1,120 @@
+"""The packed form of the FSA entry points (per-head block choices as one plan) against a float64
+reference, at the sizes where its kernels can go wrong: units of 64 and 128 keys, a half last block,
+one to 16 query rows per edge, row counts around the 32- / 64-row steps, units split over several
+workgroups, ids out of range in either id type; and the segments it replaces on the same inputs."""
+
+import pytest
+import torch
+
+from helpers import assert_parity, gen
+
+pytestmark = pytest.mark.gpu
+
+
+def _reference(q, k, v, idx, w, mode, BS, scale):
+    """sum over the chosen blocks in float64; a block past the keys keeps the keys inside."""
+    B, Tq, HQ, _ = q.shape
+    Tk, HK = k.shape[1], k.shape[2]
+    S, G = idx.shape[-1], HQ // HK
+    rows = idx.unsqueeze(-1) * BS + torch.arange(BS)                     # (B, Tq, HK, S, BS)
+    ok = (idx >= 0).unsqueeze(-1) & (rows < Tk) & (rows >= 0)
+    rows = torch.where(ok, rows, torch.zeros_like(rows))
+    out = []
+    for b in range(B):
+        kb = k[b].permute(1, 0, 2)                                       # (HK, Tk, 64)
+        vb = v[b].permute(1, 0, 2)
+        h = torch.arange(HK).view(1, HK, 1, 1)
+        kk, vv = kb[h, rows[b]], vb[h, rows[b]]                          # (Tq, HK, S, BS, 64)
+        s = torch.einsum("thgd,thsjd->thgsj", q[b].view(Tq, HK, G, 64), kk) * scale
+        s = s.masked_fill(~ok[b].unsqueeze(2), float("-inf"))
+        wb = None if w is None else (w[b] if w.dim() == 4 else w[b].unsqueeze(1).expand(Tq, HK, S))
+        if mode == 0:
+            p = torch.softmax(s, -1).nan_to_num(0.0) * wb.view(Tq, HK, 1, S, 1)
+        else:
+            if mode == 3:
+                s = s + torch.log(wb.clamp_min(1e-20)).view(Tq, HK, 1, S, 1)
+            e = torch.exp(s - s.amax((-1, -2), keepdim=True).clamp_min(-1e30))
+            if mode == 2:
+                e = e * wb.clamp_min(0).view(Tq, HK, 1, S, 1)
+            p = e / e.sum((-1, -2), keepdim=True).clamp_min(1e-300)
+        out.append(torch.einsum("thgsj,thsjd->thgd", p, vv).reshape(Tq, HQ, 64))
+    return torch.stack(out)
+
+
+# (B, Tq, HQ, HK, Tk, S, BS): a few rows per unit; G = 16 on 1.5 blocks of 128 (units split over
+# workgroups, a half last block); G = 1, 33 rows past a step; G = 3, three 64-key blocks of 192; a
+# batch of shared keys is covered by Bk = 1 below
+CASES = [(1, 33, 3, 1, 320, 2, 64), (2, 150, 16, 1, 192, 2, 128), (1, 129, 4, 4, 192, 3, 64),
+         (2, 65, 6, 2, 576, 2, 192), (1, 400, 8, 2, 384, 2, 128), (1, 300, 12, 12, 256, 4, 64)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("mode", [0, 1, 2, 3])
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_packed_against_float64(gpu_device, dtype, mode, case):
+    from memory_amd import sparse_attention as SA
+    B, Tq, HQ, HK, Tk, S, BS = CASES[case]
+    print(f"packed {CASES[case]} mode={mode} {dtype}", flush=True)
+    dev = gpu_device
+    g = gen(500 + 10 * case + mode)
+    M = -(-Tk // BS)
+    q, dO = (torch.randn(B, Tq, HQ, 64, generator=g) for _ in range(2))
+    Bk = 1 if case == 4 else B
+    k, v = (torch.randn(Bk, Tk, HK, 64, generator=g) for _ in range(2))
+    idx = torch.rand(B, Tq, HK, M, generator=g).argsort(-1)[..., :S]
+    if idx.shape[-1] < S:
+        S = idx.shape[-1]
+    if mode != 0 and S > 1:     # skipped slots: below, past the end, and far past 32 bits
+        idx[:, ::5, :, 0] = -1
+        idx[:, 1::7, :, 1] = M
+    wide = case % 2 == 1
+    dev_idx = idx.clone()
+    if wide and mode != 0 and S > 1:
+        dev_idx[:, 1::7, :, 1] = 2 ** 40
+    w = None
+    if mode == 2:
+        w = torch.rand(B, Tq, HK, S, generator=g) + 0.05
+    elif mode in (0, 3):
+        w = torch.softmax(torch.randn(B, Tq, S, generator=g), -1)
+    scale = 0.2
+    r = [t.to(dtype).double().requires_grad_(True) for t in (q, k, v)]
+    rw = None if w is None else w.double().requires_grad_(True)
+    ref = _reference(r[0], r[1].expand(B, -1, -1, -1), r[2].expand(B, -1, -1, -1), idx, rw, mode, BS, scale)
+    (ref * dO.to(dtype).double()).sum().backward()
+
+    def run():
+        t = [x.to(dev, dtype).requires_grad_(True) for x in (q, k, v)]
+        tw = None if w is None else w.to(dev).requires_grad_(True)
+        di = dev_idx.to(dev, torch.int64 if wide else torch.int32)
+        kw = dict(softmax_scale=scale, disable_causal_mask=True)
+        if mode == 0:
+            out = SA.FSA_topk_sparse_attention_weighted_bthd(*t, di, tw, BS, **kw)
+        elif mode == 3:
+            out = SA.FSA_topk_sparse_attention_weighted_joint_bias_bthd(*t, di, tw, BS, **kw)
+        else:
+            out = SA.FSA_topk_sparse_attention_bthd(*t, di, BS, block_weights_bths=tw, **kw)
+        out.backward(dO.to(dev, dtype))
+        return [out.detach()] + [x.grad for x in t] + ([] if tw is None else [tw.grad])
+
+    got = run()
+    names = ["out", "dq", "dk", "dv", "dw"]
+    want = [ref.detach()] + [x.grad for x in r] + ([] if rw is None else [rw.grad])
+    for n, a, b in zip(names, got, want):
+        assert_parity(a, b, dtype, n)
+    for n, a, b in zip(names, got, run()):      # fixed-order sums: the same bits again
+        assert torch.equal(a, b), n
+
+
+@pytest.mark.parametrize("scale", [0.125, 0.0, -0.125])
+def test_packed_scale_signs(gpu_device, scale):
+    """A softmax scale of any sign gives what the segments give (the pipelined kernels take a
+    positive one; the others stay on the one-wave-per-unit kernels)."""
+    from memory_amd import sparse_attention as SA
+    dev = gpu_device
+    g = gen(77)
+    q, k, v = (torch.randn(1, n, h, 64, generator=g).to(dev, torch.bfloat16) for n, h in ((256, 8), (256, 2), (256, 2)))
+    idx = torch.rand(1, 256, 2, 2, generator=g).argsort(-1).to(dev, torch.int32)
+    out = SA.FSA_topk_sparse_attention_bthd(q, k, v, idx, 128, softmax_scale=scale, disable_causal_mask=True)
+    seg = SA._FSAFunction.apply(q, k, v, None, (idx.unsqueeze(-1) * 2 + torch.arange(2, device=dev)).flatten(-2).int(), 1,
+                                scale)
+    assert_parity(out, seg, torch.bfloat16, f"scale {scale}")
