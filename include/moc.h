@@ -359,6 +359,16 @@ int moc_seq_layer_timing_read(double* total_ms, int32_t* launches, int32_t* drop
 int moc_xattn_fwd(int dtype, const void* q, const void* k_tiles, const void* v_tiles, int64_t kv_span, int64_t su,
                   int sh, int st, const int32_t* slot_u, const float* omega, int64_t B, int64_t L, int H, int HK, int Dh, int T,
                   int NS, float scale, void* out, float* lse, hipStream_t stream);
+/* The same with a workspace for small grids: where one workgroup per (sequence, head, 128 queries)
+ * leaves most of the chip idle, the slots of a row are split over several workgroups whose f32
+ * partial rows are merged (or, for dq, added) in split order.  workspace of at least
+ * moc_xattn_split_workspace bytes (0: these sizes are not split), 16-byte aligned; NULL runs
+ * unsplit.  The same size serves moc_xattn_bwd_dq_delta_split. */
+size_t moc_xattn_split_workspace(int dtype, int64_t B, int64_t L, int H, int NS);
+int moc_xattn_fwd_split(int dtype, const void* q, const void* k_tiles, const void* v_tiles, int64_t kv_span,
+                        int64_t su, int sh, int st, const int32_t* slot_u, const float* omega, int64_t B, int64_t L,
+                        int H, int HK, int Dh, int T, int NS, float scale, void* out, float* lse, void* workspace,
+                        size_t workspace_bytes, hipStream_t stream);
 /* The attention weights of that forward (MemoryCrossAttention.forward with return_attn_weights,
  * memory_transformer/memory_attention.py:437-447: softmax(q k^T * scale) over each sequence's
  * NS * T selected, omega-weighted keys): weights [B, H, L, NS * T] (dtype), column c * T + j for
@@ -392,6 +402,12 @@ int moc_xattn_bwd_dq_delta(int dtype, const void* q, const void* k_tiles, const 
                            int64_t su, int sh, int st, const int32_t* slot_u, const float* omega, const void* out,
                            const void* dout, const float* lse, float* delta, int64_t B, int64_t L, int H, int HK, int Dh,
                            int T, int NS, float scale, void* dq, hipStream_t stream);
+/* moc_xattn_bwd_dq_delta with the workspace of moc_xattn_fwd_split. */
+int moc_xattn_bwd_dq_delta_split(int dtype, const void* q, const void* k_tiles, const void* v_tiles, int64_t kv_span,
+                                 int64_t su, int sh, int st, const int32_t* slot_u, const float* omega,
+                                 const void* out, const void* dout, const float* lse, float* delta, int64_t B,
+                                 int64_t L, int H, int HK, int Dh, int T, int NS, float scale, void* dq,
+                                 void* workspace, size_t workspace_bytes, hipStream_t stream);
 /* dK/dV per edge (edge e = b * NS + slot): dkv_edge [B * NS * T][2 * HK * Dh] (dtype) holds for
  * the chapter in slot `slot` of sequence b the rows [dL/dk (all kv heads) | dL/dv], where
  * dL/dk, dL/dv are gradients w.r.t. the unweighted projected keys/values (omega folded in).

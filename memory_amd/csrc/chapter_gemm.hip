@@ -863,6 +863,11 @@ int cg_check(const char* who, int64_t ldx, int N, int K, int64_t max_u, int64_t 
   return MOC_OK;
 }
 
+// Few chapters (a prompt's own, a dense memory): 128-row x 256-feature tiles, two k-stages ahead, where
+// they fit one round of the grid.  A round of them is half as long as one of the wide tiles (65 chapters,
+// 1,536 features, K = 768: 198 tiles in 20 us against 66 tiles of 256 x 384 in 33 us).
+bool cg_narrow(int64_t max_u, int N) { return (max_u + 1) / 2 * (N / 256) <= cg_grid(); }
+
 // workgroups per output tile of the weight gradients: fill `budget` CUs (256: the chip), but give
 // each at least 8 row blocks
 int cg_wgrad_splits(int tiles, int64_t blocks, int budget = 256) {
@@ -921,12 +926,19 @@ int moc_chapter_project(const void* rows, int64_t ld, int gather, const int32_t*
   hipLaunchKernelGGL((chapter_gemm_kernel<SRC, CG_DST_CONTIG, bf16, 256, kCgDepth256, MOC_NORM_NONE, BN>), grid,       \
                      dim3(kCgThreads), 0, stream, (const bf16*)rows, nullptr, ld, uniq, n_uniq, nullptr, nullptr,    \
                      max_u, (const bf16*)w, N, K, (bf16*)y, ldy, max_u * 64, max_u * 64, CgNorm{})
+#define MOC_CGPN(SRC)                                                                                                \
+  hipLaunchKernelGGL((chapter_gemm_kernel<SRC, CG_DST_CONTIG, bf16, 128, kCgDepth128>), grid, dim3(kCgThreads), 0,  \
+                     stream, (const bf16*)rows, nullptr, ld, uniq, n_uniq, nullptr, nullptr, max_u, (const bf16*)w, \
+                     N, K, (bf16*)y, ldy, max_u * 64, max_u * 64, CgNorm{})
   const bool wide = N % 384 == 0;
-  if (gather) {
+  if (cg_narrow(max_u, N)) {
+    if (gather) MOC_CGPN(CG_SRC_GATHER); else MOC_CGPN(CG_SRC_CONTIG);
+  } else if (gather) {
     if (wide) MOC_CGP(CG_SRC_GATHER, 384); else MOC_CGP(CG_SRC_GATHER, 256);
   } else {
     if (wide) MOC_CGP(CG_SRC_CONTIG, 384); else MOC_CGP(CG_SRC_CONTIG, 256);
   }
+#undef MOC_CGPN
 #undef MOC_CGP
   return check_launch("chapter_gemm_kernel(project)");
 }
@@ -945,7 +957,7 @@ int moc_chapter_dx(const void* dkv_edge, int64_t ld, const int32_t* uniq, const 
   // 256 x 384 tiles where N allows (one stage ahead, 2 x 80 KB of LDS: a sixth less operand
   // traffic per product than 256 x 256; c3 dX 102 -> 76 us), else 128 x 256 tiles two stages ahead
 #define MOC_CGDX(DST, TO)                                                                                           \
-  if (N % 384 == 0)                                                                                                 \
+  if (N % 384 == 0 && !cg_narrow(max_u, N))                                                                         \
     hipLaunchKernelGGL((chapter_gemm_kernel<CG_SRC_EDGE, DST, TO, 256, kCgDepth256, MOC_NORM_NONE, 384>), grid,      \
                        dim3(kCgThreads), 0, stream, (const bf16*)dkv_edge, (const bf16*)red, ld, uniq, n_uniq,       \
                        csr_off, csr_edge, max_u, (const bf16*)w_t, N, K, (TO*)out, ldo, max_u * 64, max_u * 64,     \
@@ -1009,6 +1021,8 @@ int moc_rows_linear(const void* x, int64_t ldx, int64_t R, const void* w, int N,
   MOC_REQUIRE(x && w && y, MOC_ERR_ARG, "moc_rows_linear: null pointer");
   MOC_REQUIRE(R >= 0 && R < ((int64_t)1 << 36), MOC_ERR_ARG, "moc_rows_linear: R=%lld", (long long)R);
   if (int rc = cg_check("moc_rows_linear", ldx, N, K, (R + 63) / 64, ldy)) return rc;
+  if (mid_linear_takes(R, N, K) && (((uintptr_t)x | (uintptr_t)w | (uintptr_t)y) & 15) == 0)
+    return mid_linear(x, ldx, R, w, N, K, y, ldy, nullptr, 0, stream);
   return rows_gemm<bf16, 0>("chapter_gemm_kernel(rows)", x, ldx, R, w, N, K, y, ldy, CgEpi{}, stream);
 }
 
@@ -1020,6 +1034,8 @@ int moc_rows_linear_residual(const void* x, int64_t ldx, int64_t R, const void* 
               MOC_ERR_ARG, "moc_rows_linear_residual: residual row stride %lld (N=%d), 16-byte aligned rows",
               (long long)ldr, N);
   if (int rc = cg_check("moc_rows_linear_residual", ldx, N, K, (R + 63) / 64, ldy)) return rc;
+  if (mid_linear_takes(R, N, K) && (((uintptr_t)x | (uintptr_t)w | (uintptr_t)y) & 15) == 0)
+    return mid_linear(x, ldx, R, w, N, K, y, ldy, res, ldr, stream);
   return rows_gemm<bf16, CG_EPI_RES>("chapter_gemm_kernel(rows, residual)", x, ldx, R, w, N, K, y, ldy,
                                      CgEpi{(const bf16*)res, ldr, nullptr}, stream);
 }

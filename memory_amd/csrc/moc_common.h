@@ -360,6 +360,17 @@ int sparse_bwd_launch(int dtype, const void* q, const void* dout, int64_t ntok, 
                       float scale, void* dk, void* dv, int64_t ocs, int64_t ohs, int64_t ors, void* dq_part,
                       float* dlog, const int32_t* row_tab, hipStream_t stream, const char* who, int kvdiv);
 
+// Workgroups per (sequence, head, 128 queries) over which the attention forward and dQ kernels
+// split the slots when a workspace is given (xattn_fwd.hip); 1 = not split.
+constexpr int64_t kXattnWgs = 768;
+int xattn_splits(int dtype, int64_t B, int64_t L, int H, int NS);
+
+// y [M][N] = x [M][K] w^T (+ res) for few rows (small_linear.hip): bf16, N a multiple of 32, K of
+// 128, rows 16-byte aligned (ldx % 8 == 0), ldy and ldr multiples of 4.
+bool mid_linear_takes(int64_t M, int N, int K);
+int mid_linear(const void* x, int64_t ldx, int64_t M, const void* w, int N, int K, void* y, int64_t ldy,
+               const void* res, int64_t ldr, hipStream_t stream);
+
 // out[i] = inv * sum_j part[j * n + i] for i < n, j < nsplit, summed in a fixed order
 // (router.hip's split-row reduction); returns a MOC_ status.
 int launch_split_reduce(const float* part, int nsplit, int64_t n, float inv, float* out, hipStream_t stream);

@@ -137,7 +137,8 @@ struct SeqLayout {
   size_t q, attn, pooled, w, uniq, n_uniq, edge_u, csr_off, csr_edge, plan_ws, wkv, wkv_t, wq_t, wo_t, kv, lse;
   size_t plan_ws_bytes, saved_bytes;
   // scratch
-  size_t mlist;
+  size_t mlist, xws_f;
+  size_t xws_b, xws_bytes;
   size_t d_attn, delta, dq, dkv_edge, dom_part, red, cw_ws, lw_ws, dz, dpooled, rl_ws;
   size_t cw_ws_bytes, lw_ws_bytes, rl_ws_bytes, scratch_bytes;
 
@@ -176,6 +177,9 @@ struct SeqLayout {
     kv = take((size_t)max_u * 64 * 2 * KV * 2);
     lse = take((size_t)B * H * Lp * 4);
     mlist = take(dkv_multi_list_bytes(max_u));
+    // partial rows of the attention's slot splits (small grids only, at most 26 MB)
+    xws_bytes = moc_xattn_split_workspace(MOC_BF16, B, L, H, NS);
+    xws_f = take(xws_bytes);
     saved_bytes = o;
     o = 0;
     d_attn = take(tok * d * 2);
@@ -192,6 +196,7 @@ struct SeqLayout {
     dpooled = take((size_t)B * d * 4);
     rl_ws_bytes = moc_router_linear_bwd_workspace(B, d, C);
     rl_ws = take(rl_ws_bytes);
+    xws_b = take(xws_bytes);
     scratch_bytes = o;
     return MOC_OK;
   }
@@ -312,8 +317,9 @@ int moc_seq_layer_fwd(const void* h, const void* bank, const void* wr, int wr_dt
   MOC_HIP(hipStreamWaitEvent(main, ev[1], 0));
   const int64_t span = y.max_u * 64 * KV2 - y.KV;
   SEQ_STAGE(kStAttnFwd, main,
-            SEQ_TRY(moc_xattn_fwd(MOC_BF16, q, kv, kv + y.KV, span, (int64_t)64 * KV2, 64, KV2, edge_u, omega, B, L,
-                                  H, HK, 64, 64, y.NS, 0.125f, attn, lse, main)));
+            SEQ_TRY(moc_xattn_fwd_split(MOC_BF16, q, kv, kv + y.KV, span, (int64_t)64 * KV2, 64, KV2, edge_u, omega, B,
+                                        L, H, HK, 64, 64, y.NS, 0.125f, attn, lse, y.xws_bytes ? sv + y.xws_f : nullptr,
+                                        y.xws_bytes, main)));
   SEQ_STAGE(kStOProj, main, SEQ_TRY(moc_rows_linear(attn, d, tok, wo, (int)d, (int)d, out, d, main)));
   MOC_HIP(hipStreamWaitEvent(main, ev[2], 0));
   join.disarm();
@@ -386,9 +392,9 @@ int moc_seq_layer_bwd(const void* h, const void* bank, const void* wr, int wr_dt
     MOC_HIP(hipEventRecord(ev[2], fill));
   }
   SEQ_STAGE(kStDq, main,
-            SEQ_TRY(moc_xattn_bwd_dq_delta(MOC_BF16, q, kv, kv + y.KV, span, (int64_t)64 * KV2, 64, KV2, edge_u,
-                                           omega, attn, d_attn, lse, delta, B, L, H, HK, 64, 64, y.NS, 0.125f, dq,
-                                           main)));
+            SEQ_TRY(moc_xattn_bwd_dq_delta_split(MOC_BF16, q, kv, kv + y.KV, span, (int64_t)64 * KV2, 64, KV2, edge_u,
+                                                 omega, attn, d_attn, lse, delta, B, L, H, HK, 64, 64, y.NS, 0.125f,
+                                                 dq, y.xws_bytes ? sc + y.xws_b : nullptr, y.xws_bytes, main)));
   // aux: q_proj dX into dh beside dK/dV; fill (done with the zeros by then): q_proj dW beside
   // dK/dV, so that the aux stream reaches the router backward when dK/dV ends (both on aux, they
   // ran past dK/dV's end and the router backward past the main stream's last kernel).  When

@@ -90,14 +90,16 @@ __device__ __forceinline__ void bq_dma16(__amdgpu_buffer_rsrc_t r, uint32_t voff
 // dq: one workgroup = 128 queries of one (sequence, head), loop over its slots.  With `out` (the
 // forward's output) the pre-pass is fused: the workgroup forms delta = rowsum(dout * out) of its
 // queries from the dO fragments it loads anyway and writes it (padded rows 0) for the dK/dV
-// kernel; without it delta is read.
-template <typename T>
+// kernel; without it delta is read.  SPLIT: the slots are divided over nsplit workgroups per 128
+// queries, each writing its f32 share part[split][b][l][h][64] (delta by the first);
+// xattn_dq_sum_kernel adds them in split order.
+template <typename T, bool SPLIT>
 __global__ __launch_bounds__(kBThreads) void xattn_bwd_dq_kernel(
     const T* __restrict__ q, const T* __restrict__ ktiles, const T* __restrict__ vtiles,
     const int32_t* __restrict__ slot_u, const float* __restrict__ omega,
     const T* __restrict__ dout, const T* __restrict__ out, const float* __restrict__ lse, float* __restrict__ delta,
     int B, int L, int H, int HK, int NS, int64_t kv_span, int64_t kv_su, int kv_sh, int kv_st, float scale_log2,
-    float scale, T* __restrict__ dq) {
+    float scale, T* __restrict__ dq, int nsplit, float* __restrict__ part) {
   typedef typename Frag<T>::type F8;
   using Tile = SwzTile<T, 64>;
   constexpr int TB = kBT * kBDh * (int)sizeof(T);
@@ -108,9 +110,14 @@ __global__ __launch_bounds__(kBThreads) void xattn_bwd_dq_kernel(
 
   // tiles: (sequence, head) major, 128-query block minor (XCD-local chapter tiles)
   const int nqb = (L + 127) / 128;
-  const int64_t t = xcd_tile((int64_t)B * H * nqb);
+  const int nsp = SPLIT ? nsplit : 1;
+  const int64_t t = xcd_tile((int64_t)B * H * nsp * nqb);
   if (t < 0) return;
-  const int b = (int)(t / ((int64_t)H * nqb)), h = (int)((t / nqb) % H);
+  const int64_t bh = t / ((int64_t)nsp * nqb);
+  const int b = (int)(bh / H), h = (int)(bh % H);
+  const int sp = SPLIT ? (int)((t / nqb) % nsp) : 0;
+  const int s_begin = SPLIT ? (int)((int64_t)NS * sp / nsp) : 0;
+  const int s_end = SPLIT ? (int)((int64_t)NS * (sp + 1) / nsp) : NS;
   const int hk = h / (H / HK);
   const int q0 = (int)(t % nqb) * 128;
   const int Lp = nqb * 128;
@@ -145,7 +152,7 @@ __global__ __launch_bounds__(kBThreads) void xattn_bwd_dq_kernel(
       sacc += __shfl_xor(sacc, 16);
       sacc += __shfl_xor(sacc, 32);
       dl[qb] = sacc;
-      if (g == 0) delta[((size_t)b * H + h) * Lp + qi] = sacc;
+      if (g == 0 && sp == 0) delta[((size_t)b * H + h) * Lp + qi] = sacc;
     } else {
       dl[qb] = ok ? delta[((size_t)b * H + h) * Lp + qi] : 0.f;
     }
@@ -181,19 +188,19 @@ __global__ __launch_bounds__(kBThreads) void xattn_bwd_dq_kernel(
       vio.load_rows(vb, tile_off(u), row_bytes, tid);
     }
   };
-  int u_cur = su[0];
+  int u_cur = su[s_begin];
   if (u_cur >= 0) {
-    fetch(u_cur, 0);
+    fetch(u_cur, s_begin & 1);
     if constexpr (!kDma) {
-      kio.store(sK[0], tid);
-      vio.store(sV[0], tid);
+      kio.store(sK[s_begin & 1], tid);
+      vio.store(sV[s_begin & 1], tid);
     }
   }
   vm_wait_all();  // Q / dO fragments (and the first tiles) have landed on every path into the loop
   __syncthreads();
-  for (int s = 0; s < NS; ++s) {
+  for (int s = s_begin; s < s_end; ++s) {
     const int buf = s & 1;
-    const int u_next = (s + 1 < NS) ? su[s + 1] : -1;
+    const int u_next = (s + 1 < s_end) ? su[s + 1] : -1;
     // (buffer buf ^ 1 was last read in slot s - 1, which every wave has finished)
     if (u_next >= 0) fetch(u_next, buf ^ 1);
     // a slot of zero router weight has dS = 0 (its keys and values are zero): no dQ contribution;
@@ -272,11 +279,31 @@ __global__ __launch_bounds__(kBThreads) void xattn_bwd_dq_kernel(
     for (int e = 0; e < 4; ++e) {
       const int qi = q0 + 32 * wave + 16 * qb + 4 * g + e;
       if (qi < L) {
-        T* dst = dq + ((size_t)(b * (size_t)L + qi) * H + h) * kBDh;
+        if constexpr (SPLIT) {
+          float* dst = part + ((((size_t)sp * B + b) * L + qi) * H + h) * kBDh;
 #pragma unroll
-        for (int db = 0; db < 4; ++db) dst[16 * db + c16] = from_f<T>(acc[qb][db][e]);
+          for (int db = 0; db < 4; ++db) dst[16 * db + c16] = acc[qb][db][e];
+        } else {
+          T* dst = dq + ((size_t)(b * (size_t)L + qi) * H + h) * kBDh;
+#pragma unroll
+          for (int db = 0; db < 4; ++db) dst[16 * db + c16] = from_f<T>(acc[qb][db][e]);
+        }
       }
     }
+}
+
+// dq = sum of the splits' shares, in split order, four consecutive elements per thread
+template <typename T>
+__global__ __launch_bounds__(256) void xattn_dq_sum_kernel(const float* __restrict__ part, int nsplit, int64_t n4,
+                                                           T* __restrict__ dq) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n4) return;
+  const f32x4* p = reinterpret_cast<const f32x4*>(part) + i;
+  f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+  for (int sp = 0; sp < nsplit; ++sp) s += p[(size_t)sp * n4];
+#pragma unroll
+  for (int x = 0; x < 4; ++x) dq[4 * i + x] = from_f<T>(s[x]);
 }
 
 // dk/dv, slot-group decomposition.  One workgroup = one (sequence b, kv head hk,
@@ -820,28 +847,43 @@ namespace {
 int bwd_dq(const char* who, int dtype, const void* q, const void* k_tiles, const void* v_tiles, int64_t kv_span,
            int64_t su, int sh, int st, const int32_t* slot_u, const float* omega, const void* out, const void* dout,
            const float* lse, float* delta, int64_t B, int64_t L, int H, int HK, int Dh, int T, int NS, float scale,
-           void* dq, hipStream_t stream) {
+           void* dq, void* workspace, size_t workspace_bytes, hipStream_t stream) {
   MOC_REQUIRE(q && k_tiles && v_tiles && slot_u && omega && dout && lse && delta && dq, MOC_ERR_ARG,
               "%s: null pointer", who);
   MOC_REQUIRE(Dh == kBDh && T == kBT, MOC_ERR_UNSUPPORTED, "%s: needs head_dim 64 and T 64", who);
   MOC_REQUIRE(H > 0 && HK > 0 && H % HK == 0 && NS > 0, MOC_ERR_ARG, "%s: bad shape", who);
   if (int rc = check_kv_layout(who, dtype, kv_span, su, sh, st)) return rc;
+  MOC_REQUIRE(dtype == MOC_BF16 || dtype == MOC_F32, MOC_ERR_UNSUPPORTED, "%s: dtype %d", who, dtype);
   if (B == 0 || L == 0) return MOC_OK;
   MOC_REQUIRE(B * H * ((L + 127) / 128) < ((int64_t)1 << 31), MOC_ERR_UNSUPPORTED, "%s: grid too large", who);
-  dim3 grid(xcd_grid(B * H * ((L + 127) / 128)));
+  const int ns = workspace ? xattn_splits(dtype, B, L, H, NS) : 1;
+  MOC_REQUIRE(ns == 1 || (workspace_bytes >= moc_xattn_split_workspace(dtype, B, L, H, NS) &&
+                          ((uintptr_t)workspace & 15) == 0),
+              MOC_ERR_ARG, "%s: workspace of %zu bytes (16-byte aligned, at least %zu)", who, workspace_bytes,
+              moc_xattn_split_workspace(dtype, B, L, H, NS));
+  dim3 grid(xcd_grid(B * H * ns * ((L + 127) / 128)));
   const float sl2 = scale * 1.4426950408889634f;
+#define XQ(TT, SP)                                                                                                  \
+  hipLaunchKernelGGL((xattn_bwd_dq_kernel<TT, SP>), grid, dim3(kBThreads), 0, stream, (const TT*)q,                 \
+                     (const TT*)k_tiles, (const TT*)v_tiles, slot_u, omega, (const TT*)dout, (const TT*)out, lse,   \
+                     delta, (int)B, (int)L, H, HK, NS, kv_span, su, sh, st, sl2, scale, (TT*)dq, ns,                \
+                     (float*)workspace)
+  if (dtype == MOC_BF16) {
+    if (ns > 1) XQ(bf16, true); else XQ(bf16, false);
+  } else {
+    if (ns > 1) XQ(float, true); else XQ(float, false);
+  }
+#undef XQ
+  if (int rc = check_launch("xattn_bwd_dq_kernel")) return rc;
+  if (ns == 1) return MOC_OK;
+  const int64_t n4 = B * L * H * kBDh / 4;
+  const dim3 sgrid((unsigned)((n4 + 255) / 256));
   if (dtype == MOC_BF16)
-    hipLaunchKernelGGL(xattn_bwd_dq_kernel<bf16>, grid, dim3(kBThreads), 0, stream, (const bf16*)q, (const bf16*)k_tiles,
-                       (const bf16*)v_tiles, slot_u, omega, (const bf16*)dout, (const bf16*)out, lse, delta, (int)B,
-                       (int)L, H, HK, NS, kv_span, su, sh, st, sl2, scale, (bf16*)dq);
-  else if (dtype == MOC_F32)
-    hipLaunchKernelGGL(xattn_bwd_dq_kernel<float>, grid, dim3(kBThreads), 0, stream, (const float*)q,
-                       (const float*)k_tiles, (const float*)v_tiles, slot_u, omega, (const float*)dout,
-                       (const float*)out, lse, delta, (int)B, (int)L, H, HK, NS, kv_span, su, sh, st, sl2, scale,
-                       (float*)dq);
+    hipLaunchKernelGGL(xattn_dq_sum_kernel<bf16>, sgrid, dim3(256), 0, stream, (const float*)workspace, ns, n4, (bf16*)dq);
   else
-    return set_error(MOC_ERR_UNSUPPORTED, "%s: dtype %d", who, dtype);
-  return check_launch("xattn_bwd_dq_kernel");
+    hipLaunchKernelGGL(xattn_dq_sum_kernel<float>, sgrid, dim3(256), 0, stream, (const float*)workspace, ns, n4,
+                       (float*)dq);
+  return check_launch("xattn_dq_sum_kernel");
 }
 }  // namespace
 }  // namespace moc
@@ -853,16 +895,25 @@ int moc_xattn_bwd_dq(int dtype, const void* q, const void* k_tiles, const void* 
                      const float* delta, int64_t B, int64_t L, int H, int HK, int Dh, int T, int NS, float scale,
                      void* dq, hipStream_t stream) {
   return bwd_dq("moc_xattn_bwd_dq", dtype, q, k_tiles, v_tiles, kv_span, su, sh, st, slot_u, omega, nullptr, dout, lse,
-                const_cast<float*>(delta), B, L, H, HK, Dh, T, NS, scale, dq, stream);
+                const_cast<float*>(delta), B, L, H, HK, Dh, T, NS, scale, dq, nullptr, 0, stream);
 }
 
 int moc_xattn_bwd_dq_delta(int dtype, const void* q, const void* k_tiles, const void* v_tiles, int64_t kv_span,
                            int64_t su, int sh, int st, const int32_t* slot_u, const float* omega, const void* out,
-                           const void* dout, const float* lse, float* delta, int64_t B, int64_t L, int H, int HK, int Dh,
-                           int T, int NS, float scale, void* dq, hipStream_t stream) {
-  MOC_REQUIRE(out, MOC_ERR_ARG, "moc_xattn_bwd_dq_delta: null pointer");
+                           const void* dout, const float* lse, float* delta, int64_t B, int64_t L, int H, int HK,
+                           int Dh, int T, int NS, float scale, void* dq, hipStream_t stream) {
+  return moc_xattn_bwd_dq_delta_split(dtype, q, k_tiles, v_tiles, kv_span, su, sh, st, slot_u, omega, out, dout, lse,
+                                      delta, B, L, H, HK, Dh, T, NS, scale, dq, nullptr, 0, stream);
+}
+
+int moc_xattn_bwd_dq_delta_split(int dtype, const void* q, const void* k_tiles, const void* v_tiles, int64_t kv_span,
+                                 int64_t su, int sh, int st, const int32_t* slot_u, const float* omega,
+                                 const void* out, const void* dout, const float* lse, float* delta, int64_t B,
+                                 int64_t L, int H, int HK, int Dh, int T, int NS, float scale, void* dq,
+                                 void* workspace, size_t workspace_bytes, hipStream_t stream) {
+  MOC_REQUIRE(out != nullptr, MOC_ERR_ARG, "moc_xattn_bwd_dq_delta: null pointer");
   return bwd_dq("moc_xattn_bwd_dq_delta", dtype, q, k_tiles, v_tiles, kv_span, su, sh, st, slot_u, omega, out, dout,
-                lse, delta, B, L, H, HK, Dh, T, NS, scale, dq, stream);
+                lse, delta, B, L, H, HK, Dh, T, NS, scale, dq, workspace, workspace_bytes, stream);
 }
 
 int moc_xattn_bwd_dkv(int dtype, const void* q, const void* dout,

@@ -22,6 +22,8 @@
 // K and V blocks (both [key][dim]) are double-buffered in
 // LDS; the V^T operand is read from the V tile with the transposing LDS read, whose lane
 // order is the key order of the P~^T fragments.
+#include <math.h>
+
 #include "moc_common.h"
 
 namespace moc {
@@ -57,11 +59,15 @@ __device__ __forceinline__ void fwd_dma16(__amdgpu_buffer_rsrc_t r, uint32_t vof
   asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(r), "s"(soff), "{m0}"(m0) : "memory");
 }
 
-template <typename T>
+// SPLIT: the slots of a (sequence, head) are divided over nsplit workgroups per 128 queries, each
+// writing normalised f32 partial rows part[split][b][l][h][64] and their log-sum-exp (log2 units,
+// -inf when every slot was skipped) lse[split][b][h][Lp]; xattn_merge_kernel combines them.
+template <typename T, bool SPLIT>
 __global__ __launch_bounds__(kFwdThreads) void xattn_fwd_kernel(
     const T* __restrict__ q, const T* __restrict__ ktiles, const T* __restrict__ vtiles,
     const int32_t* __restrict__ slot_u, const float* __restrict__ omega, int B, int L, int H, int HK, int NS,
-    int64_t kv_span, int64_t kv_su, int kv_sh, int kv_st, float scale_log2, T* __restrict__ out, float* __restrict__ lse) {
+    int64_t kv_span, int64_t kv_su, int kv_sh, int kv_st, float scale_log2, T* __restrict__ out,
+    float* __restrict__ lse, int nsplit, float* __restrict__ part) {
   typedef typename Frag<T>::type F8;
   using Tile = SwzTile<T, 64>;
   constexpr int TB = kTch * kDh * (int)sizeof(T);
@@ -71,9 +77,14 @@ __global__ __launch_bounds__(kFwdThreads) void xattn_fwd_kernel(
   // tiles: (sequence, head) major, 128-query block minor, so the query blocks that read
   // the same chapter tiles share one XCD's L2
   const int nqb = (L + 127) / 128;
-  const int64_t t = xcd_tile((int64_t)B * H * nqb);
+  const int nsp = SPLIT ? nsplit : 1;
+  const int64_t t = xcd_tile((int64_t)B * H * nsp * nqb);
   if (t < 0) return;
-  const int b = (int)(t / ((int64_t)H * nqb)), h = (int)((t / nqb) % H);
+  const int64_t bh = t / ((int64_t)nsp * nqb);
+  const int b = (int)(bh / H), h = (int)(bh % H);
+  const int sp = SPLIT ? (int)((t / nqb) % nsp) : 0;
+  const int s_begin = SPLIT ? (int)((int64_t)NS * sp / nsp) : 0;
+  const int s_end = SPLIT ? (int)((int64_t)NS * (sp + 1) / nsp) : NS;
   const int hk = h / (H / HK);
   const int q0 = (int)(t % nqb) * 128;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -135,12 +146,12 @@ __global__ __launch_bounds__(kFwdThreads) void xattn_fwd_kernel(
     }
   };
 
-  int u_cur = su[0];
+  int u_cur = su[s_begin];
   if (u_cur >= 0) {
-    fetch(u_cur, 0);
+    fetch(u_cur, s_begin & 1);
     if constexpr (!kDma) {
-      kio.store(sK[0], tid);
-      vio.store(sV[0], tid);
+      kio.store(sK[s_begin & 1], tid);
+      vio.store(sV[s_begin & 1], tid);
     }
   }
   // Q fragments must have landed before the loop on every path (also when slot 0
@@ -149,9 +160,9 @@ __global__ __launch_bounds__(kFwdThreads) void xattn_fwd_kernel(
   vm_wait_all();
   __syncthreads();
 
-  for (int s = 0; s < NS; ++s) {
+  for (int s = s_begin; s < s_end; ++s) {
     const int buf = s & 1;
-    const int u_next = (s + 1 < NS) ? su[s + 1] : -1;
+    const int u_next = (s + 1 < s_end) ? su[s + 1] : -1;
     // (buffer buf ^ 1 was last read in slot s - 1, which every wave has finished)
     if (u_next >= 0) fetch(u_next, buf ^ 1);
     if (u_cur >= 0) {
@@ -267,6 +278,15 @@ __global__ __launch_bounds__(kFwdThreads) void xattn_fwd_kernel(
     const float l = lsum[qb];
     const float inv = l > 0.f ? 1.f / l : 0.f;
     const int qi = q0 + 32 * wave + 16 * qb + c16;
+    if constexpr (SPLIT) {
+      if (qi < L) {
+        float* pp = part + ((((size_t)sp * B + b) * L + qi) * H + h) * kDh + 4 * g;
+#pragma unroll
+        for (int db = 0; db < 4; ++db) *reinterpret_cast<f32x4*>(pp + 16 * db) = o[db][qb] * inv;
+      }
+      if (g == 0) lse[(((size_t)sp * B + b) * H + h) * Lp + qi] = l > 0.f ? m[qb] + log2f(l) : -INFINITY;
+      continue;
+    }
     if (qi < L) {
       T* op = out + ((size_t)(b * (size_t)L + qi) * H + h) * kDh;
 #pragma unroll
@@ -276,6 +296,46 @@ __global__ __launch_bounds__(kFwdThreads) void xattn_fwd_kernel(
     }
     if (g == 0) lse[((size_t)b * H + h) * Lp + qi] = (qi < L && l > 0.f) ? m[qb] + log2f(l) : INFINITY;
   }
+}
+
+// out = sum_i 2^(lse_i - M) o_i / sum_i 2^(lse_i - M) over the splits of a (sequence, query, head) row
+// and the row's log-sum-exp (+inf when every slot was skipped, and in the padding rows L .. Lp - 1):
+// 16 lanes of 4 dims per row, rows in [b][l][h] order.
+template <typename T>
+__global__ __launch_bounds__(256) void xattn_merge_kernel(const float* __restrict__ part,
+                                                          const float* __restrict__ lse_part, int nsplit, int B, int L,
+                                                          int Lp, int H, T* __restrict__ out, float* __restrict__ lse) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t row = i >> 4;
+  const int ch = (int)(i & 15);
+  if (row >= (int64_t)B * Lp * H) return;
+  const int h = (int)(row % H);
+  const int64_t bl = row / H;
+  const int b = (int)(bl / Lp), qi = (int)(bl % Lp);
+  float* lo = lse + ((size_t)b * H + h) * Lp + qi;
+  if (qi >= L) {
+    if (ch == 0) *lo = INFINITY;
+    return;
+  }
+  const size_t ls = (size_t)B * H * Lp, ps = (size_t)B * L * H * kDh;
+  const float* lp = lse_part + ((size_t)b * H + h) * Lp + qi;
+  const float* pp = part + (((size_t)b * L + qi) * H + h) * kDh + 4 * ch;
+  float M = -INFINITY;
+#pragma unroll 8
+  for (int sp = 0; sp < nsplit; ++sp) M = fmaxf(M, lp[sp * ls]);
+  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+  float den = 0.f;
+#pragma unroll 8
+  for (int sp = 0; sp < nsplit; ++sp) {
+    const float a = M > -INFINITY ? fast_exp2(lp[sp * ls] - M) : 0.f;
+    acc += *reinterpret_cast<const f32x4*>(pp + sp * ps) * a;
+    den += a;
+  }
+  const float inv = den > 0.f ? 1.f / den : 0.f;
+  T* op = out + (((size_t)b * L + qi) * H + h) * kDh + 4 * ch;
+#pragma unroll
+  for (int x = 0; x < 4; ++x) op[x] = from_f<T>(acc[x] * inv);
+  if (ch == 0) *lo = den > 0.f ? M + log2f(den) : INFINITY;
 }
 
 // Attention weights of the forward above, materialised (MemoryCrossAttention.forward with
@@ -353,31 +413,85 @@ __global__ __launch_bounds__(256) void xattn_weights_kernel(
 
 using namespace moc;
 
+// The loop over the slots is a serial chain, ~1.15 us (bf16; f32 ~6) a slot at low occupancy, and a
+// launch has one workgroup per (sequence, head, 128 queries), a "tile"; three fit a CU.  Splitting the
+// slots n ways costs a merge launch (~5 us) and its f32 partial rows (~0.016 us per tile and split,
+// written and read): n at the minimum of chain + partial rows, while n tiles fit the chip, and only
+// where the sum is smaller.  Measured (forward; dQ is alike), 65 slots: 48 tiles 76 -> 27 us, 96 tiles
+// 76 -> 35, 192 tiles 78 -> 54, 288 tiles 96 -> 81, 384 tiles 98 -> 86; 17 slots: 32 tiles 23 -> 17,
+// 384 tiles 32 -> 39 (not split); the plain minimum chain length (one slot a split) was slower
+// everywhere (48 tiles 42 us).
+int moc::xattn_splits(int dtype, int64_t B, int64_t L, int H, int NS) {
+  const int64_t tiles = B * H * ((L + 127) / 128);
+  if (tiles <= 0 || NS <= 1) return 1;
+  const double slot = dtype == MOC_F32 ? 6.0 : 1.15, tile = 0.016;
+  int64_t n = kXattnWgs / tiles;
+  const int64_t best = (int64_t)(sqrt(slot * NS / (tile * (double)tiles)) + 0.5);
+  if (n > best) n = best;
+  if (n > NS) n = NS;
+  if (n < 2) return 1;
+  const int64_t per = (NS + n - 1) / n;
+  n = (NS + per - 1) / per;
+  return slot * (double)(NS - per) > 5.0 + tile * (double)(n * tiles) ? (int)n : 1;
+}
+
 extern "C" {
+
+size_t moc_xattn_split_workspace(int dtype, int64_t B, int64_t L, int H, int NS) {
+  const int n = xattn_splits(dtype, B, L, H, NS);
+  return n > 1 ? (size_t)n * ((size_t)B * L * H * kDh + (size_t)B * H * ((L + 127) / 128 * 128)) * sizeof(float) : 0;
+}
 
 int moc_xattn_fwd(int dtype, const void* q, const void* k_tiles, const void* v_tiles, int64_t kv_span, int64_t su,
                   int sh, int st, const int32_t* slot_u, const float* omega, int64_t B, int64_t L, int H, int HK, int Dh, int T,
                   int NS, float scale, void* out, float* lse, hipStream_t stream) {
+  return moc_xattn_fwd_split(dtype, q, k_tiles, v_tiles, kv_span, su, sh, st, slot_u, omega, B, L, H, HK, Dh, T, NS,
+                             scale, out, lse, nullptr, 0, stream);
+}
+
+int moc_xattn_fwd_split(int dtype, const void* q, const void* k_tiles, const void* v_tiles, int64_t kv_span,
+                        int64_t su, int sh, int st, const int32_t* slot_u, const float* omega, int64_t B, int64_t L,
+                        int H, int HK, int Dh, int T, int NS, float scale, void* out, float* lse, void* workspace,
+                        size_t workspace_bytes, hipStream_t stream) {
   MOC_REQUIRE(q && k_tiles && v_tiles && slot_u && omega && out && lse, MOC_ERR_ARG, "moc_xattn_fwd: null pointer");
   MOC_REQUIRE(Dh == kDh && T == kTch, MOC_ERR_UNSUPPORTED, "moc_xattn_fwd: needs head_dim 64 and 64 tokens per chapter (got %d, %d)", Dh, T);
   MOC_REQUIRE(H > 0 && HK > 0 && H % HK == 0, MOC_ERR_ARG, "moc_xattn_fwd: H=%d HK=%d", H, HK);
   MOC_REQUIRE(NS > 0 && B >= 0 && L >= 0, MOC_ERR_ARG, "moc_xattn_fwd: bad shape");
   MOC_REQUIRE(B < 65536 && H < 65536, MOC_ERR_UNSUPPORTED, "moc_xattn_fwd: grid too large");
   if (int rc = check_kv_layout("moc_xattn_fwd", dtype, kv_span, su, sh, st)) return rc;
+  MOC_REQUIRE(dtype == MOC_BF16 || dtype == MOC_F32, MOC_ERR_UNSUPPORTED, "moc_xattn_fwd: dtype %d", dtype);
   if (B == 0 || L == 0) return MOC_OK;
   MOC_REQUIRE(B * H * ((L + 127) / 128) < ((int64_t)1 << 31), MOC_ERR_UNSUPPORTED, "moc_xattn_fwd: grid too large");
-  dim3 grid(xcd_grid(B * H * ((L + 127) / 128)));
   const float sl2 = scale * 1.4426950408889634f;
+  const int ns = workspace ? xattn_splits(dtype, B, L, H, NS) : 1;
+  MOC_REQUIRE(ns == 1 || (workspace_bytes >= moc_xattn_split_workspace(dtype, B, L, H, NS) &&
+                          ((uintptr_t)workspace & 15) == 0),
+              MOC_ERR_ARG, "moc_xattn_fwd: workspace of %zu bytes (16-byte aligned, at least %zu)", workspace_bytes,
+              moc_xattn_split_workspace(dtype, B, L, H, NS));
+  const int Lp = (int)((L + 127) / 128 * 128);
+  float* part = (float*)workspace;
+  float* lse_part = ns > 1 ? part + (size_t)ns * B * L * H * kDh : lse;
+  dim3 grid(xcd_grid(B * H * ns * ((L + 127) / 128)));
+#define XF(TT, SP)                                                                                                  \
+  hipLaunchKernelGGL((xattn_fwd_kernel<TT, SP>), grid, dim3(kFwdThreads), 0, stream, (const TT*)q,                  \
+                     (const TT*)k_tiles, (const TT*)v_tiles, slot_u, omega, (int)B, (int)L, H, HK, NS, kv_span, su, \
+                     sh, st, sl2, (TT*)out, lse_part, ns, part)
+  if (dtype == MOC_BF16) {
+    if (ns > 1) XF(bf16, true); else XF(bf16, false);
+  } else {
+    if (ns > 1) XF(float, true); else XF(float, false);
+  }
+#undef XF
+  if (int rc = check_launch("xattn_fwd_kernel")) return rc;
+  if (ns == 1) return MOC_OK;
+  const dim3 mgrid((unsigned)(((int64_t)B * Lp * H * 16 + 255) / 256));
   if (dtype == MOC_BF16)
-    hipLaunchKernelGGL(xattn_fwd_kernel<bf16>, grid, dim3(kFwdThreads), 0, stream, (const bf16*)q, (const bf16*)k_tiles,
-                       (const bf16*)v_tiles, slot_u, omega, (int)B, (int)L, H, HK, NS, kv_span, su, sh, st, sl2, (bf16*)out, lse);
-  else if (dtype == MOC_F32)
-    hipLaunchKernelGGL(xattn_fwd_kernel<float>, grid, dim3(kFwdThreads), 0, stream, (const float*)q,
-                       (const float*)k_tiles, (const float*)v_tiles, slot_u, omega, (int)B, (int)L, H, HK, NS, kv_span, su, sh, st,
-                       sl2, (float*)out, lse);
+    hipLaunchKernelGGL(xattn_merge_kernel<bf16>, mgrid, dim3(256), 0, stream, part, lse_part, ns, (int)B, (int)L, Lp, H,
+                       (bf16*)out, lse);
   else
-    return set_error(MOC_ERR_UNSUPPORTED, "moc_xattn_fwd: dtype %d", dtype);
-  return check_launch("xattn_fwd_kernel");
+    hipLaunchKernelGGL(xattn_merge_kernel<float>, mgrid, dim3(256), 0, stream, part, lse_part, ns, (int)B, (int)L, Lp, H,
+                       (float*)out, lse);
+  return check_launch("xattn_merge_kernel");
 }
 
 int moc_xattn_weights(int dtype, const void* q, const void* k_tiles, int64_t kv_span, int64_t su, int sh, int st,

@@ -606,6 +606,13 @@ def _tiny_chapters(max_u: int, T: int, d: int, KV: int) -> bool:
     return max_u * T <= 256 and d % 128 == 0 and (2 * KV) % 128 == 0
 
 
+def _split_workspace(dtype, B: int, Lq: int, H: int, NS: int, dev):
+    """(workspace, bytes) of the attention forward / dQ kernels where small grids split the slots
+    over workgroups; (None, 0) where they do not."""
+    n = L.query("moc_xattn_split_workspace", L.dtype_code(dtype), B, Lq, H, NS)
+    return (torch.empty(n, device=dev, dtype=torch.uint8), n) if n else (None, 0)
+
+
 def routed_attn_forward(q, bank, wk, wv, omega, idx_star, num_chapters, T, norm, eps, HK, wkv=None):
     """Forward body of the sequence-routed attention (plan, gather + K/V projection, joint
     attention): returns (out, saved tensors in _ATTN_SAVED order, cfg).  ``wkv``: the packed
@@ -666,8 +673,9 @@ def routed_attn_forward(q, bank, wk, wv, omega, idx_star, num_chapters, T, norm,
     out = torch.empty(B, Lq, H, Dh, device=q.device, dtype=dtype)
     Lp = (Lq + 127) // 128 * 128
     lse = torch.empty(B, H, Lp, device=q.device, dtype=torch.float32)
-    call("moc_xattn_fwd", L.dtype_code(dtype), ptr(q), ptr(kv), ptr(kv) + KV * kv.element_size(), *kvl,
-         ptr(plan.edge_u), ptr(om), B, Lq, H, HK, Dh, T, NS, float(Dh) ** -0.5, ptr(out), ptr(lse),
+    ws, ws_bytes = _split_workspace(dtype, B, Lq, H, NS, q.device)
+    call("moc_xattn_fwd_split", L.dtype_code(dtype), ptr(q), ptr(kv), ptr(kv) + KV * kv.element_size(), *kvl,
+         ptr(plan.edge_u), ptr(om), B, Lq, H, HK, Dh, T, NS, float(Dh) ** -0.5, ptr(out), ptr(lse), ptr(ws), ws_bytes,
          stream_ptr(q.device))
     saved = (q, bank, wkv, om, out, lse, kv, mean, rstd, plan.uniq, plan.n_uniq, plan.edge_u, plan.csr_off,
              plan.csr_edge)
@@ -703,8 +711,10 @@ def routed_attn_backward(saved, cfg, dout, needs, row_grad=None, after_dq=None, 
     dq = torch.empty_like(q)
     kvl = kv_rows_layout(kv, T, HK, Dh)
     vptr = ptr(kv) + KV * kv.element_size()
-    call("moc_xattn_bwd_dq_delta", dt, ptr(q), ptr(kv), vptr, *kvl, ptr(edge_u), ptr(om), ptr(out),
-         ptr(dout), ptr(lse), ptr(delta), B, Lq, H, HK, Dh, T, NS, scale, ptr(dq), st)
+    ws, ws_bytes = _split_workspace(dtype, B, Lq, H, NS, dev)
+    call("moc_xattn_bwd_dq_delta_split", dt, ptr(q), ptr(kv), vptr, *kvl, ptr(edge_u), ptr(om), ptr(out),
+         ptr(dout), ptr(lse), ptr(delta), B, Lq, H, HK, Dh, T, NS, scale, ptr(dq), ptr(ws), ws_bytes, st)
+    del ws
     if after_dq is not None:
         after_dq(dq)
     dkv_edge = torch.empty(B * NS * T, 2 * KV, device=dev, dtype=dtype)
