@@ -179,6 +179,12 @@ int moc_chapter_plan_noalloc(const int32_t* chap, int64_t E, int64_t C, int32_t*
 
 /* --------------------------------------------------- gather + K/V projection */
 
+/* The rows of the plan's chapters normalised (model.py:423-432; norm = MOC_NORM_RMS or
+ * MOC_NORM_LAYERNORM) into a contiguous block in one pass: out bf16 [max_u * 64][d] = (row - mean) *
+ * rstd, mean / rstd f32 [max_u * 64] (rows of plan slots >= n_uniq are not written): moc_row_stats +
+ * moc_gather_rows for a bf16 bank, T = 64.  d % 8 == 0, d <= 4096, 16-byte aligned. */
+int moc_norm_gather_rows(const void* bank, int64_t d, const int32_t* uniq, const int32_t* n_uniq, int64_t max_u,
+                         int norm, float eps, float* mean, float* rstd, void* out, hipStream_t stream);
 /* Per-row statistics of the gathered rows for MemoryTransformer._normalize_shared_routed_memory_vectors
  * (memory_transformer/model.py:393-432): mean f32 and rstd f32 [max_u * T]. */
 int moc_row_stats(const void* bank, int bank_dtype, int64_t d, int T, const int32_t* uniq, const int32_t* n_uniq,
@@ -329,6 +335,24 @@ int moc_seq_layer_bwd(const void* h, const void* bank, const void* wr, int wr_dt
                       size_t saved_bytes, const void* dout, const float* dlogits, void* dh, void* dbank,
                       int64_t bank_rows, float* dwr, float* dbr, void* dwq, void* dwkv, int dwkv_dtype, void* dwo,
                       void* scratch, size_t scratch_bytes, hipStream_t main, hipStream_t aux, hipStream_t fill);
+/* The same with a row-normalised bank (norm != MOC_NORM_NONE: the selected chapters' rows normalised
+ * before the K/V projection, model.py:681-688) and, train = 0, a forward that no backward follows:
+ * `saved` is then a temporary of *infer bytes, free as soon as the call's work on `main` is done.
+ * moc_seq_layer_sizes gives the bytes of the three buffers (an error status for shapes outside the
+ * layer's). */
+int moc_seq_layer_sizes(int64_t B, int64_t L, int64_t d, int H, int HK, int64_t C, int S, int k, int norm,
+                        size_t* saved, size_t* scratch, size_t* infer);
+int moc_seq_layer_fwd_ex(const void* h, const void* bank, const void* wr, int wr_dtype, const float* br,
+                         const void* wq, const void* wk, const void* wv, const void* wo, const float* coef, int64_t B,
+                         int64_t L, int64_t d, int H, int HK, int64_t C, int S, int k, float routed_scale, int norm,
+                         float eps, int train, void* out, float* logits, int32_t* idx, int32_t* idx_star, float* omega,
+                         void* saved, size_t saved_bytes, hipStream_t main, hipStream_t aux);
+int moc_seq_layer_bwd_ex(const void* h, const void* bank, const void* wr, int wr_dtype, const float* coef, int64_t B,
+                         int64_t L, int64_t d, int H, int HK, int64_t C, int S, int k, float routed_scale, int norm,
+                         const float* logits, const int32_t* idx, const float* omega, const void* saved,
+                         size_t saved_bytes, const void* dout, const float* dlogits, void* dh, void* dbank,
+                         int64_t bank_rows, float* dwr, float* dbr, void* dwq, void* dwkv, int dwkv_dtype, void* dwo,
+                         void* scratch, size_t scratch_bytes, hipStream_t main, hipStream_t aux, hipStream_t fill);
 /* Stage timing of the two calls above (no counterpart in the reference, which times whole steps
  * with torch.cuda.Event in its benchmarks, kernels-final/benchmark_kernels_final.py): stage s is
  * one or a few launches on one stream, named by moc_seq_layer_stage_name(s) (the entry point

@@ -47,6 +47,11 @@ _SIGS = {
                                _P, _P, _P, _P, _P, _P, _SZ, _P, _P]),
     "moc_seq_layer_bwd": (_I, [_P, _P, _P, _I, _P, _I64, _I64, _I64, _I, _I, _I64, _I, _I, _F, _P, _P, _P, _P, _SZ,
                                _P, _P, _P, _P, _I64, _P, _P, _P, _P, _I, _P, _P, _SZ, _P, _P, _P]),
+    "moc_seq_layer_sizes": (_I, [_I64, _I64, _I64, _I, _I, _I64, _I, _I, _I, _P, _P, _P]),
+    "moc_seq_layer_fwd_ex": (_I, [_P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I, _I, _I64, _I, _I, _F,
+                                  _I, _F, _I, _P, _P, _P, _P, _P, _P, _SZ, _P, _P]),
+    "moc_seq_layer_bwd_ex": (_I, [_P, _P, _P, _I, _P, _I64, _I64, _I64, _I, _I, _I64, _I, _I, _F, _I, _P, _P, _P, _P,
+                                  _SZ, _P, _P, _P, _P, _I64, _P, _P, _P, _P, _I, _P, _P, _SZ, _P, _P, _P]),
     "moc_seq_layer_stage_count": (_I, []),
     "moc_seq_layer_stage_name": (ctypes.c_char_p, [_I]),
     "moc_seq_layer_timing": (_I, [ctypes.c_uint64, _I]),
@@ -63,6 +68,7 @@ _SIGS = {
     "moc_chapter_plan_workspace": (_SZ, [_I64, _I64]),
     "moc_chapter_plan": (_I, [_P, _I64, _I64, _P, _SZ, _P, _P, _P, _P, _P, _P]),
     "moc_chapter_plan_noalloc": (_I, [_P, _I64, _I64, _P, _P, _P, _P, _P, _P]),
+    "moc_norm_gather_rows": (_I, [_P, _I64, _P, _P, _I64, _I, _F, _P, _P, _P, _P]),
     "moc_row_stats": (_I, [_P, _I, _I64, _I, _P, _P, _I64, _I, _F, _P, _P, _P]),
     "moc_kv_project": (_I, [_I, _P, _I, _I64, _I, _P, _P, _I64, _P, _P, _P, _I, _I, _P, _P, _P, _P, _P]),
     "moc_chapter_project": (_I, [_P, _I64, _I, _P, _P, _I64, _P, _I, _I, _P, _I64, _P]),

@@ -9,12 +9,14 @@
 // weight gradients); this file only orders them over three streams, so that a training step costs
 // two host calls instead of one per kernel:
 //
-// forward   main: pool -> router linear -> top-k + prepend -> chapter plan -> K/V projection ->
-//                 attention -> o_proj
+// forward   main: pool -> router linear -> top-k + prepend -> chapter plan -> [normalised rows ->]
+//                 K/V projection -> attention -> o_proj
 //           aux:  q projection and the weight packs ([Wk; Wv], [Wk; Wv]^T, Wq^T, Wo^T), which do
-//                 not depend on the routing, beside the latency-bound router launches
+//                 not depend on the routing, beside the latency-bound router launches; without a
+//                 backward to come (train = 0) the transposed ones and the multi-edge list are left out
 // backward  main: o_proj dX -> dQ (+ delta) -> dK/dV -> multi-edge sums -> K/V weight gradient
-//                 -> dX of the projection into the chapters' bank rows
+//                 -> dX of the projection into the chapters' bank rows (a normalised bank: f32 rows,
+//                 then the norm's backward into the bank rows)
 //           aux:  o_proj dW (beside dX / dQ); after dQ: q_proj dX (into dh, beside dK/dV); after
 //                 dK/dV: the router backward and the pooling's gradient added into dh
 //           fill: the dense bank gradient's zeros (beside dQ); after dQ: q_proj dW (beside dK/dV)
@@ -142,8 +144,16 @@ struct SeqLayout {
   size_t d_attn, delta, dq, dkv_edge, dom_part, red, cw_ws, lw_ws, dz, dpooled, rl_ws;
   size_t cw_ws_bytes, lw_ws_bytes, rl_ws_bytes, scratch_bytes;
 
-  int init(int64_t B_, int64_t L_, int64_t d_, int H_, int HK_, int64_t C_, int S_, int k_) {
+  // normalised bank: the plan's rows normalised to bf16 with their statistics (saved), the f32 input
+  // gradient of those rows (scratch)
+  size_t xn, mean, rstd, dxc;
+  size_t infer_bytes;   // the forward without a backward: `saved` without what only the backward reads
+
+  // train: the layout of saved_bytes / scratch_bytes; otherwise that of infer_bytes
+  int init(int64_t B_, int64_t L_, int64_t d_, int H_, int HK_, int64_t C_, int S_, int k_, int norm, bool train) {
     B = B_, L = L_, d = d_, C = C_, H = H_, HK = HK_, S = S_, k = k_;
+    MOC_REQUIRE(norm == MOC_NORM_NONE || norm == MOC_NORM_RMS || norm == MOC_NORM_LAYERNORM, MOC_ERR_ARG,
+                "moc_seq_layer: norm %d", norm);
     MOC_REQUIRE(B > 0 && B <= 64 && L > 0 && d > 0 && H > 0 && HK > 0 && H % HK == 0 && d == (int64_t)H * 64,
                 MOC_ERR_UNSUPPORTED, "moc_seq_layer: B=%lld (1..64), L=%lld, d=%lld = 64 heads of 64 (H=%d, HK=%d)",
                 (long long)B, (long long)L, (long long)d, H, HK);
@@ -171,15 +181,26 @@ struct SeqLayout {
     plan_ws_bytes = moc_chapter_plan_workspace(E, C);
     plan_ws = take(plan_ws_bytes);
     wkv = take((size_t)2 * KV * d * 2);
-    wkv_t = take((size_t)2 * KV * d * 2);
-    wq_t = take((size_t)d * d * 2);
-    wo_t = take((size_t)d * d * 2);
+    if (train) {
+      wkv_t = take((size_t)2 * KV * d * 2);
+      wq_t = take((size_t)d * d * 2);
+      wo_t = take((size_t)d * d * 2);
+    }
     kv = take((size_t)max_u * 64 * 2 * KV * 2);
     lse = take((size_t)B * H * Lp * 4);
-    mlist = take(dkv_multi_list_bytes(max_u));
+    if (train) mlist = take(dkv_multi_list_bytes(max_u));
+    if (norm != MOC_NORM_NONE) {
+      xn = take((size_t)max_u * 64 * d * 2);
+      mean = take((size_t)max_u * 64 * 4);
+      rstd = take((size_t)max_u * 64 * 4);
+    }
     // partial rows of the attention's slot splits (small grids only, at most 26 MB)
     xws_bytes = moc_xattn_split_workspace(MOC_BF16, B, L, H, NS);
     xws_f = take(xws_bytes);
+    if (!train) {
+      infer_bytes = o;
+      return MOC_OK;
+    }
     saved_bytes = o;
     o = 0;
     d_attn = take(tok * d * 2);
@@ -197,6 +218,7 @@ struct SeqLayout {
     rl_ws_bytes = moc_router_linear_bwd_workspace(B, d, C);
     rl_ws = take(rl_ws_bytes);
     xws_b = take(xws_bytes);
+    if (norm != MOC_NORM_NONE) dxc = take((size_t)max_u * 64 * d * 4);
     scratch_bytes = o;
     return MOC_OK;
   }
@@ -237,12 +259,24 @@ extern "C" {
 
 size_t moc_seq_layer_saved_bytes(int64_t B, int64_t L, int64_t d, int H, int HK, int64_t C, int S, int k) {
   SeqLayout lay;
-  return lay.init(B, L, d, H, HK, C, S, k) == MOC_OK ? lay.saved_bytes : 0;
+  return lay.init(B, L, d, H, HK, C, S, k, MOC_NORM_NONE, true) == MOC_OK ? lay.saved_bytes : 0;
 }
 
 size_t moc_seq_layer_scratch_bytes(int64_t B, int64_t L, int64_t d, int H, int HK, int64_t C, int S, int k) {
   SeqLayout lay;
-  return lay.init(B, L, d, H, HK, C, S, k) == MOC_OK ? lay.scratch_bytes : 0;
+  return lay.init(B, L, d, H, HK, C, S, k, MOC_NORM_NONE, true) == MOC_OK ? lay.scratch_bytes : 0;
+}
+
+int moc_seq_layer_sizes(int64_t B, int64_t L, int64_t d, int H, int HK, int64_t C, int S, int k, int norm,
+                        size_t* saved, size_t* scratch, size_t* infer) {
+  MOC_REQUIRE(saved && scratch && infer, MOC_ERR_ARG, "moc_seq_layer_sizes: null pointer");
+  SeqLayout t, i;
+  SEQ_TRY(t.init(B, L, d, H, HK, C, S, k, norm, true));
+  SEQ_TRY(i.init(B, L, d, H, HK, C, S, k, norm, false));
+  *saved = t.saved_bytes;
+  *scratch = t.scratch_bytes;
+  *infer = i.infer_bytes;
+  return MOC_OK;
 }
 
 int moc_seq_layer_fwd(const void* h, const void* bank, const void* wr, int wr_dtype, const float* br, const void* wq,
@@ -250,13 +284,22 @@ int moc_seq_layer_fwd(const void* h, const void* bank, const void* wr, int wr_dt
                       int64_t d, int H, int HK, int64_t C, int S, int k, float routed_scale, void* out,
                       float* logits, int32_t* idx, int32_t* idx_star, float* omega, void* saved, size_t saved_bytes,
                       hipStream_t main, hipStream_t aux) {
+  return moc_seq_layer_fwd_ex(h, bank, wr, wr_dtype, br, wq, wk, wv, wo, coef, B, L, d, H, HK, C, S, k, routed_scale,
+                              MOC_NORM_NONE, 0.f, 1, out, logits, idx, idx_star, omega, saved, saved_bytes, main, aux);
+}
+
+int moc_seq_layer_fwd_ex(const void* h, const void* bank, const void* wr, int wr_dtype, const float* br,
+                         const void* wq, const void* wk, const void* wv, const void* wo, const float* coef, int64_t B,
+                         int64_t L, int64_t d, int H, int HK, int64_t C, int S, int k, float routed_scale, int norm,
+                         float eps, int train, void* out, float* logits, int32_t* idx, int32_t* idx_star, float* omega,
+                         void* saved, size_t saved_bytes, hipStream_t main, hipStream_t aux) {
   MOC_REQUIRE(h && bank && wr && wq && wk && wv && wo && out && logits && idx && idx_star && omega && saved,
               MOC_ERR_ARG, "moc_seq_layer_fwd: null pointer");
   MOC_REQUIRE(main != aux, MOC_ERR_ARG, "moc_seq_layer_fwd: main and aux must be different streams");
   SeqLayout y;
-  SEQ_TRY(y.init(B, L, d, H, HK, C, S, k));
-  MOC_REQUIRE(saved_bytes >= y.saved_bytes, MOC_ERR_ARG, "moc_seq_layer_fwd: saved buffer %zu < %zu bytes",
-              saved_bytes, y.saved_bytes);
+  SEQ_TRY(y.init(B, L, d, H, HK, C, S, k, norm, train != 0));
+  MOC_REQUIRE(saved_bytes >= (train ? y.saved_bytes : y.infer_bytes), MOC_ERR_ARG,
+              "moc_seq_layer_fwd: saved buffer %zu < %zu bytes", saved_bytes, train ? y.saved_bytes : y.infer_bytes);
   hipEvent_t* ev = nullptr;
   SEQ_TRY(seq_events(&ev));
   char* sv = (char*)saved;
@@ -285,7 +328,7 @@ int moc_seq_layer_fwd(const void* h, const void* bank, const void* wr, int wr_dt
   MOC_HIP(hipEventRecord(ev[3], aux));
   SEQ_STAGE(kStQProj, aux, SEQ_TRY(moc_rows_linear(h, d, tok, wq, (int)d, (int)d, q, d, aux)));
   MOC_HIP(hipEventRecord(ev[1], aux));
-  SEQ_STAGE(kStPackT, aux, {
+  if (train) SEQ_STAGE(kStPackT, aux, {
     SEQ_TRY(moc_weight_pack(wk, MOC_BF16, wv, MOC_BF16, y.KV, d, nullptr, sv + y.wkv_t, aux));
     SEQ_TRY(moc_weight_pack(wq, MOC_BF16, (const bf16*)wq + (d / 2) * d, MOC_BF16, d / 2, d, nullptr, sv + y.wq_t,
                             aux));
@@ -303,17 +346,28 @@ int moc_seq_layer_fwd(const void* h, const void* bank, const void* wr, int wr_dt
                                      csr_edge, main)));
   // aux: the plan's multi-edge chapters listed for the backward's per-chapter dK|dV sums (beside
   // the projection; the list lives in the saved buffer)
-  MOC_HIP(hipEventRecord(ev[4], main));
-  MOC_HIP(hipStreamWaitEvent(aux, ev[4], 0));
-  SEQ_TRY(dkv_multi_list(n_uniq, csr_off, csr_edge, y.max_u, (int32_t*)(sv + y.mlist), aux));
-  MOC_HIP(hipEventRecord(ev[2], aux));
+  if (train) {
+    MOC_HIP(hipEventRecord(ev[4], main));
+    MOC_HIP(hipStreamWaitEvent(aux, ev[4], 0));
+    SEQ_TRY(dkv_multi_list(n_uniq, csr_off, csr_edge, y.max_u, (int32_t*)(sv + y.mlist), aux));
+    MOC_HIP(hipEventRecord(ev[2], aux));
+  }
   // main: K/V projection (gather fused), attention, o_proj.  The projection waits for the [Wk; Wv]
   // pack only and the attention for the q projection: both events have completed when the main
   // stream reaches them, so the waits cost nothing (the q projection ends about when the router
   // does, and waiting for it before the projection cost ~6 us of wake-up).
+  // (a normalised bank: the chapters' rows normalised into a contiguous block first, which the
+  // backward's weight gradient reads again)
   MOC_HIP(hipStreamWaitEvent(main, ev[3], 0));
-  SEQ_STAGE(kStKVProj, main,
-            SEQ_TRY(moc_chapter_project(bank, d, 1, uniq, n_uniq, y.max_u, wkv, KV2, (int)d, kv, KV2, main)));
+  SEQ_STAGE(kStKVProj, main, {
+    if (norm == MOC_NORM_NONE) {
+      SEQ_TRY(moc_chapter_project(bank, d, 1, uniq, n_uniq, y.max_u, wkv, KV2, (int)d, kv, KV2, main));
+    } else {
+      SEQ_TRY(moc_norm_gather_rows(bank, d, uniq, n_uniq, y.max_u, norm, eps, (float*)(sv + y.mean),
+                                   (float*)(sv + y.rstd), sv + y.xn, main));
+      SEQ_TRY(moc_chapter_project(sv + y.xn, d, 0, uniq, n_uniq, y.max_u, wkv, KV2, (int)d, kv, KV2, main));
+    }
+  });
   MOC_HIP(hipStreamWaitEvent(main, ev[1], 0));
   const int64_t span = y.max_u * 64 * KV2 - y.KV;
   SEQ_STAGE(kStAttnFwd, main,
@@ -321,7 +375,7 @@ int moc_seq_layer_fwd(const void* h, const void* bank, const void* wr, int wr_dt
                                         L, H, HK, 64, 64, y.NS, 0.125f, attn, lse, y.xws_bytes ? sv + y.xws_f : nullptr,
                                         y.xws_bytes, main)));
   SEQ_STAGE(kStOProj, main, SEQ_TRY(moc_rows_linear(attn, d, tok, wo, (int)d, (int)d, out, d, main)));
-  MOC_HIP(hipStreamWaitEvent(main, ev[2], 0));
+  if (train) MOC_HIP(hipStreamWaitEvent(main, ev[2], 0));   // (else the wait on ev[1] joined the aux stream)
   join.disarm();
   return MOC_OK;
 }
@@ -332,6 +386,17 @@ int moc_seq_layer_bwd(const void* h, const void* bank, const void* wr, int wr_dt
                       size_t saved_bytes, const void* dout, const float* dlogits, void* dh, void* dbank,
                       int64_t bank_rows, float* dwr, float* dbr, void* dwq, void* dwkv, int dwkv_dtype, void* dwo,
                       void* scratch, size_t scratch_bytes, hipStream_t main, hipStream_t aux, hipStream_t fill) {
+  return moc_seq_layer_bwd_ex(h, bank, wr, wr_dtype, coef, B, L, d, H, HK, C, S, k, routed_scale, MOC_NORM_NONE, logits,
+                              idx, omega, saved, saved_bytes, dout, dlogits, dh, dbank, bank_rows, dwr, dbr, dwq, dwkv,
+                              dwkv_dtype, dwo, scratch, scratch_bytes, main, aux, fill);
+}
+
+int moc_seq_layer_bwd_ex(const void* h, const void* bank, const void* wr, int wr_dtype, const float* coef, int64_t B,
+                         int64_t L, int64_t d, int H, int HK, int64_t C, int S, int k, float routed_scale, int norm,
+                         const float* logits, const int32_t* idx, const float* omega, const void* saved,
+                         size_t saved_bytes, const void* dout, const float* dlogits, void* dh, void* dbank,
+                         int64_t bank_rows, float* dwr, float* dbr, void* dwq, void* dwkv, int dwkv_dtype, void* dwo,
+                         void* scratch, size_t scratch_bytes, hipStream_t main, hipStream_t aux, hipStream_t fill) {
   MOC_REQUIRE(h && bank && wr && logits && idx && omega && saved && dout && scratch, MOC_ERR_ARG,
               "moc_seq_layer_bwd: null pointer");
   MOC_REQUIRE(main != aux && main != fill && aux != fill, MOC_ERR_ARG,
@@ -339,7 +404,7 @@ int moc_seq_layer_bwd(const void* h, const void* bank, const void* wr, int wr_dt
   MOC_REQUIRE(dwkv_dtype == MOC_BF16 || dwkv_dtype == MOC_F32, MOC_ERR_UNSUPPORTED,
               "moc_seq_layer_bwd: dwkv dtype %d", dwkv_dtype);
   SeqLayout y;
-  SEQ_TRY(y.init(B, L, d, H, HK, C, S, k));
+  SEQ_TRY(y.init(B, L, d, H, HK, C, S, k, norm, true));
   MOC_REQUIRE(saved_bytes >= y.saved_bytes && scratch_bytes >= y.scratch_bytes, MOC_ERR_ARG,
               "moc_seq_layer_bwd: saved %zu < %zu or scratch %zu < %zu bytes", saved_bytes, y.saved_bytes,
               scratch_bytes, y.scratch_bytes);
@@ -437,7 +502,7 @@ int moc_seq_layer_bwd(const void* h, const void* bank, const void* wr, int wr_dt
                                             main)));
   if (dwkv)
     SEQ_STAGE(kStKVWgrad, main,
-              SEQ_TRY(chapter_wgrad_budget(dkv_edge, KV2, red, bank, d, 1, uniq, n_uniq, y.max_u, csr_off, csr_edge,
+              SEQ_TRY(chapter_wgrad_budget(dkv_edge, KV2, red, norm ? (const void*)(sv + y.xn) : bank, d, norm ? 0 : 1, uniq, n_uniq, y.max_u, csr_off, csr_edge,
                                            KV2, (int)d, sc + y.cw_ws, y.cw_ws_bytes, dwkv_dtype, dwkv,
                                            kSeqWgradBudget, main)));
   if (dbank) {
@@ -445,9 +510,17 @@ int moc_seq_layer_bwd(const void* h, const void* bank, const void* wr, int wr_dt
     // dK/dV and has ended long before (waited for right after dQ, the step waited ~20 us for
     // it once dQ took its tiles by LDS DMA)
     MOC_HIP(hipStreamWaitEvent(main, ev[2], 0));
-    SEQ_STAGE(kStBankDx, main,
-              SEQ_TRY(moc_chapter_dx(dkv_edge, KV2, uniq, n_uniq, y.max_u, csr_off, csr_edge, red, sv + y.wkv_t,
-                                     (int)d, KV2, MOC_BF16, dbank, d, 1, main)));
+    SEQ_STAGE(kStBankDx, main, {
+      if (norm == MOC_NORM_NONE) {
+        SEQ_TRY(moc_chapter_dx(dkv_edge, KV2, uniq, n_uniq, y.max_u, csr_off, csr_edge, red, sv + y.wkv_t, (int)d, KV2,
+                               MOC_BF16, dbank, d, 1, main));
+      } else {
+        SEQ_TRY(moc_chapter_dx(dkv_edge, KV2, uniq, n_uniq, y.max_u, csr_off, csr_edge, red, sv + y.wkv_t, (int)d, KV2,
+                               MOC_F32, sc + y.dxc, d, 0, main));
+        SEQ_TRY(moc_bank_scatter(MOC_F32, sc + y.dxc, bank, MOC_BF16, d, 64, uniq, n_uniq, y.max_u, nullptr, nullptr,
+                                 (const float*)(sv + y.mean), (const float*)(sv + y.rstd), norm, dbank, main));
+      }
+    });
   }
   MOC_HIP(hipStreamWaitEvent(main, ev[5], 0));
   if (dwq) MOC_HIP(hipStreamWaitEvent(main, ev[7], 0));

@@ -22,15 +22,19 @@ backward   main stream: o_proj dX -> attention backward (dQ, then dK/dV) -> K/V 
 Every tensor the aux stream writes and the caller sees is allocated on the main stream before
 the fork, so the caching allocator never hands its memory to another stream early.
 
-For a plain bf16 bank (no row norm, no BankAdamW mirror, no row-sparse gradient) the same schedule
-runs natively: moc_seq_layer_fwd / moc_seq_layer_bwd issue every launch, event and stream wait
-from C++ (the q / o projections on the chapter GEMM, their transposed weights packed in the
+For a bf16 bank, row-normalised or not (no BankAdamW mirror, no row-sparse gradient), the same
+schedule runs natively: moc_seq_layer_fwd_ex / moc_seq_layer_bwd_ex issue every launch, event and stream
+wait from C++ (the q / o projections on the chapter GEMM, their transposed weights packed in the
 forward), so a training step costs two host calls; PyTorch only allocates the outputs, one saved
-buffer and one scratch buffer.  ``NATIVE = False`` keeps the Python-scheduled sequence.
+buffer and one scratch buffer.  A forward that no backward follows (grad mode off, or no input that
+requires a gradient) leaves out what only the backward reads, and its buffer is a temporary.
+``NATIVE = False`` keeps the Python-scheduled sequence.
 """
 
 from __future__ import annotations
 
+import ctypes
+import functools
 from typing import Optional
 
 import torch
@@ -54,25 +58,35 @@ def supported(h: torch.Tensor, bank: torch.Tensor, wq: torch.Tensor, wo: torch.T
 NATIVE = True
 
 
-def _native_saved_bytes(h, bank, wr, br, wq, wk, wv, wo, cfg) -> int:
-    """Bytes of the native path's saved buffer, or 0 when the layer's configuration is outside
-    moc_seq_layer_fwd / _bwd (those then run as the Python-scheduled sequence below)."""
+@functools.lru_cache(maxsize=256)
+def _layer_sizes(B, Lq, d, H, HK, C, S, k, norm):
+    """(saved, scratch, inference) buffer bytes of the native layer, or None for shapes outside it."""
+    n = (ctypes.c_size_t * 3)()
+    at = [ctypes.addressof(n) + i * ctypes.sizeof(ctypes.c_size_t) for i in range(3)]
+    return tuple(n) if L.query("moc_seq_layer_sizes", B, Lq, d, H, HK, C, S, k, norm, *at) == L.MOC_OK else None
+
+
+def _native_sizes(h, bank, br, wq, wk, wv, wo, cfg):
+    """_layer_sizes of a call that moc_seq_layer_fwd_ex / _bwd_ex take, or None (such calls run as the
+    Python-scheduled sequence below)."""
     if not NATIVE:
-        return 0
-    C, T, S, k, scale, H, HK, norm, eps = cfg
+        return None
+    C, T, S, k, scale, H, HK, norm, eps, _train = cfg
     B, Lq, d = h.shape
-    if (norm != L.MOC_NORM_NONE or bank.dtype != torch.bfloat16 or bank.dim() != 2 or bank.shape[1] != d
-            or T != 64 or d != 64 * H or any(t.dtype != torch.bfloat16 for t in (wq, wk, wv, wo))
+    bf = torch.bfloat16
+    if (bank.dtype != bf or bank.dim() != 2 or bank.shape[1] != d or T != 64 or d != 64 * H or d > 4096
+            or wq.dtype != bf or wk.dtype != bf or wv.dtype != bf or wo.dtype != bf
+            or (norm != L.MOC_NORM_NONE and bank.data_ptr() % 16)     # rows read in 16-byte pieces
             or getattr(bank, "_moc_bank_opt", None) is not None or getattr(bank, "_moc_row_grad", None) is not None
-            or (br is not None and br.dtype not in (torch.float32, torch.bfloat16))):
-        return 0
-    return int(L.query("moc_seq_layer_saved_bytes", B, Lq, d, H, HK, C, S, k))
+            or (br is not None and br.dtype not in (torch.float32, bf))):
+        return None
+    return _layer_sizes(B, Lq, d, H, HK, C, S, k, norm)
 
 
 class _SeqRoutedLayer(torch.autograd.Function):
     @staticmethod
     def forward(ctx, h, bank, wr, br, wq, wk, wv, wo, coef, cfg):
-        C, T, S, k, scale, H, HK, norm, eps = cfg
+        C, T, S, k, scale, H, HK, norm, eps, train = cfg
         dev = h.device
         B, Lq, d = h.shape
         Dh = d // H
@@ -82,10 +96,12 @@ class _SeqRoutedLayer(torch.autograd.Function):
         ctx.cfg = cfg
         ctx.wdt = (wr.dtype, None if br is None else br.dtype)
         ctx.set_materialize_grads(False)
-        nbytes = _native_saved_bytes(h, bank, wr, br, wq, wk, wv, wo, cfg)
-        ctx.native = nbytes > 0
+        sizes = _native_sizes(h, bank, br, wq, wk, wv, wo, cfg)
+        ctx.native = sizes is not None
         if ctx.native:
-            # the whole forward in one host call (moc_seq_layer_fwd)
+            # the whole forward in one host call (moc_seq_layer_fwd_ex); without a backward to come
+            # `saved` is a temporary
+            nbytes = sizes[0] if train else sizes[2]
             main = torch.cuda.current_stream(dev)
             aux = ops._side_stream(dev, "aux")
             wrc = wr.contiguous()
@@ -98,10 +114,13 @@ class _SeqRoutedLayer(torch.autograd.Function):
             idx_star = torch.empty(B, NS, device=dev, dtype=torch.int32)
             omega = torch.empty(B, NS, device=dev, dtype=torch.float32)
             wq, wk, wv, wo, bank = wq.contiguous(), wk.contiguous(), wv.contiguous(), wo.contiguous(), bank.contiguous()
-            call("moc_seq_layer_fwd", ptr(h), ptr(bank), ptr(wrc), L.dtype_code(wrc.dtype), ptr(brc), ptr(wq),
-                 ptr(wk), ptr(wv), ptr(wo), ptr(cf), B, Lq, d, H, HK, C, S, k, float(scale), ptr(out), ptr(logits),
-                 ptr(idx), ptr(idx_star), ptr(omega), ptr(saved), nbytes, main.cuda_stream, aux.cuda_stream)
-            ctx.save_for_backward(h, bank, wrc, cf, logits, idx, omega, saved)
+            call("moc_seq_layer_fwd_ex", ptr(h), ptr(bank), ptr(wrc), L.dtype_code(wrc.dtype), ptr(brc), ptr(wq),
+                 ptr(wk), ptr(wv), ptr(wo), ptr(cf), B, Lq, d, H, HK, C, S, k, scale, norm, eps, 1 if train else 0,
+                 ptr(out), ptr(logits), ptr(idx), ptr(idx_star), ptr(omega), ptr(saved), nbytes, main.cuda_stream,
+                 aux.cuda_stream)
+            if train:
+                ctx.save_for_backward(h, bank, wrc, cf, logits, idx, omega, saved)
+                ctx.nscratch = sizes[1]
             ctx.mark_non_differentiable(idx, idx_star, omega)
             return out, logits, idx, idx_star, omega
         h2 = h.view(B * Lq, d)
@@ -156,7 +175,7 @@ class _SeqRoutedLayer(torch.autograd.Function):
             return _native_backward(ctx, dout, dlogits)
         h, wrc, wqc, wo, pooled, logits, idx, w, cf = ctx.saved_tensors[:9]
         saved = ctx.saved_tensors[9:]
-        C, T, S, k, scale, H, HK, norm, eps = ctx.cfg
+        C, T, S, k, scale, H, HK, norm, eps, _train = ctx.cfg
         need_h, need_bank, need_wr, need_br, need_wq, need_wk, need_wv, need_wo = ctx.needs_input_grad[:8]
         dev = h.device
         B, Lq, d = h.shape
@@ -234,9 +253,9 @@ class _SeqRoutedLayer(torch.autograd.Function):
 
 
 def _native_backward(ctx, dout, dlogits):
-    """The whole backward in one host call (moc_seq_layer_bwd)."""
+    """The whole backward in one host call (moc_seq_layer_bwd_ex)."""
     h, bank, wrc, cf, logits, idx, omega, saved = ctx.saved_tensors
-    C, T, S, k, scale, H, HK, norm, eps = ctx.cfg
+    C, T, S, k, scale, H, HK, norm, eps, _train = ctx.cfg
     need_h, need_bank, need_wr, need_br, need_wq, need_wk, need_wv, need_wo = ctx.needs_input_grad[:8]
     dev = h.device
     B, Lq, d = h.shape
@@ -252,13 +271,13 @@ def _native_backward(ctx, dout, dlogits):
     dwq = torch.empty(d, d, device=dev, dtype=torch.bfloat16) if need_wq else None
     dwkv = torch.empty(2 * KV, d, device=dev, dtype=torch.bfloat16) if (need_wk or need_wv) else None
     dwo = torch.empty(d, d, device=dev, dtype=torch.bfloat16) if need_wo else None
-    nscratch = int(L.query("moc_seq_layer_scratch_bytes", B, Lq, d, H, HK, C, S, k))
+    nscratch = ctx.nscratch
     scratch = torch.empty(nscratch, device=dev, dtype=torch.uint8)
     main = torch.cuda.current_stream(dev)
     aux = ops._side_stream(dev, "aux")
     fill = ops._side_stream(dev, "fill")
-    call("moc_seq_layer_bwd", ptr(h), ptr(bank), ptr(wrc), L.dtype_code(wrc.dtype), ptr(cf), B, Lq, d, H, HK, C, S, k,
-         float(scale), ptr(logits), ptr(idx), ptr(omega), ptr(saved), saved.numel(), ptr(dout), ptr(dz_in), ptr(dh),
+    call("moc_seq_layer_bwd_ex", ptr(h), ptr(bank), ptr(wrc), L.dtype_code(wrc.dtype), ptr(cf), B, Lq, d, H, HK, C, S,
+         k, scale, norm, ptr(logits), ptr(idx), ptr(omega), ptr(saved), saved.numel(), ptr(dout), ptr(dz_in), ptr(dh),
          ptr(dbank), bank.shape[0], ptr(dwr), ptr(dbr), ptr(dwq), ptr(dwkv), L.MOC_BF16, ptr(dwo), ptr(scratch),
          nscratch, main.cuda_stream, aux.cuda_stream, fill.cuda_stream)
     dwk = dwkv[:KV] if need_wk else None
@@ -274,6 +293,9 @@ def seq_routed_layer(h, bank, wr, br, wq, wk, wv, wo, *, num_chapters: int, toke
                      num_shared: int, top_k: int, routed_scale: float, num_heads: int, num_kv_heads: int,
                      norm_type: Optional[str] = None, eps: float = 1e-6, coef: Optional[torch.Tensor] = None):
     """(out (B, L, d), logits f32 (B, C), idx int32 (B, k), idx_star int32 (B, S+k), omega f32 (B, S+k))."""
+    # grad mode is read here: it is off inside the function's forward
+    train = torch.is_grad_enabled() and any(t is not None and t.requires_grad
+                                            for t in (h, bank, wr, br, wq, wk, wv, wo))
     cfg = (int(num_chapters), int(tokens_per_chapter), int(num_shared), int(top_k), float(routed_scale),
-           int(num_heads), int(num_kv_heads), ops.norm_code(norm_type), float(eps))
+           int(num_heads), int(num_kv_heads), ops.norm_code(norm_type), float(eps), train)
     return _SeqRoutedLayer.apply(h, bank, wr, br, wq, wk, wv, wo, coef, cfg)

@@ -57,7 +57,7 @@ def _layer(dev, dtype, Wr, br, Wq, Wk, Wv, Wo, normalize, strategy="sequence", w
 @pytest.mark.parametrize("Lq", [128, 96])
 def test_config1_layer_forward_backward(gpu_device, monkeypatch, dtype, fused, normalize, strategy, window, Lq):
     """bf16 runs the whole-layer autograd function (memory_amd.seq_layer) with its native
-    schedule (moc_seq_layer_fwd / _bwd; a normalised bank takes the Python-scheduled one) and
+    schedule (moc_seq_layer_fwd_ex / _bwd_ex, a normalised bank included) and
     with the Python-scheduled one, and the per-op functions; fp32 always takes the per-op path."""
     from memory_amd import seq_layer
     print(f"config1 layer dtype={dtype} fused={fused} normalize={normalize} strategy={strategy} L={Lq}", flush=True)
