@@ -147,7 +147,8 @@ def compute_total_router_loss(losses: Dict[str, torch.Tensor], load_balance_coef
         if reference_tensor is not None:
             return reference_tensor.new_tensor(0.0)
         return torch.tensor(0.0)
-    total = next(iter(losses.values())).new_tensor(0.0)
+    # (new_zeros fills on the device; new_tensor would copy from host memory and wait for the stream)
+    total = next(iter(losses.values())).new_zeros(())
     if "load_balance" in losses and load_balance_coef > 0:
         total = total + load_balance_coef * losses["load_balance"]
     if "auxiliary" in losses and auxiliary_coef > 0:
