@@ -507,6 +507,14 @@ int moc_bank_grad_accumulate(int dx_dtype, const void* dX, const void* bank, int
 
 /* ------------------------------------------------------------ few-row linear */
 
+/* Small float32 products c [M][N] (row stride ldc) = op(a) op(b) on the fp32 matrix cores: a is [M][K]
+ * (row stride lda) or, ta, [K][M]; b is [K][N] or, tb, [N][K].  Exact fp32 operands and accumulation
+ * (nn.Linear and its gradients in float32, memory_attention.py:140-143).  16-byte aligned operands, N
+ * and the strides of operands with a contiguous reduction multiples of 4; moc_gemm_f32_takes says
+ * whether a size is one of the small ones (larger products belong to a library GEMM). */
+int moc_gemm_f32_takes(int ta, int tb, int64_t M, int64_t N, int64_t K);
+int moc_gemm_f32(int ta, int tb, int64_t M, int64_t N, int64_t K, const float* a, int64_t lda, const float* b,
+                 int64_t ldb, float* c, int64_t ldc, hipStream_t stream);
 /* y [M][N] = x [M][K] W[N][K]^T for M <= 256 rows (bf16 x and W, fp32 accumulation, y bf16 or
  * f32): the decode step's q_proj / o_proj (memory_attention.py:140-143, :241, :456) on one
  * token per sequence.  K % 128 == 0, N % 16 == 0, 16-byte aligned x and W. */

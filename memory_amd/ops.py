@@ -7,6 +7,7 @@ allocator), the current stream and autograd bookkeeping only.
 
 from __future__ import annotations
 
+import functools
 from dataclasses import dataclass
 from typing import Optional
 
@@ -328,6 +329,26 @@ def rows_gemm_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
             and K % 64 == 0)
 
 
+@functools.lru_cache(maxsize=1024)
+def _gemm_f32_takes(ta: bool, tb: bool, M: int, N: int, K: int) -> bool:
+    return bool(L.query("moc_gemm_f32_takes", int(ta), int(tb), M, N, K))
+
+
+def matmul2d(a: torch.Tensor, b: torch.Tensor, ta: bool = False, tb: bool = False) -> torch.Tensor:
+    """op(a) op(b) of 2-D tensors (ta / tb: transposed).  Small float32 products run on
+    moc_gemm_f32, everything else on the library."""
+    if a.dtype == torch.float32 and b.dtype == torch.float32 and a.is_cuda and b.is_cuda:
+        K, M = a.shape if ta else a.shape[::-1]
+        N, Kb = b.shape if tb else b.shape[::-1]
+        if (K == Kb and _gemm_f32_takes(ta, tb, M, N, K) and a.is_contiguous() and b.is_contiguous()
+                and a.data_ptr() % 16 == 0 and b.data_ptr() % 16 == 0):
+            c = torch.empty(M, N, device=a.device, dtype=torch.float32)
+            call("moc_gemm_f32", int(ta), int(tb), M, N, K, ptr(a), a.shape[1], ptr(b), b.shape[1], ptr(c), N,
+                 stream_ptr(a.device))
+            return c
+    return torch.matmul(a.t() if ta else a, b.t() if tb else b)
+
+
 class _Linear(torch.autograd.Function):
     """y = x W^T (bias-free nn.Linear of the memory layer's q_proj / o_proj,
     memory_transformer/memory_attention.py:140-143, :241 and :456).  The weight gradient
@@ -341,6 +362,8 @@ class _Linear(torch.autograd.Function):
         if _few_rows(x, w):
             return linear_rows(x, w)
         with L.region("lib_linear_fwd"):
+            if x.dtype == torch.float32:
+                return matmul2d(x.reshape(-1, x.shape[-1]), w, tb=True).view(*x.shape[:-1], w.shape[0])
             return F.linear(x, w)
 
     @staticmethod
@@ -349,7 +372,10 @@ class _Linear(torch.autograd.Function):
         dx = dw = None
         if ctx.needs_input_grad[0]:
             with L.region("lib_linear_dx"):
-                dx = torch.matmul(dy, w)
+                if dy.dtype == torch.float32:
+                    dx = matmul2d(dy.reshape(-1, dy.shape[-1]), w).view(*dy.shape[:-1], w.shape[1])
+                else:
+                    dx = torch.matmul(dy, w)
         if ctx.needs_input_grad[1]:
             n_out, n_in = w.shape
             dy2 = dy.reshape(-1, n_out).contiguous()
@@ -399,7 +425,8 @@ class _LinearResidual(torch.autograd.Function):
                  n_out, ptr(out), n_out, stream_ptr(x.device))
             return out.view(residual.shape)
         with L.region("lib_linear_fwd"):
-            out = residual.reshape(-1, n_out) + F.linear(x2, w)
+            out = residual.reshape(-1, n_out) + (matmul2d(x2, w, tb=True) if x2.dtype == torch.float32
+                                                  else F.linear(x2, w))
         return out.view(residual.shape)
 
     @staticmethod
@@ -417,7 +444,7 @@ class _LinearResidual(torch.autograd.Function):
                 dx = rows_linear(g, wt).view(x.shape)
             else:
                 with L.region("lib_linear_dx"):
-                    dx = torch.matmul(g, w.to(x.dtype)).view(x.shape)
+                    dx = matmul2d(g, w.to(x.dtype)).view(x.shape)
         if ctx.needs_input_grad[1]:
             dw = linear_wgrad(g, x.reshape(-1, n_in).contiguous(), w.dtype)
         return dx, dw, dres
@@ -583,6 +610,8 @@ def linear_wgrad(dy: torch.Tensor, x: torch.Tensor, out_dtype: torch.dtype,
     tensor of out_dtype to write (allocated here when None)."""
     R, N = dy.shape
     K = x.shape[1]
+    if out is None and dy.dtype == x.dtype == out_dtype == torch.float32:
+        return matmul2d(dy, x, ta=True)
     dw = torch.empty(N, K, device=dy.device, dtype=out_dtype) if out is None else out
     if (dy.dtype == torch.bfloat16 and x.dtype in (torch.bfloat16, torch.float32) and dy.is_cuda and N % 8 == 0
             and K % 8 == 0 and out_dtype in (torch.float32, torch.bfloat16)):
@@ -666,7 +695,7 @@ def routed_attn_forward(q, bank, wk, wv, omega, idx_star, num_chapters, T, norm,
         call("moc_gather_rows", L.dtype_code(dtype), ptr(bank), L.dtype_code(bank.dtype), d, T,
              ptr(plan.uniq), ptr(plan.n_uniq), plan.max_u, ptr(mean), ptr(rstd), ptr(X), stream_ptr(q.device))
         with L.region("lib_kv_project_gemm"):
-            kv = F.linear(X, wkv)
+            kv = matmul2d(X, wkv, tb=True)
         del X
     kvl = kv_rows_layout(kv, T, HK, Dh)
     om = omega.float().contiguous()
@@ -826,11 +855,11 @@ def routed_attn_backward(saved, cfg, dout, needs, row_grad=None, after_dq=None, 
         X = torch.empty(max_u * T, d, device=dev, dtype=dtype)
         call("moc_gather_rows", dt, ptr(bank), L.dtype_code(bank.dtype), d, T, ptr(uniq), ptr(n_uniq),
              max_u, ptr(mean), ptr(rstd), ptr(X), st)
-        dwkv = torch.matmul(dkv.t(), X)
+        dwkv = matmul2d(dkv, X, ta=True)
         dwk = dwkv[:KV].to(wk_dtype) if need_wk else None
         dwv = dwkv[KV:].to(wv_dtype) if need_wv else None
     if need_bank:
-        dX = torch.matmul(dkv, wkv)
+        dX = matmul2d(dkv, wkv)
         if row_grad is not None:
             row_grad.accumulate(dX, bank, uniq, n_uniq, max_u, None, None, mean, rstd, norm)
         else:
