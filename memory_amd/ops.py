@@ -336,8 +336,11 @@ def _gemm_f32_takes(ta: bool, tb: bool, M: int, N: int, K: int) -> bool:
 
 def matmul2d(a: torch.Tensor, b: torch.Tensor, ta: bool = False, tb: bool = False) -> torch.Tensor:
     """op(a) op(b) of 2-D tensors (ta / tb: transposed).  Small float32 products run on
-    moc_gemm_f32, everything else on the library."""
-    if a.dtype == torch.float32 and b.dtype == torch.float32 and a.is_cuda and b.is_cuda:
+    moc_gemm_f32; everything else on the library, autocast and a backward that is itself recorded
+    (create_graph) included."""
+    if (a.dtype == torch.float32 and b.dtype == torch.float32 and a.is_cuda and b.is_cuda
+            and not torch.is_autocast_enabled()
+            and not (torch.is_grad_enabled() and (a.requires_grad or b.requires_grad))):
         K, M = a.shape if ta else a.shape[::-1]
         N, Kb = b.shape if tb else b.shape[::-1]
         if (K == Kb and _gemm_f32_takes(ta, tb, M, N, K) and a.is_contiguous() and b.is_contiguous()

@@ -47,3 +47,21 @@ def test_matmul2d_routes(gpu_device):
         assert ((ops.matmul2d(a, b, tb=True).double() - ref).norm() / ref.norm()).item() < tol
     with pytest.raises(RuntimeError):
         ops.matmul2d(x, w)
+
+
+def test_recorded_backward_and_autocast(gpu_device):
+    """A backward that is itself differentiated, and autocast, keep the library's products."""
+    from memory_amd import ops
+    dev = gpu_device
+    g = gen(4)
+    x, w, u = (torch.randn(*s, generator=g).to(dev) for s in ((80, 64), (64, 64), (80, 64)))
+    second = []
+    for f in (ops.linear, torch.nn.functional.linear):
+        a, b = x.clone().requires_grad_(), w.clone().requires_grad_()
+        ga, gb = torch.autograd.grad(f(a, b), (a, b), u, create_graph=True)
+        (ga.square().sum() + gb.square().sum()).backward()
+        second.append((a.grad, b.grad))
+    for got, want in zip(*second):
+        assert ((got - want).norm() / want.norm()).item() < 1e-5
+    with torch.autocast("cuda", torch.bfloat16):
+        assert ops.matmul2d(x, w, tb=True).dtype == torch.bfloat16
