@@ -353,6 +353,23 @@ int moc_seq_layer_bwd_ex(const void* h, const void* bank, const void* wr, int wr
                          size_t saved_bytes, const void* dout, const float* dlogits, void* dh, void* dbank,
                          int64_t bank_rows, float* dwr, float* dbr, void* dwq, void* dwkv, int dwkv_dtype, void* dwo,
                          void* scratch, size_t scratch_bytes, hipStream_t main, hipStream_t aux, hipStream_t fill);
+/* The float32 layer in one host call each way, on one stream, for sizes whose products moc_gemm_f32's
+ * tiles serve (moc_seq_layer_f32_sizes returns an error status for others): arguments as
+ * moc_seq_layer_fwd_ex / _bwd_ex with float32 tensors; dwkv [2*HK*64][d]. */
+int moc_seq_layer_f32_sizes(int64_t B, int64_t L, int64_t d, int H, int HK, int64_t C, int S, int k, int norm,
+                            size_t* saved, size_t* scratch);
+int moc_seq_layer_f32_fwd(const float* h, const float* bank, const void* wr, int wr_dtype, const float* br,
+                          const float* wq, const float* wk, const float* wv, const float* wo, const float* coef,
+                          int64_t B, int64_t L, int64_t d, int H, int HK, int64_t C, int S, int k, float routed_scale,
+                          int norm, float eps, float* out, float* logits, int32_t* idx, int32_t* idx_star, float* omega,
+                          void* saved, size_t saved_bytes, hipStream_t st);
+int moc_seq_layer_f32_bwd(const float* h, const float* bank, const void* wr, int wr_dtype, const float* wq,
+                          const float* wk, const float* wv, const float* wo, const float* coef, int64_t B, int64_t L,
+                          int64_t d, int H, int HK, int64_t C, int S, int k, float routed_scale, int norm,
+                          const float* logits, const int32_t* idx, const float* omega, const void* saved,
+                          size_t saved_bytes, const float* dout, const float* dlogits, float* dh, float* dbank,
+                          int64_t bank_rows, float* dwr, float* dbr, float* dwq, float* dwkv, float* dwo, void* scratch,
+                          size_t scratch_bytes, hipStream_t st);
 /* Stage timing of the two calls above (no counterpart in the reference, which times whole steps
  * with torch.cuda.Event in its benchmarks, kernels-final/benchmark_kernels_final.py): stage s is
  * one or a few launches on one stream, named by moc_seq_layer_stage_name(s) (the entry point

@@ -52,6 +52,11 @@ _SIGS = {
                                   _I, _F, _I, _P, _P, _P, _P, _P, _P, _SZ, _P, _P]),
     "moc_seq_layer_bwd_ex": (_I, [_P, _P, _P, _I, _P, _I64, _I64, _I64, _I, _I, _I64, _I, _I, _F, _I, _P, _P, _P, _P,
                                   _SZ, _P, _P, _P, _P, _I64, _P, _P, _P, _P, _I, _P, _P, _SZ, _P, _P, _P]),
+    "moc_seq_layer_f32_sizes": (_I, [_I64, _I64, _I64, _I, _I, _I64, _I, _I, _I, _P, _P]),
+    "moc_seq_layer_f32_fwd": (_I, [_P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I, _I, _I64, _I, _I, _F,
+                                   _I, _F, _P, _P, _P, _P, _P, _P, _SZ, _P]),
+    "moc_seq_layer_f32_bwd": (_I, [_P, _P, _P, _I, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I, _I, _I64, _I, _I, _F, _I,
+                                   _P, _P, _P, _P, _SZ, _P, _P, _P, _P, _I64, _P, _P, _P, _P, _P, _P, _SZ, _P]),
     "moc_seq_layer_stage_count": (_I, []),
     "moc_seq_layer_stage_name": (ctypes.c_char_p, [_I]),
     "moc_seq_layer_timing": (_I, [ctypes.c_uint64, _I]),

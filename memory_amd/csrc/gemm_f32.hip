@@ -37,7 +37,7 @@ __device__ __forceinline__ f32x8 gf_load(const float* __restrict__ p, int64_t ld
 template <bool AK, bool BK>
 __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__ a, int64_t lda,
                                                        const float* __restrict__ b, int64_t ldb, int M, int N, int K,
-                                                       float* __restrict__ c, int64_t ldc) {
+                                                       float* __restrict__ c, int64_t ldc, int add) {
   __shared__ f32x4 red[4][8][64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int g = lane >> 4, c16 = lane & 15;
@@ -79,8 +79,34 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
 #pragma unroll
     for (int w = 1; w < 4; ++w) s += red[w][tile][lane];
     const int m = m0 + 16 * j + c16, n = n0 + 16 * i + 4 * g;
-    if (m < M && n < N) *reinterpret_cast<f32x4*>(c + (int64_t)m * ldc + n) = s;   // N % 4 == 0
+    if (m < M && n < N) {   // N % 4 == 0
+      f32x4* o = reinterpret_cast<f32x4*>(c + (int64_t)m * ldc + n);
+      *o = add ? *o + s : s;
+    }
   }
+}
+
+int gemm_f32(int ta, int tb, int64_t M, int64_t N, int64_t K, const float* a, int64_t lda, const float* b, int64_t ldb,
+             float* c, int64_t ldc, int add, hipStream_t stream) {
+  MOC_REQUIRE(M > 0 && N > 0 && K > 0 && N % 4 == 0 && M < (1 << 21) && N < (1 << 21) && K < (1 << 21) &&
+                  ((ta && !tb) || K % 8 == 0),
+              MOC_ERR_UNSUPPORTED, "moc_gemm_f32: M=%lld, N=%lld, K=%lld", (long long)M, (long long)N, (long long)K);
+  MOC_REQUIRE(lda >= (ta ? M : K) && ldb >= (tb ? K : N) && ldc >= N && ldc % 4 == 0 && (ta || lda % 4 == 0) &&
+                  (!tb || ldb % 4 == 0) && (((uintptr_t)a | (uintptr_t)b | (uintptr_t)c) & 15) == 0,
+              MOC_ERR_ARG, "moc_gemm_f32: row strides %lld, %lld, %lld (multiples of 4, 16-byte aligned operands)",
+              (long long)lda, (long long)ldb, (long long)ldc);
+  const dim3 grid((unsigned)((N + kGfCols - 1) / kGfCols), (unsigned)((M + kGfRows - 1) / kGfRows));
+  MOC_REQUIRE(grid.y < 65536, MOC_ERR_UNSUPPORTED, "moc_gemm_f32: M=%lld", (long long)M);
+#define GF(AK, BK)                                                                                                   \
+  hipLaunchKernelGGL((gemm_f32_kernel<AK, BK>), grid, dim3(256), 0, stream, a, lda, b, ldb, (int)M, (int)N, (int)K, \
+                     c, ldc, add)
+  if (!ta) {
+    if (tb) GF(true, true); else GF(true, false);
+  } else {
+    if (tb) GF(false, true); else GF(false, false);
+  }
+#undef GF
+  return check_launch("gemm_f32_kernel");
 }
 
 }  // namespace moc
@@ -105,22 +131,7 @@ int moc_gemm_f32(int ta, int tb, int64_t M, int64_t N, int64_t K, const float* a
   MOC_REQUIRE(a && b && c, MOC_ERR_ARG, "moc_gemm_f32: null pointer");
   MOC_REQUIRE(moc_gemm_f32_takes(ta, tb, M, N, K), MOC_ERR_UNSUPPORTED, "moc_gemm_f32: M=%lld, N=%lld, K=%lld",
               (long long)M, (long long)N, (long long)K);
-  MOC_REQUIRE(lda >= (ta ? M : K) && ldb >= (tb ? K : N) && ldc >= N && ldc % 4 == 0 && (ta || lda % 4 == 0) &&
-                  (!tb || ldb % 4 == 0) && (((uintptr_t)a | (uintptr_t)b | (uintptr_t)c) & 15) == 0,
-              MOC_ERR_ARG, "moc_gemm_f32: row strides %lld, %lld, %lld (multiples of 4, 16-byte aligned operands)",
-              (long long)lda, (long long)ldb, (long long)ldc);
-  const dim3 grid((unsigned)((N + kGfCols - 1) / kGfCols), (unsigned)((M + kGfRows - 1) / kGfRows));
-  MOC_REQUIRE(grid.y < 65536, MOC_ERR_UNSUPPORTED, "moc_gemm_f32: M=%lld", (long long)M);
-#define GF(AK, BK)                                                                                                   \
-  hipLaunchKernelGGL((gemm_f32_kernel<AK, BK>), grid, dim3(256), 0, stream, a, lda, b, ldb, (int)M, (int)N, (int)K, \
-                     c, ldc)
-  if (!ta) {
-    if (tb) GF(true, true); else GF(true, false);
-  } else {
-    if (tb) GF(false, true); else GF(false, false);
-  }
-#undef GF
-  return check_launch("gemm_f32_kernel");
+  return gemm_f32(ta, tb, M, N, K, a, lda, b, ldb, c, ldc, 0, stream);
 }
 
 }  // extern "C"

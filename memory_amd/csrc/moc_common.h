@@ -371,6 +371,10 @@ bool mid_linear_takes(int64_t M, int N, int K);
 int mid_linear(const void* x, int64_t ldx, int64_t M, const void* w, int N, int K, void* y, int64_t ldy,
                const void* res, int64_t ldr, hipStream_t stream);
 
+// moc_gemm_f32 of any size it can index, with c += op(a) op(b) when `add` is set (gemm_f32.hip).
+int gemm_f32(int ta, int tb, int64_t M, int64_t N, int64_t K, const float* a, int64_t lda, const float* b, int64_t ldb,
+             float* c, int64_t ldc, int add, hipStream_t stream);
+
 // out[i] = inv * sum_j part[j * n + i] for i < n, j < nsplit, summed in a fixed order
 // (router.hip's split-row reduction); returns a MOC_ status.
 int launch_split_reduce(const float* part, int nsplit, int64_t n, float inv, float* out, hipStream_t stream);

@@ -65,6 +65,13 @@ int seq_events(hipEvent_t** out) {
   return MOC_OK;
 }
 
+// Multiply-adds of one d x d projection of the tokens plus one K or V projection of the rows up to which
+// the float32 layer runs as one host call on moc_gemm_f32.  A training step against the per-op functions,
+// which need 600 to 850 us of host time at any size: 295 against 693 us at 2 x 128 tokens of d = 256 with
+// 10 chapters (2.7e7), 501 against 853 at 8 x 512 with 56 (5.0e8), 746 against 830 at 8 x 1,024 with 40
+// (7.0e8); past the line the library's larger tiles win, 1,021 against 829 at 8 x 1,024 with 128 (1.1e9).
+constexpr int64_t kSeqF32Work = (int64_t)3 << 28;
+
 inline size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // Joins the side streams a layer call has forked into the main stream on every early return (an
@@ -219,6 +226,74 @@ struct SeqLayout {
     rl_ws = take(rl_ws_bytes);
     xws_b = take(xws_bytes);
     if (norm != MOC_NORM_NONE) dxc = take((size_t)max_u * 64 * d * 4);
+    scratch_bytes = o;
+    return MOC_OK;
+  }
+};
+
+// The float32 layer (moc_seq_layer_f32_*): the reference's small configurations, where a step is some
+// thirty launches of 2 to 20 us each and the host issuing them one autograd function at a time was what it
+// waited for (692 us of host time for 199 us of kernels at 2 x 128 tokens, d = 256; in one call each way
+// 295 us).  One stream: nothing here is long enough to be worth an event.
+struct SeqF32Layout {
+  int64_t B, L, d, C, E, max_u;
+  int NS, KV, Lp;
+  size_t q, attn, pooled, w, uniq, n_uniq, edge_u, csr_off, csr_edge, plan_ws, kv, lse, x, mean, rstd, xws_f;
+  size_t plan_ws_bytes, xws_bytes, saved_bytes;
+  size_t d_attn, delta, dq, dkv_edge, dom_part, dkv, dxc, dz, dpooled, rl_ws, xws_b;
+  size_t rl_ws_bytes, scratch_bytes;
+
+  int init(int64_t B_, int64_t L_, int64_t d_, int H, int HK, int64_t C_, int S, int k, int norm) {
+    B = B_, L = L_, d = d_, C = C_;
+    MOC_REQUIRE(norm == MOC_NORM_NONE || norm == MOC_NORM_RMS || norm == MOC_NORM_LAYERNORM, MOC_ERR_ARG,
+                "moc_seq_layer_f32: norm %d", norm);
+    MOC_REQUIRE(B > 0 && B <= 64 && L > 0 && H > 0 && HK > 0 && H % HK == 0 && d == (int64_t)H * 64 && d <= 4096 &&
+                    S > 0 && S <= 1024 && k > 0 && k <= 1024 && k <= C - S && C <= 8192,
+                MOC_ERR_UNSUPPORTED, "moc_seq_layer_f32: B=%lld, L=%lld, d=%lld, H=%d, HK=%d, C=%lld, S=%d, k=%d",
+                (long long)B, (long long)L, (long long)d, H, HK, (long long)C, S, k);
+    NS = S + k;
+    KV = HK * 64;
+    Lp = (int)((L + 127) / 128 * 128);
+    E = B * NS;
+    max_u = E < C ? E : C;
+    const int64_t tok = B * L, rows = max_u * 64;
+    MOC_REQUIRE(tok < (1 << 21) && tok * d * d + rows * KV * d <= kSeqF32Work, MOC_ERR_UNSUPPORTED,
+                "moc_seq_layer_f32: %lld tokens, %lld rows of d=%lld (larger products belong to a library GEMM)",
+                (long long)tok, (long long)rows, (long long)d);
+    size_t o = 0;
+    auto take = [&](size_t bytes) { const size_t at = o; o = al256(o + bytes); return at; };
+    q = take(tok * d * 4);
+    attn = take(tok * d * 4);
+    pooled = take(B * d * 4);
+    w = take(B * k * 4);
+    uniq = take(max_u * 4);
+    n_uniq = take(2 * 4);
+    edge_u = take(E * 4);
+    csr_off = take((max_u + 1) * 4);
+    csr_edge = take(E * 4);
+    plan_ws_bytes = moc_chapter_plan_workspace(E, C);
+    plan_ws = take(plan_ws_bytes);
+    kv = take((size_t)rows * 2 * KV * 4);
+    lse = take((size_t)B * H * Lp * 4);
+    x = take((size_t)rows * d * 4);
+    mean = take(norm ? (size_t)rows * 4 : 0);
+    rstd = take(norm ? (size_t)rows * 4 : 0);
+    xws_bytes = moc_xattn_split_workspace(MOC_F32, B, L, H, NS);
+    xws_f = take(xws_bytes);
+    saved_bytes = o;
+    o = 0;
+    d_attn = take(tok * d * 4);
+    delta = take((size_t)B * H * Lp * 4);
+    dq = take(tok * d * 4);
+    dkv_edge = take((size_t)E * 64 * 2 * KV * 4);
+    dom_part = take((size_t)E * HK * 4);
+    dkv = take((size_t)rows * 2 * KV * 4);
+    dxc = take((size_t)rows * d * 4);
+    dz = take((size_t)B * C * 4);
+    dpooled = take((size_t)B * d * 4);
+    rl_ws_bytes = moc_router_linear_bwd_workspace(B, d, C);
+    rl_ws = take(rl_ws_bytes);
+    xws_b = take(xws_bytes);
     scratch_bytes = o;
     return MOC_OK;
   }
@@ -525,6 +600,106 @@ int moc_seq_layer_bwd_ex(const void* h, const void* bank, const void* wr, int wr
   MOC_HIP(hipStreamWaitEvent(main, ev[5], 0));
   if (dwq) MOC_HIP(hipStreamWaitEvent(main, ev[7], 0));
   join.disarm();
+  return MOC_OK;
+}
+
+int moc_seq_layer_f32_sizes(int64_t B, int64_t L, int64_t d, int H, int HK, int64_t C, int S, int k, int norm,
+                            size_t* saved, size_t* scratch) {
+  MOC_REQUIRE(saved && scratch, MOC_ERR_ARG, "moc_seq_layer_f32_sizes: null pointer");
+  SeqF32Layout y;
+  SEQ_TRY(y.init(B, L, d, H, HK, C, S, k, norm));
+  *saved = y.saved_bytes;
+  *scratch = y.scratch_bytes;
+  return MOC_OK;
+}
+
+int moc_seq_layer_f32_fwd(const float* h, const float* bank, const void* wr, int wr_dtype, const float* br,
+                          const float* wq, const float* wk, const float* wv, const float* wo, const float* coef,
+                          int64_t B, int64_t L, int64_t d, int H, int HK, int64_t C, int S, int k, float routed_scale,
+                          int norm, float eps, float* out, float* logits, int32_t* idx, int32_t* idx_star, float* omega,
+                          void* saved, size_t saved_bytes, hipStream_t st) {
+  MOC_REQUIRE(h && bank && wr && wq && wk && wv && wo && out && logits && idx && idx_star && omega && saved,
+              MOC_ERR_ARG, "moc_seq_layer_f32_fwd: null pointer");
+  SeqF32Layout y;
+  SEQ_TRY(y.init(B, L, d, H, HK, C, S, k, norm));
+  MOC_REQUIRE(saved_bytes >= y.saved_bytes, MOC_ERR_ARG, "moc_seq_layer_f32_fwd: saved buffer %zu < %zu bytes",
+              saved_bytes, y.saved_bytes);
+  char* sv = (char*)saved;
+  float *q = (float*)(sv + y.q), *attn = (float*)(sv + y.attn), *kv = (float*)(sv + y.kv), *x = (float*)(sv + y.x);
+  float *mean = norm ? (float*)(sv + y.mean) : nullptr, *rstd = norm ? (float*)(sv + y.rstd) : nullptr;
+  int32_t *uniq = (int32_t*)(sv + y.uniq), *n_uniq = (int32_t*)(sv + y.n_uniq), *edge_u = (int32_t*)(sv + y.edge_u);
+  const int64_t tok = B * L, rows = y.max_u * 64, KV = y.KV, KV2 = 2 * KV;
+  SEQ_TRY(moc_router_pool1(h, MOC_F32, B, L, d, coef, (float*)(sv + y.pooled), st));
+  SEQ_TRY(moc_router_linear((const float*)(sv + y.pooled), B, d, wr, wr_dtype, br, C, logits, st));
+  SEQ_TRY(moc_router_topk_prepend(logits, B, C, S, k, routed_scale, idx, (float*)(sv + y.w), idx_star, omega, st));
+  SEQ_TRY(moc_chapter_plan(idx_star, y.E, C, sv + y.plan_ws, y.plan_ws_bytes, uniq, n_uniq, edge_u,
+                           (int32_t*)(sv + y.csr_off), (int32_t*)(sv + y.csr_edge), st));
+  if (norm) SEQ_TRY(moc_row_stats(bank, MOC_F32, d, 64, uniq, n_uniq, y.max_u, norm, eps, mean, rstd, st));
+  SEQ_TRY(moc_gather_rows(MOC_F32, bank, MOC_F32, d, 64, uniq, n_uniq, y.max_u, mean, rstd, x, st));
+  SEQ_TRY(gemm_f32(0, 1, rows, KV, d, x, d, wk, d, kv, KV2, 0, st));
+  SEQ_TRY(gemm_f32(0, 1, rows, KV, d, x, d, wv, d, kv + KV, KV2, 0, st));
+  SEQ_TRY(gemm_f32(0, 1, tok, d, d, h, d, wq, d, q, d, 0, st));
+  SEQ_TRY(moc_xattn_fwd_split(MOC_F32, q, kv, kv + KV, rows * KV2 - KV, 64 * KV2, 64, (int)KV2, edge_u, omega, B, L, H, HK,
+                              64, 64, y.NS, 0.125f, attn, (float*)(sv + y.lse), y.xws_bytes ? sv + y.xws_f : nullptr,
+                              y.xws_bytes, st));
+  return gemm_f32(0, 1, tok, d, d, attn, d, wo, d, out, d, 0, st);
+}
+
+int moc_seq_layer_f32_bwd(const float* h, const float* bank, const void* wr, int wr_dtype, const float* wq,
+                          const float* wk, const float* wv, const float* wo, const float* coef, int64_t B, int64_t L,
+                          int64_t d, int H, int HK, int64_t C, int S, int k, float routed_scale, int norm,
+                          const float* logits, const int32_t* idx, const float* omega, const void* saved,
+                          size_t saved_bytes, const float* dout, const float* dlogits, float* dh, float* dbank,
+                          int64_t bank_rows, float* dwr, float* dbr, float* dwq, float* dwkv, float* dwo, void* scratch,
+                          size_t scratch_bytes, hipStream_t st) {
+  MOC_REQUIRE(h && bank && wr && wq && wk && wv && wo && logits && idx && omega && saved && dout && scratch, MOC_ERR_ARG,
+              "moc_seq_layer_f32_bwd: null pointer");
+  SeqF32Layout y;
+  SEQ_TRY(y.init(B, L, d, H, HK, C, S, k, norm));
+  MOC_REQUIRE(saved_bytes >= y.saved_bytes && scratch_bytes >= y.scratch_bytes, MOC_ERR_ARG,
+              "moc_seq_layer_f32_bwd: saved %zu < %zu or scratch %zu < %zu bytes", saved_bytes, y.saved_bytes,
+              scratch_bytes, y.scratch_bytes);
+  const char* sv = (const char*)saved;
+  char* sc = (char*)scratch;
+  const float *q = (const float*)(sv + y.q), *attn = (const float*)(sv + y.attn), *kv = (const float*)(sv + y.kv);
+  const float *x = (const float*)(sv + y.x), *lse = (const float*)(sv + y.lse);
+  const float *mean = norm ? (const float*)(sv + y.mean) : nullptr, *rstd = norm ? (const float*)(sv + y.rstd) : nullptr;
+  const int32_t *uniq = (const int32_t*)(sv + y.uniq), *n_uniq = (const int32_t*)(sv + y.n_uniq);
+  const int32_t *edge_u = (const int32_t*)(sv + y.edge_u), *csr_off = (const int32_t*)(sv + y.csr_off);
+  const int32_t* csr_edge = (const int32_t*)(sv + y.csr_edge);
+  float *d_attn = (float*)(sc + y.d_attn), *delta = (float*)(sc + y.delta), *dq = (float*)(sc + y.dq);
+  float *dkv_edge = (float*)(sc + y.dkv_edge), *dom = (float*)(sc + y.dom_part), *dkv = (float*)(sc + y.dkv);
+  const int64_t tok = B * L, rows = y.max_u * 64, KV = y.KV, KV2 = 2 * KV, span = rows * KV2 - KV;
+  const bool router_grads = dh || dwr || dbr;
+  if (dwo) SEQ_TRY(gemm_f32(1, 0, d, d, tok, dout, d, attn, d, dwo, d, 0, st));
+  if (router_grads || dwq || dwkv || dbank) {
+    SEQ_TRY(gemm_f32(0, 0, tok, d, d, dout, d, wo, d, d_attn, d, 0, st));
+    SEQ_TRY(moc_xattn_bwd_dq_delta_split(MOC_F32, q, kv, kv + KV, span, 64 * KV2, 64, (int)KV2, edge_u, omega, attn,
+                                         d_attn, lse, delta, B, L, H, HK, 64, 64, y.NS, 0.125f, dq,
+                                         y.xws_bytes ? sc + y.xws_b : nullptr, y.xws_bytes, st));
+    SEQ_TRY(moc_xattn_bwd_dkv(MOC_F32, q, d_attn, kv, kv + KV, span, 64 * KV2, 64, (int)KV2, edge_u, omega, lse, delta, B,
+                              L, H, HK, 64, 64, y.NS, 0.125f, dkv_edge, dom, st));
+  }
+  if (dh) SEQ_TRY(gemm_f32(0, 0, tok, d, d, dq, d, wq, d, dh, d, 0, st));
+  if (dwq) SEQ_TRY(gemm_f32(1, 0, d, d, tok, dq, d, h, d, dwq, d, 0, st));
+  if (router_grads) {
+    float *dz = (float*)(sc + y.dz), *dpooled = dh ? (float*)(sc + y.dpooled) : nullptr;
+    SEQ_TRY(moc_router_seq_bwd(logits, idx, (const float*)(sv + y.w), dom, HK, B, C, S, k, routed_scale, dlogits, dz, st));
+    SEQ_TRY(moc_router_linear_bwd(dz, (const float*)(sv + y.pooled), B, d, wr, wr_dtype, C, dpooled, dwr, dbr,
+                                  sc + y.rl_ws, y.rl_ws_bytes, st));
+    if (dh) SEQ_TRY(moc_rows_add_bcast(dh, MOC_F32, B, L, d, dpooled, coef, 1.f / (float)L, st));
+  }
+  if (dwkv || dbank)
+    SEQ_TRY(moc_dkv_reduce(MOC_F32, dkv_edge, n_uniq, csr_off, csr_edge, y.max_u, KV2, dkv, st));
+  if (dwkv) SEQ_TRY(gemm_f32(1, 0, KV2, d, rows, dkv, KV2, x, d, dwkv, d, 0, st));
+  if (dbank) {
+    float* dxc = (float*)(sc + y.dxc);
+    SEQ_TRY(gemm_f32(0, 0, rows, d, KV, dkv, KV2, wk, d, dxc, d, 0, st));
+    SEQ_TRY(gemm_f32(0, 0, rows, d, KV, dkv + KV, KV2, wv, d, dxc, d, 1, st));
+    SEQ_TRY(moc_fill_zero(dbank, bank_rows * d * 4, 2048, st));
+    SEQ_TRY(moc_bank_scatter(MOC_F32, dxc, bank, MOC_F32, d, 64, uniq, n_uniq, y.max_u, nullptr, nullptr, mean, rstd, norm,
+                             dbank, st));
+  }
   return MOC_OK;
 }
 

@@ -134,6 +134,13 @@ def split_rows(x: torch.Tensor, n: int):
     return _SplitRows.apply(x, n)
 
 
+def _has_hooks(m: nn.Module) -> bool:
+    """Whether calling `m` would run anything beside its class's own forward."""
+    return bool(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+                or "forward" in m.__dict__ or type(m) is not MemoryCrossAttention
+                or torch.nn.modules.module._has_any_global_hook())
+
+
 class RoutedMemoryLayer(nn.Module):
     """One sequence-routed memory sublayer (router + memory cross-attention).
 
@@ -190,19 +197,29 @@ class RoutedMemoryLayer(nn.Module):
         if attn.gradient_checkpointing and self.training:
             return None
         k = min(int(self.router.top_k), C - S)
-        if not seq_layer.supported(hidden_states, bank, attn.q_proj.weight, attn.o_proj.weight,
-                                   self.router.router.weight, S, k, C, self.tokens_per_chapter):
+        normalize = self.normalize and 0 < S < S + k
+        norm_type = self.norm_type if normalize else None
+        router = self.router.router
+        if hidden_states.dtype == torch.float32:
+            # hooks on the attention module run where it is called
+            if _has_hooks(attn) or not seq_layer.supported_f32(
+                    hidden_states, bank, router.weight, router.bias, attn.q_proj.weight, attn.k_proj.weight,
+                    attn.v_proj.weight, attn.o_proj.weight, num_chapters=C, tokens_per_chapter=self.tokens_per_chapter,
+                    num_shared=S, top_k=k, num_heads=attn.num_heads, num_kv_heads=attn.num_kv_heads,
+                    norm_type=norm_type):
+                return None
+        elif not seq_layer.supported(hidden_states, bank, attn.q_proj.weight, attn.o_proj.weight, router.weight, S, k, C,
+                                     self.tokens_per_chapter):
             return None
         coef = None
         if strategy in ("sequence-rolling", "sequence_rolling"):
             coef = rolling_coefficients(hidden_states.shape[1], self.routing_window_size, hidden_states.device)
-        normalize = self.normalize and 0 < S < S + k
         return seq_layer.seq_routed_layer(
-            hidden_states, bank, self.router.router.weight, self.router.router.bias, attn.q_proj.weight,
+            hidden_states, bank, router.weight, router.bias, attn.q_proj.weight,
             attn.k_proj.weight, attn.v_proj.weight, attn.o_proj.weight, num_chapters=C,
             tokens_per_chapter=self.tokens_per_chapter, num_shared=S, top_k=k,
             routed_scale=self.routed_scaling_factor, num_heads=attn.num_heads, num_kv_heads=attn.num_kv_heads,
-            norm_type=self.norm_type if normalize else None, eps=self.norm_eps, coef=coef)
+            norm_type=norm_type, eps=self.norm_eps, coef=coef)
 
     @float16_via_float32
     def forward(self, hidden_states: torch.Tensor, bank: torch.Tensor,

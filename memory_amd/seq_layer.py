@@ -29,6 +29,10 @@ forward), so a training step costs two host calls; PyTorch only allocates the ou
 buffer and one scratch buffer.  A forward that no backward follows (grad mode off, or no input that
 requires a gradient) leaves out what only the backward reads, and its buffer is a temporary.
 ``NATIVE = False`` keeps the Python-scheduled sequence.
+
+The float32 layer at the reference's small sizes runs as one host call each way on one stream
+(moc_seq_layer_f32_fwd / _bwd): its launches take a few microseconds each and the step is what the
+host needs to issue them.
 """
 
 from __future__ import annotations
@@ -252,6 +256,89 @@ class _SeqRoutedLayer(torch.autograd.Function):
         return dh, dbank, dwr, dbr, dwq, dwk, dwv, dwo, None, None
 
 
+@functools.lru_cache(maxsize=256)
+def _f32_sizes(B, Lq, d, H, HK, C, S, k, norm):
+    """(saved, scratch) buffer bytes of the native float32 layer, or None for shapes outside it."""
+    n = (ctypes.c_size_t * 2)()
+    at = [ctypes.addressof(n) + i * ctypes.sizeof(ctypes.c_size_t) for i in range(2)]
+    return tuple(n) if L.query("moc_seq_layer_f32_sizes", B, Lq, d, H, HK, C, S, k, norm, *at) == L.MOC_OK else None
+
+
+def supported_f32(h, bank, wr, br, wq, wk, wv, wo, *, num_chapters: int, tokens_per_chapter: int, num_shared: int,
+                  top_k: int, num_heads: int, num_kv_heads: int, norm_type: Optional[str] = None) -> bool:
+    """Whether moc_seq_layer_f32_fwd / _bwd take this call; every other float32 call keeps the per-op
+    autograd functions.  Under autocast those cast, so such calls stay with them too."""
+    f32 = torch.float32
+    if not (h.dtype == f32 and h.is_cuda and h.dim() == 3 and h.shape[1] > 0 and tokens_per_chapter == 64
+            and num_shared > 0 and top_k > 0 and not torch.is_autocast_enabled()):
+        return False
+    d = h.shape[2]
+    KV = num_kv_heads * 64
+    if (bank.dim() != 2 or bank.shape[0] < num_chapters * 64 or bank.shape[1] != d or wr.dtype not in (f32, torch.bfloat16)
+            or wr.shape != (num_chapters, d) or wq.shape != (d, d) or wo.shape != (d, d) or wk.shape != (KV, d)
+            or wv.shape != (KV, d) or getattr(bank, "_moc_bank_opt", None) is not None
+            or getattr(bank, "_moc_row_grad", None) is not None):
+        return False
+    for t in (h, bank, wq, wk, wv, wo, wr, br):     # the kernels read 16-byte pieces of packed rows
+        if t is not None and (t.device != h.device or not t.is_contiguous() or t.data_ptr() % 16
+                              or (t is not wr and t.dtype != f32)):
+            return False
+    return _f32_sizes(h.shape[0], h.shape[1], d, num_heads, num_kv_heads, num_chapters, num_shared, top_k,
+                      ops.norm_code(norm_type)) is not None
+
+
+class _SeqF32Layer(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, h, bank, wr, br, wq, wk, wv, wo, coef, cfg):
+        C, T, S, k, scale, H, HK, norm, eps, train = cfg
+        dev = h.device
+        B, Lq, d = h.shape
+        nsaved, ctx.nscratch = _f32_sizes(B, Lq, d, H, HK, C, S, k, norm)
+        cf = None if coef is None else coef.to(device=dev, dtype=torch.float32).contiguous()
+        saved = torch.empty(nsaved, device=dev, dtype=torch.uint8)
+        out = torch.empty(B, Lq, d, device=dev, dtype=torch.float32)
+        logits = torch.empty(B, C, device=dev, dtype=torch.float32)
+        idx = torch.empty(B, k, device=dev, dtype=torch.int32)
+        idx_star = torch.empty(B, S + k, device=dev, dtype=torch.int32)
+        omega = torch.empty(B, S + k, device=dev, dtype=torch.float32)
+        call("moc_seq_layer_f32_fwd", ptr(h), ptr(bank), ptr(wr), L.dtype_code(wr.dtype), ptr(br), ptr(wq), ptr(wk),
+             ptr(wv), ptr(wo), ptr(cf), B, Lq, d, H, HK, C, S, k, scale, norm, eps, ptr(out), ptr(logits), ptr(idx),
+             ptr(idx_star), ptr(omega), ptr(saved), nsaved, stream_ptr(dev))
+        ctx.cfg = cfg
+        ctx.set_materialize_grads(False)
+        if train:
+            ctx.save_for_backward(h, bank, wr, wq, wk, wv, wo, cf, logits, idx, omega, saved)
+        ctx.mark_non_differentiable(idx, idx_star, omega)
+        return out, logits, idx, idx_star, omega
+
+    @staticmethod
+    def backward(ctx, dout, dlogits, _didx, _didx_star, _domega):
+        h, bank, wr, wq, wk, wv, wo, cf, logits, idx, omega, saved = ctx.saved_tensors
+        C, T, S, k, scale, H, HK, norm, eps, _train = ctx.cfg
+        need_h, need_bank, need_wr, need_br, need_wq, need_wk, need_wv, need_wo = ctx.needs_input_grad[:8]
+        dev = h.device
+        B, Lq, d = h.shape
+        KV = HK * 64
+
+        def new(need, *shape):
+            return torch.empty(shape, device=dev, dtype=torch.float32) if need else None
+
+        dout = torch.zeros(B, Lq, d, device=dev) if dout is None else dout.contiguous()
+        if dout.data_ptr() % 16:
+            dout = dout.clone()
+        dz = None if dlogits is None else dlogits.float().contiguous()
+        dh, dbank, dwr, dbr = new(need_h, B, Lq, d), new(need_bank, *bank.shape), new(need_wr, C, d), new(need_br, C)
+        dwq, dwkv, dwo = new(need_wq, d, d), new(need_wk or need_wv, 2 * KV, d), new(need_wo, d, d)
+        scratch = torch.empty(ctx.nscratch, device=dev, dtype=torch.uint8)
+        call("moc_seq_layer_f32_bwd", ptr(h), ptr(bank), ptr(wr), L.dtype_code(wr.dtype), ptr(wq), ptr(wk), ptr(wv),
+             ptr(wo), ptr(cf), B, Lq, d, H, HK, C, S, k, scale, norm, ptr(logits), ptr(idx), ptr(omega), ptr(saved),
+             saved.numel(), ptr(dout), ptr(dz), ptr(dh), ptr(dbank), bank.shape[0], ptr(dwr), ptr(dbr), ptr(dwq),
+             ptr(dwkv), ptr(dwo), ptr(scratch), ctx.nscratch, stream_ptr(dev))
+        dwk = dwkv[:KV] if need_wk else None
+        dwv = dwkv[KV:] if need_wv else None
+        return (dh, dbank, dwr if dwr is None else dwr.to(wr.dtype), dbr, dwq, dwk, dwv, dwo, None, None)
+
+
 def _native_backward(ctx, dout, dlogits):
     """The whole backward in one host call (moc_seq_layer_bwd_ex)."""
     h, bank, wrc, cf, logits, idx, omega, saved = ctx.saved_tensors
@@ -298,4 +385,5 @@ def seq_routed_layer(h, bank, wr, br, wq, wk, wv, wo, *, num_chapters: int, toke
                                             for t in (h, bank, wr, br, wq, wk, wv, wo))
     cfg = (int(num_chapters), int(tokens_per_chapter), int(num_shared), int(top_k), float(routed_scale),
            int(num_heads), int(num_kv_heads), ops.norm_code(norm_type), float(eps), train)
-    return _SeqRoutedLayer.apply(h, bank, wr, br, wq, wk, wv, wo, coef, cfg)
+    layer = _SeqF32Layer if h.dtype == torch.float32 else _SeqRoutedLayer
+    return layer.apply(h, bank, wr, br, wq, wk, wv, wo, coef, cfg)

@@ -1,0 +1,134 @@
+"""The float32 sequence layer in one host call each way (moc_seq_layer_f32_*) against the per-op
+autograd functions, over the forms it accepts, and the calls that stay with those functions."""
+
+import pytest
+import torch
+
+from helpers import gen
+
+pytestmark = pytest.mark.gpu
+
+
+def _layer(dev, d, H, HK, C, S, k, norm, strategy="sequence", wr_dtype=torch.float32):
+    from memory_amd.model import RoutedMemoryLayer
+    layer = RoutedMemoryLayer(d, H, C, 64, k, num_shared_chapters=S, num_kv_heads=HK, wo_init_zero=False,
+                              normalize_shared_routed_before_mixing=norm != "none",
+                              shared_routed_norm_type="rms" if norm == "none" else norm, routing_strategy=strategy,
+                              routing_window_size=7)
+    g = gen(d + C + k)
+    with torch.no_grad():
+        for p in layer.parameters():
+            p.copy_(torch.randn(p.shape, generator=g) * 0.05)
+    layer = layer.to(dev)
+    layer.router.to(wr_dtype) if wr_dtype != torch.float32 else None
+    return layer
+
+
+def _step(layer, h, bank, up, fused, frozen=(), losses=True):
+    layer.fused = fused
+    for p in layer.parameters():
+        p.grad = None
+    h = h.detach().clone().requires_grad_("h" not in frozen)
+    bank = bank.detach().clone().requires_grad_("bank" not in frozen)
+    out, ls = layer(h, bank, return_losses=losses)
+    loss = (out * up).sum() + sum(v for v in ls.values())
+    loss.backward()
+    grads = {n: p.grad for n, p in layer.named_parameters()}
+    grads.update(h=h.grad, bank=bank.grad)
+    return out.detach(), {n: v.detach() for n, v in ls.items()}, grads
+
+
+def _same(a, b, name):
+    assert (a is None) == (b is None), name
+    if a is None:
+        return
+    # the two paths differ in the products' summation order only: a few roundings of 2^-24 per
+    # product of up to ~1,000 terms, carried through the chain's four products
+    err = ((a.double() - b.double()).norm() / b.double().norm().clamp_min(1e-12)).item()
+    assert err < 2e-5, (name, err)
+
+
+CASES = [
+    # B, L, d, H, HK, C, S, k, norm, strategy
+    (1, 1, 64, 1, 1, 3, 1, 2, "none", "sequence"),
+    (2, 128, 256, 4, 4, 33, 1, 4, "none", "sequence"),
+    (3, 251, 256, 4, 2, 257, 1, 16, "rms", "sequence"),
+    (2, 33, 128, 2, 1, 9, 3, 6, "layernorm", "sequence-rolling"),
+    (1, 130, 320, 5, 5, 40, 2, 1, "rms", "sequence"),
+]
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_f32_layer_equals_per_op(gpu_device, case, monkeypatch):
+    from memory_amd import _lib as lib
+    from memory_amd import seq_layer
+    B, L, d, H, HK, C, S, k, norm, strategy = case
+    dev = gpu_device
+    layer = _layer(dev, d, H, HK, C, S, k, norm, strategy)
+    g = gen(B * L)
+    h, up = torch.randn(B, L, d, generator=g).to(dev), torch.randn(B, L, d, generator=g).to(dev)
+    bank = (torch.randn(C * 64, d, generator=g) * 0.1).to(dev)
+    called = []
+    real = seq_layer.call
+    monkeypatch.setattr(seq_layer, "call", lambda name, *a: (called.append(name), real(name, *a))[1])
+    for frozen in ((), ("h",), ("bank",)):
+        got = _step(layer, h, bank, up, True, frozen)
+        assert called == ["moc_seq_layer_f32_fwd", "moc_seq_layer_f32_bwd"]
+        called.clear()
+        want = _step(layer, h, bank, up, False, frozen)
+        assert not called
+        _same(got[0], want[0], "out")
+        for n in want[1]:
+            _same(got[1][n], want[1][n], n)
+        for n in want[2]:
+            _same(got[2][n], want[2][n], n)
+    layer.fused = True
+    with torch.no_grad():
+        assert torch.equal(layer(h, bank, return_losses=False)[0], got[0])
+    for p in (layer.memory_attn.k_proj.weight, layer.memory_attn.o_proj.weight, layer.router.router.bias):
+        p.requires_grad_(False)
+    got, want = _step(layer, h, bank, up, True, losses=False), _step(layer, h, bank, up, False, losses=False)
+    for n in want[2]:
+        _same(got[2][n], want[2][n], n)
+
+
+def test_f32_layer_stays_per_op(gpu_device, monkeypatch):
+    """Unpacked or unaligned inputs, other sizes and types, hooks and autocast keep the per-op functions."""
+    from memory_amd import seq_layer
+    dev = gpu_device
+    layer = _layer(dev, 128, 2, 2, 9, 1, 3, "none")
+    g = gen(5)
+    h, bank = torch.randn(2, 40, 128, generator=g).to(dev), (torch.randn(9 * 64, 128, generator=g) * 0.1).to(dev)
+    up = torch.randn(2, 40, 128, generator=g).to(dev)
+    called = []
+    real = seq_layer.call
+    monkeypatch.setattr(seq_layer, "call", lambda name, *a: (called.append(name), real(name, *a))[1])
+    want = layer(h, bank)[0]
+    assert called.pop() == "moc_seq_layer_f32_fwd"
+    flat = torch.empty(h.numel() + 1, device=dev)
+    flat[1:] = h.reshape(-1)
+    for x in (flat[1:].view(h.shape), h.transpose(0, 1).contiguous().transpose(0, 1)):
+        _same(layer(x, bank)[0], want, "layout")
+    hits = []
+    handle = layer.memory_attn.register_forward_hook(lambda *a: hits.append(1))
+    _same(layer(h, bank)[0], want, "hook")
+    handle.remove()
+    assert hits == [1]
+    with torch.autocast("cuda", torch.bfloat16):
+        layer(h, bank)
+    assert not called
+    # an unaligned or absent upstream gradient reaches the same backward
+    x = h.clone().requires_grad_()
+    out, losses = layer(x, bank)
+    flat[1:] = up.reshape(-1)
+    out.backward(flat[1:].view(h.shape))
+    y = h.clone().requires_grad_()
+    layer.fused = False
+    layer(y, bank)[0].backward(up)
+    _same(x.grad, y.grad, "unaligned upstream")
+    layer.fused = True
+    x.grad = y.grad = None
+    sum(layer(x, bank)[1].values()).backward()
+    layer.fused = False
+    sum(layer(y, bank)[1].values()).backward()
+    _same(x.grad, y.grad, "losses alone")
