@@ -6,8 +6,8 @@ Entry points with the reference's signatures:
   * FSA_topk_sparse_attention_weighted_joint_bias_bthd
                                               (kernels-final/kernel_v5.py:819; v5, same signature)
 and ``token_routed_attention`` for MemoryCrossAttention's token path
-(memory_attention.py:480-716), which projects the routed bank once per call
-instead of once per batch element.
+(memory_attention.py:480-716), which projects the routed bank (few tokens: its selected chapters)
+once per call instead of once per batch element.
 
 Combine modes (see csrc/sparse_xattn.hip): 0 = exact per-chapter MoE
 (sum_s w_s softmax_s V_s); 1 = joint softmax over all selected keys;
@@ -22,6 +22,7 @@ end on a 64-key boundary.
 
 from __future__ import annotations
 
+import dataclasses
 from typing import List, Optional
 
 import torch
@@ -32,6 +33,14 @@ from ._lib import call, ptr, stream_ptr
 from . import ops
 
 BLOCK = 64
+
+# The token path projects only the chapters its tokens select while they make fewer than this many
+# selections per chapter of the bank: evenly spread selections then leave e^-4 = 2% of it out, and the
+# gathered projection and its gradients cost what the whole bank's do (4,096 chapters of 64 x 768 rows,
+# forward / training step, whole bank -> selected: 668 -> 309 / 2,017 -> 1,187 us at 0.16 selections per
+# chapter, 804 -> 638 / 2,325 -> 1,904 at 1.2, 830 -> 758 / 2,422 -> 2,235 at 2, 861 -> 857 / 2,553 -> 2,541
+# at 4, 892 -> 885 / 2,656 -> 2,666 at 8).  Selections that crowd on fewer chapters gain more.
+SELECT_FACTOR = 4
 
 
 class _Segment:
@@ -484,7 +493,8 @@ def FSA_topk_sparse_attention_weighted_joint_bias_bthd(q_bthd, k_bthd, v_bthd, b
 
 class _TokenRouted(torch.autograd.Function):
     """Routed branch of the token-level memory layer: K/V of the routed bank are
-    projected once (one GEMM over every routed chapter), then sparse attention.
+    projected once (one GEMM over every routed chapter, or over the selected ones when the
+    tokens are few), then sparse attention.
 
     q (B, L, H, 64); routed (N_r, d); wk/wv (HK*64, d); idx (B, L, k) local chapter
     ids; w (B, L, k) or None.  Returns (B, L, H, 64)."""
@@ -506,18 +516,28 @@ class _TokenRouted(torch.autograd.Function):
             wkv, wkv_t = ops.weight_pack(wk, wv, transposed=True)
         else:
             wkv = torch.cat([wk, wv], 0).to(dtype).contiguous()
-        # every routed chapter is projected (no gather, no norm): one rows GEMM over the routed
-        # bank (the chapter GEMM's wide tiles for bf16), K and V read by the sparse kernels as
-        # strided column blocks of kv [Nr][2 KV]
+        # K and V are read by the sparse kernels as strided column blocks of kv [rows][2 KV]
         KV = HK * D
-        rows = routed.to(dtype)
-        if ops.rows_gemm_ok(rows, wkv):
-            kv = ops.rows_linear(rows, wkv)
-        else:
-            with L.region("lib_token_kv_project"):
-                kv = F.linear(rows, wkv)
         S = idx.shape[-1]
         segs = _segments(idx, w, mode, C, False, HQ, HK, C)
+        ctx.sel = None
+        if _selected_only(routed, wkv, idx, C):
+            # only the plan's distinct chapters: block u of kv is chapter uniq[u], so the sparse
+            # kernels read it under the ids 0, 1, ...
+            plan = segs[0].plan
+            kv = ops.chapter_project(routed, plan, wkv, gather=True)
+            ar = torch.arange(plan.max_u + 1, device=q.device, dtype=torch.int32)
+            segs[0].plan = dataclasses.replace(plan, uniq=ar[:plan.max_u])
+            ctx.sel = (plan.uniq, ar)
+        else:
+            # every routed chapter (no gather, no norm): one rows GEMM over the routed bank (the
+            # chapter GEMM's wide tiles for bf16)
+            rows = routed.to(dtype)
+            if ops.rows_gemm_ok(rows, wkv):
+                kv = ops.rows_linear(rows, wkv)
+            else:
+                with L.region("lib_token_kv_project"):
+                    kv = F.linear(rows, wkv)
         out, saved = _forward(q, kv[:, :KV], kv[:, KV:], "rows", segs, mode, S, D ** -0.5)
         ctx.segs, ctx.saved_parts = segs, saved
         ctx.save_for_backward(q, routed, wkv, wkv_t, kv, out)
@@ -532,29 +552,68 @@ class _TokenRouted(torch.autograd.Function):
         D = q.shape[-1]
         KV = HK * D
         Nr, d = routed.shape
-        # dk / dv written as rows [chapter*64 + key][hk*64 + dim] (dv at column offset KV); blocks
+        # dk / dv written as rows [block*64 + key][hk*64 + dim] (dv at column offset KV); blocks
         # of chapters no token selected are zeroed by the backward instead of a 2 KV x Nr fill
-        dkv = torch.empty(Nr, 2 * KV, device=q.device, dtype=dtype)
+        # (with the selected chapters alone there are none that anything reads)
+        dkv = torch.empty(kv.shape[0], 2 * KV, device=q.device, dtype=dtype)
         elem = dkv.element_size()
         dq, dws = _backward(q, kv[:, :KV], kv[:, KV:], "rows", out, dout, ctx.segs, ctx.saved_parts, mode, S,
-                            D ** -0.5, dkv, None, (64 * 2 * KV, 64, 2 * KV, KV * elem), zero_chapters=Nr // BLOCK)
+                            D ** -0.5, dkv, None, (64 * 2 * KV, 64, 2 * KV, KV * elem),
+                            zero_chapters=Nr // BLOCK if ctx.sel is None else 0)
         need_r, need_wk, need_wv = ctx.needs_input_grad[1:4]
         dr = dwk = dwv = None
         if need_wk or need_wv:
-            dwkv = ops.linear_wgrad(dkv, routed, torch.float32 if torch.float32 in (wk_dtype, wv_dtype) else dtype)
+            out_dt = torch.float32 if torch.float32 in (wk_dtype, wv_dtype) else dtype
+            if ctx.sel is None:
+                dwkv = ops.linear_wgrad(dkv, routed, out_dt)
+            else:
+                dwkv = _selected_wgrad(dkv, routed, ctx.segs[0].plan, *ctx.sel, out_dt)
             dwk = dwkv[:KV].to(wk_dtype) if need_wk else None
             dwv = dwkv[KV:].to(wv_dtype) if need_wv else None
         if need_r:
-            dr = _rows_grad(routed, dkv, wkv, wkv_t)
+            dr = _rows_grad(routed, dkv, wkv, wkv_t, None if ctx.sel is None else (ctx.segs[0].plan, *ctx.sel))
         dw = None
         if w_shape is not None and dws:
             dw = dws[0].view(w_shape) if len(dws) == 1 else torch.stack(dws, 0).sum(0).view(w_shape)
         return dq, dr, dwk, dwv, dw, None, None, None
 
 
-def _rows_grad(routed: torch.Tensor, dkv: torch.Tensor, wkv: torch.Tensor,
-               wkv_t: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """d routed = dkv [Wk; Wv] (bf16: the chapter GEMM's rows mode with W = [Wk; Wv]^T).  When
+def _selected_only(routed: torch.Tensor, wkv: torch.Tensor, idx: torch.Tensor, C: int) -> bool:
+    """Whether the routed branch projects only the chapters its tokens select: bf16 operands that the
+    chapter GEMMs tile (forward, weight gradient and input gradient), one plan for all heads, and
+    fewer selections than SELECT_FACTOR times the bank's chapters."""
+    N, d = wkv.shape
+    return (idx.dim() == 3 and 0 < idx.numel() < SELECT_FACTOR * C and routed.is_cuda
+            and routed.dtype == torch.bfloat16 and wkv.dtype == torch.bfloat16 and N % 256 == 0 and d % 256 == 0
+            and routed.data_ptr() % 16 == 0)
+
+
+def _selected_wgrad(dkv, routed, plan, uniq, ar, out_dtype):
+    """d[Wk; Wv] of the selected chapters: block u of dkv against the bank rows of chapter uniq[u] (every
+    block its chapter's only edge)."""
+    N, K = dkv.shape[1], routed.shape[1]
+    ws_bytes = L.query("moc_chapter_wgrad_workspace", N, K, plan.max_u)
+    ws = torch.empty(ws_bytes // 4, device=dkv.device, dtype=torch.float32)
+    dw = torch.empty(N, K, device=dkv.device, dtype=out_dtype)
+    call("moc_chapter_wgrad", ptr(dkv), N, ptr(dkv), ptr(routed), K, 1, ptr(uniq), ptr(plan.n_uniq), plan.max_u,
+         ptr(ar), ptr(ar), N, K, ptr(ws), ws_bytes, L.dtype_code(out_dtype), ptr(dw), stream_ptr(dkv.device))
+    return dw
+
+
+def _selected_dx(dkv, plan, uniq, ar, wkv_t, out):
+    """out[chapter uniq[u]] = dkv[u] [Wk; Wv], zeros in the rows of every other chapter."""
+    C, d = out.shape[0] // BLOCK, out.shape[1]
+    mark = torch.empty(C, device=out.device, dtype=torch.int32)
+    # a chapter's 64 x d block as two halves of d / 128 column blocks (the two pointers)
+    call("moc_sparse_zero_untouched", L.MOC_BF16, ptr(out), ptr(out) + d, BLOCK * d, 64, d, C, 0, d // 128, ptr(uniq),
+         ptr(plan.n_uniq), plan.max_u, ptr(mark), stream_ptr(out.device))
+    return ops.chapter_dx(dkv, dkv, uniq, plan.n_uniq, plan.max_u, ar, ar, wkv_t, out, bank_rows=True)
+
+
+def _rows_grad(routed: torch.Tensor, dkv: torch.Tensor, wkv: torch.Tensor, wkv_t: Optional[torch.Tensor] = None,
+               sel=None) -> torch.Tensor:
+    """d routed = dkv [Wk; Wv] (bf16: the chapter GEMM's rows mode with W = [Wk; Wv]^T; ``sel`` =
+    (plan, uniq, iota): dkv holds the selected chapters' rows only).  When
     `routed` is the tail rows of a larger tensor (the routed part of a bank whose first rows are
     the shared chapters, split off by model.split_rows), the product is written into the tail of
     a buffer of the whole bank's shape, so the split's backward can hand that buffer on after
@@ -564,6 +623,8 @@ def _rows_grad(routed: torch.Tensor, dkv: torch.Tensor, wkv: torch.Tensor,
     native = ops.rows_gemm_ok(dkv, wkv_t)
 
     def product(out=None):
+        if sel is not None:
+            return _selected_dx(dkv, *sel, wkv_t, torch.empty_like(routed) if out is None else out)
         if native:
             return ops.rows_linear(dkv, wkv_t, out=out)
         with L.region("lib_token_kv_dx"):
