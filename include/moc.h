@@ -706,6 +706,28 @@ int moc_plan_row_table(const int32_t* n_uniq, const int32_t* csr_off, const int3
                        int width, int32_t* row_tab, hipStream_t stream);
 int moc_decode_row_table(const int32_t* n_uniq, const int32_t* csr_off, const int32_t* csr_edge, int64_t max_u,
                          int32_t* row_tab, hipStream_t stream);
+/* A rolling window of hidden states moved on and pooled: out [B][L][d] = the last L rows of old [B][n_old][d]
+ * (batch stride old_bs elements) followed by fresh [B][n_new][d] (fresh_bs); pooled f32 [B][d] = their mean,
+ * summed as moc_router_pool sums them.  d and the strides multiples of 8, pointers 16-byte aligned; workspace
+ * of moc_router_pool_workspace(B, L, d) bytes; out must not overlap old or fresh. */
+int moc_window_pool(const void* old, int64_t old_bs, int64_t n_old, const void* fresh, int64_t fresh_bs, int64_t n_new,
+                    int dtype, int64_t B, int64_t L, int64_t d, void* out, float* pooled, void* workspace,
+                    size_t workspace_bytes, hipStream_t stream);
+/* Routing of one decode step in one host call: moc_router_linear, moc_router_topk_prepend, moc_chapter_plan over
+ * the B * (S + k) selections and moc_decode_row_table, with those functions' arguments. */
+int moc_decode_route(const float* pooled, int64_t B, int64_t d, const void* W, int w_dtype, const float* bias, int64_t C,
+                     int S, int k, float scale, float* logits, int32_t* idx, float* w, int32_t* idx_star, float* omega,
+                     void* plan_ws, size_t plan_ws_bytes, int32_t* uniq, int32_t* n_uniq, int32_t* edge_u,
+                     int32_t* csr_off, int32_t* csr_edge, int64_t max_u, int32_t* row_tab, hipStream_t stream);
+/* One decode step of a bf16 memory layer in one host call: q = x wq^T (moc_linear_rows), moc_decode_partial,
+ * moc_sparse_combine (joint) and out [B][N] = a wo^T, with those functions' limits (B <= 256).  workspace:
+ * moc_decode_step_workspace bytes, 16-byte aligned. */
+size_t moc_decode_step_workspace(int64_t B, int H, int NS);
+int moc_decode_step(const void* x, int64_t B, int64_t d, const void* wq, int H, const void* k_tiles, const void* v_tiles,
+                    int HK, int T, const int32_t* uniq, const int32_t* n_uniq, const int32_t* csr_off,
+                    const int32_t* csr_edge, const int32_t* edge_u, int64_t max_u, const float* omega, int NS,
+                    float scale, const void* wo, int64_t N, void* workspace, size_t workspace_bytes, void* out,
+                    const int32_t* row_tab, hipStream_t stream);
 
 #ifdef __cplusplus
 }

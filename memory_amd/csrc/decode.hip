@@ -78,4 +78,59 @@ int moc_decode_partial(int dtype, const void* q, int64_t B, int H, const void* k
                            "moc_decode_partial", row_tab);
 }
 
+int moc_decode_route(const float* pooled, int64_t B, int64_t d, const void* W, int w_dtype, const float* bias, int64_t C,
+                     int S, int k, float scale, float* logits, int32_t* idx, float* w, int32_t* idx_star, float* omega,
+                     void* plan_ws, size_t plan_ws_bytes, int32_t* uniq, int32_t* n_uniq, int32_t* edge_u,
+                     int32_t* csr_off, int32_t* csr_edge, int64_t max_u, int32_t* row_tab, hipStream_t stream) {
+  const int64_t E = B * (S + k);
+  MOC_REQUIRE(max_u >= 0 && max_u <= E && max_u <= C, MOC_ERR_ARG, "moc_decode_route: max_u %lld", (long long)max_u);
+  if (int rc = moc_router_linear(pooled, B, d, W, w_dtype, bias, C, logits, stream)) return rc;
+  if (int rc = moc_router_topk_prepend(logits, B, C, S, k, scale, idx, w, idx_star, omega, stream)) return rc;
+  if (int rc = moc_chapter_plan(idx_star, E, C, plan_ws, plan_ws_bytes, uniq, n_uniq, edge_u, csr_off, csr_edge, stream))
+    return rc;
+  return moc_decode_row_table(n_uniq, csr_off, csr_edge, max_u, row_tab, stream);
+}
+
+namespace {
+struct StepLayout {
+  size_t q, o_part, a, lse_part, lse, bytes;
+  StepLayout(int64_t B, int H, int NS) {
+    const size_t row = (size_t)B * H * 64 * 2;
+    size_t o = 0;
+    auto take = [&](size_t n) { const size_t at = o; o += (n + 255) / 256 * 256; return at; };
+    q = take(row);
+    o_part = take(row * NS);
+    a = take(row);
+    lse_part = take((size_t)B * NS * H * 4);
+    lse = take((size_t)B * H * 4);
+    bytes = o;
+  }
+};
+}  // namespace
+
+size_t moc_decode_step_workspace(int64_t B, int H, int NS) {
+  return B < 0 || H <= 0 || NS <= 0 ? 0 : StepLayout(B, H, NS).bytes;
+}
+
+int moc_decode_step(const void* x, int64_t B, int64_t d, const void* wq, int H, const void* k_tiles, const void* v_tiles,
+                    int HK, int T, const int32_t* uniq, const int32_t* n_uniq, const int32_t* csr_off,
+                    const int32_t* csr_edge, const int32_t* edge_u, int64_t max_u, const float* omega, int NS,
+                    float scale, const void* wo, int64_t N, void* workspace, size_t workspace_bytes, void* out,
+                    const int32_t* row_tab, hipStream_t stream) {
+  MOC_REQUIRE(x && wq && wo && workspace && out && edge_u, MOC_ERR_ARG, "moc_decode_step: null pointer");
+  MOC_REQUIRE(B > 0 && H > 0 && NS > 0, MOC_ERR_ARG, "moc_decode_step: B=%lld H=%d NS=%d", (long long)B, H, NS);
+  const StepLayout y(B, H, NS);
+  MOC_REQUIRE(workspace_bytes >= y.bytes, MOC_ERR_ARG, "moc_decode_step: workspace %zu < %zu bytes", workspace_bytes,
+              y.bytes);
+  char* ws = (char*)workspace;
+  if (int rc = moc_linear_rows(x, B, d, wq, (int64_t)H * 64, MOC_BF16, ws + y.q, stream)) return rc;
+  if (int rc = moc_decode_partial(MOC_BF16, ws + y.q, B, H, k_tiles, v_tiles, HK, 64, T, uniq, n_uniq, csr_off, csr_edge,
+                                  max_u, omega, NS, scale, ws + y.o_part, (float*)(ws + y.lse_part), row_tab, stream))
+    return rc;
+  if (int rc = moc_sparse_combine(MOC_BF16, ws + y.o_part, (const float*)(ws + y.lse_part), edge_u, nullptr, 1, NS, H, B,
+                                  H, 0, ws + y.a, (float*)(ws + y.lse), stream))
+    return rc;
+  return moc_linear_rows(ws + y.a, B, (int64_t)H * 64, wo, N, MOC_BF16, out, stream);
+}
+
 }  // extern "C"

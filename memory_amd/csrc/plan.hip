@@ -194,11 +194,14 @@ __global__ __launch_bounds__(256) void plan_place_kernel(const int32_t* __restri
   }
 }
 
-// Whole plan in one workgroup for small batches (E <= 1024 edges, C <= 8192): the
-// histogram, both scans and the stable placement run out of LDS, so the plan
-// costs one launch instead of four (the sequence-level path has B * (S + k)
-// edges, 520 at the paper shape).  Same outputs as the general path.
-constexpr int kPlanSmallE = 1024;
+// Whole plan in one workgroup for small batches (E <= 4,096 edges, C <= 8,192): the histogram, both
+// scans and the stable placement run out of LDS, so the plan costs one launch instead of four (the
+// sequence-level path has B * (S + k) edges, 520 at the paper shape; re-routed decode of 16 sequences
+// 1,040).  Same outputs as the general path.  P edges per thread, placed 1,024 at a time.  Latency-bound
+// (one workgroup's barriers and LDS round trips): 5.4 us for 1,040 edges of 4,097 chapters, where the
+// four launches take 32.1.  The limit is what one workgroup's LDS holds beside 8,192 chapters' counts.
+constexpr int kPlanSmallP = 4;
+constexpr int kPlanSmallE = 1024 * kPlanSmallP;
 constexpr int kPlanSmallC = 8192;
 
 __device__ __forceinline__ int wave_incl_scan(int v) {
@@ -211,6 +214,7 @@ __device__ __forceinline__ int wave_incl_scan(int v) {
   return v;
 }
 
+template <int P>
 __global__ __launch_bounds__(1024) void plan_small_kernel(const int32_t* __restrict__ chap, int64_t E, int64_t C,
                                                           int32_t* __restrict__ uniq, int32_t* __restrict__ n_uniq,
                                                           int32_t* __restrict__ edge_u,
@@ -220,20 +224,20 @@ __global__ __launch_bounds__(1024) void plan_small_kernel(const int32_t* __restr
   int32_t* cnt = lds;          // [C] counts, then first csr position of each chapter
   int32_t* uid = lds + C;      // [C] unique index of each present chapter
   int32_t* fill = lds + 2 * C;  // [C] edges placed so far
-  __shared__ int32_t ids[kPlanSmallE];
-  __shared__ int32_t tmp[kPlanSmallE];
+  __shared__ int32_t tmp[1024 * P];
   __shared__ int32_t wsum[2][16];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   for (int64_t c = tid; c < C; c += 1024) {
     cnt[c] = 0;
     fill[c] = 0;
   }
-  if (tid < E) ids[tid] = chap[tid];
+  int32_t ids[P];   // edge 1024 p + tid
+#pragma unroll
+  for (int p = 0; p < P; ++p) ids[p] = 1024 * p + tid < E ? chap[1024 * p + tid] : -1;
   __syncthreads();
-  if (tid < E) {
-    const int32_t c = ids[tid];
-    if (c >= 0 && c < C) atomicAdd(&cnt[c], 1);  // out-of-range ids are dropped (counted below)
-  }
+#pragma unroll
+  for (int p = 0; p < P; ++p)
+    if (ids[p] >= 0 && ids[p] < C) atomicAdd(&cnt[ids[p]], 1);  // out-of-range ids are dropped (counted below)
   __syncthreads();
   // thread t owns bins [t * per, (t + 1) * per): local totals, block exclusive scan
   const int per = (int)((C + 1023) / 1024);
@@ -263,19 +267,29 @@ __global__ __launch_bounds__(1024) void plan_small_kernel(const int32_t* __restr
   }
   if (tid == 0) { n_uniq[0] = tot_f; n_uniq[1] = (int32_t)(E - tot_t); csr_off[tot_f] = tot_t; }
   __syncthreads();
-  // placement into the chapter's segment in arrival order, then the stable order: an edge's
-  // slot is the segment start plus the number of the segment's edges with a smaller id
-  const int32_t c = tid < E ? ids[tid] : -1;
-  const bool ok = c >= 0 && c < C;
-  if (ok) tmp[cnt[c] + atomicAdd(&fill[c], 1)] = tid;
-  __syncthreads();
-  if (tid < E) {
-    edge_u[tid] = ok ? uid[c] : -1;
-    if (ok) {
-      const int s0 = cnt[c], n = fill[c];
-      int before = 0;
-      for (int j = 0; j < n; ++j) before += tmp[s0 + j] < tid;
-      csr_edge[s0 + before] = tid;
+  // placement into the chapter's segment in arrival order, then the stable order: an edge's slot is
+  // the segment start plus the edges of earlier blocks of 1,024 plus those of its own block with a
+  // smaller id
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    const int e = 1024 * p + tid;
+    const int32_t c = ids[p];
+    const bool ok = c >= 0 && c < C;
+    int n0 = 0;
+    if (p > 0) {
+      if (ok) n0 = fill[c];
+      __syncthreads();
+    }
+    if (ok) tmp[cnt[c] + atomicAdd(&fill[c], 1)] = e;
+    __syncthreads();
+    if (e < E) {
+      edge_u[e] = ok ? uid[c] : -1;
+      if (ok) {
+        const int s0 = cnt[c], n = fill[c];
+        int before = n0;
+        for (int j = n0; j < n; ++j) before += tmp[s0 + j] < e;
+        csr_edge[s0 + before] = e;
+      }
     }
   }
 }
@@ -317,8 +331,13 @@ size_t plan_workspace_bytes(int64_t E, int64_t C) {
 int plan_launch(const int32_t* chap, int64_t E, int64_t C, void* workspace, int32_t* uniq, int32_t* n_uniq,
                 int32_t* edge_u, int32_t* csr_off, int32_t* csr_edge, hipStream_t stream) {
   if (E <= kPlanSmallE && C <= kPlanSmallC) {
-    hipLaunchKernelGGL(plan_small_kernel, dim3(1), dim3(1024), 3 * (size_t)C * sizeof(int32_t), stream, chap, E, C,
-                       uniq, n_uniq, edge_u, csr_off, csr_edge);
+    const size_t lds = 3 * (size_t)C * sizeof(int32_t);
+    if (E <= 1024)
+      hipLaunchKernelGGL(plan_small_kernel<1>, dim3(1), dim3(1024), lds, stream, chap, E, C, uniq, n_uniq, edge_u,
+                         csr_off, csr_edge);
+    else
+      hipLaunchKernelGGL(plan_small_kernel<kPlanSmallP>, dim3(1), dim3(1024), lds, stream, chap, E, C, uniq, n_uniq,
+                         edge_u, csr_off, csr_edge);
     return check_launch("plan_small_kernel");
   }
   const int G = (int)((E + kPlanEdgesPerBlock - 1) / kPlanEdgesPerBlock);

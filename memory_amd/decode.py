@@ -112,6 +112,34 @@ class DecodeRouting:
         call("moc_decode_row_table", ptr(self.plan.n_uniq), ptr(self.plan.csr_off), ptr(self.plan.csr_edge),
              self.max_units, ptr(self.row_tab), stream_ptr(self.idx.device))
 
+    @classmethod
+    def _decided(cls, pooled, router, num_chapters: int, num_shared: int, top_k: int, scale: float):
+        """(routing, logits) of pooled rows (B, d) f32: router linear, top-k with the shared prefix, plan and
+        row table in one host call (moc_decode_route), equal to the separate ones."""
+        B, d = pooled.shape
+        C, S, k = int(num_chapters), int(num_shared), int(top_k)
+        NS = S + k
+        E = B * NS
+        max_u = min(E, C)
+        dev = pooled.device
+        W = router.weight.contiguous()
+        bias = None if router.bias is None else router.bias.float().contiguous()
+        ws_bytes = L.query("moc_chapter_plan_workspace", E, C)
+        logits = torch.empty(B, C, device=dev, dtype=torch.float32)
+        w, omega = torch.empty(B * (k + NS), device=dev, dtype=torch.float32).split((B * k, E))
+        sizes = (ws_bytes // 4, max_u, 2, E, max_u + 1, E, 16 * max_u, E, B * k)
+        ws, uniq, n_uniq, edge_u, csr_off, csr_edge, row_tab, idx_star, idx = torch.empty(
+            sum(sizes), device=dev, dtype=torch.int32).split(sizes)
+        call("moc_decode_route", ptr(pooled), B, d, ptr(W), L.dtype_code(W.dtype), ptr(bias), C, S, k, scale, ptr(logits),
+             ptr(idx), ptr(w), ptr(idx_star), ptr(omega), ptr(ws), ws_bytes, ptr(uniq), ptr(n_uniq), ptr(edge_u),
+             ptr(csr_off), ptr(csr_edge), max_u, ptr(row_tab), stream_ptr(dev))
+        self = cls.__new__(cls)
+        self.idx, self.omega = idx_star.view(B, NS), omega.view(B, NS)
+        self.B, self.NS = B, NS
+        self.plan = ops.ChapterPlan(uniq, n_uniq, edge_u, csr_off, csr_edge, max_u, C)
+        self._n_unique, self.max_units, self.row_tab = None, max_u, row_tab
+        return self, logits
+
     def unique_chapters(self) -> int:
         if self._n_unique is None:
             self._n_unique = int(self.plan.n_uniq[0].item())
@@ -133,6 +161,17 @@ def _masked_mean(states: torch.Tensor, mask: Optional[torch.Tensor]) -> torch.Te
         mask = mask[:, -states.shape[1]:]
     m = mask.to(device=states.device, dtype=torch.float32).unsqueeze(-1)
     return (states.float() * m).sum(dim=1) / m.sum(dim=1).clamp(min=1.0)
+
+
+def _window_native(old: torch.Tensor, h: torch.Tensor) -> bool:
+    """Whether moc_window_pool takes the window and the new states (packed rows of one type, 16-byte aligned,
+    any batch stride)."""
+    d = h.shape[-1]
+    return (h.dim() == 3 and h.shape[1] > 0 and old.shape[1] > 0 and old.shape[0] == h.shape[0] and 0 < h.shape[0] < 65536
+            and old.shape[2] == d and d % 8 == 0 and h.dtype == old.dtype and h.dtype in (torch.float32, torch.bfloat16)
+            and h.device == old.device and all(
+                t.stride(2) == 1 and (t.stride(1) == d or t.shape[1] == 1) and t.stride(0) % 8 == 0
+                and t.data_ptr() % 16 == 0 for t in (old, h)))
 
 
 class DecodeRouter:
@@ -175,10 +214,15 @@ class DecodeRouter:
     def _decide(self, pooled: torch.Tensor) -> DecodeRouting:
         from .model import prepend_shared_chapters32
         r = self.router.router
-        logits = ops.router_linear(pooled, r.weight, r.bias)
-        self.last_logits = logits
         C, S = self.num_chapters, self.num_shared
         k = min(int(self.router.top_k), C - S)
+        if (S > 0 and k > 0 and pooled.shape[0] > 0 and pooled.dtype == torch.float32 and pooled.is_contiguous()
+                and r.weight.dtype in (torch.float32, torch.bfloat16) and r.weight.shape == (C, pooled.shape[1])
+                and r.weight.is_cuda and (r.bias is None or r.bias.is_cuda) and L.KERNEL_EVENTS is None):
+            routing, self.last_logits = DecodeRouting._decided(pooled, r, C, S, k, self.routed_scale)
+            return routing
+        logits = ops.router_linear(pooled, r.weight, r.bias)
+        self.last_logits = logits
         if k > 0:
             idx, w = ops.router_topk(logits, k, S)
         else:
@@ -196,11 +240,27 @@ class DecodeRouter:
         return ops.router_pool(hidden_states, coef)
 
     def _window(self, hidden_states: torch.Tensor, attention_mask: Optional[torch.Tensor]) -> torch.Tensor:
+        if self.cache is not None and attention_mask is None and _window_native(self.cache, hidden_states):
+            return self._advance(hidden_states)
         combined = hidden_states if self.cache is None else torch.cat([self.cache, hidden_states], dim=1)
         if combined.shape[1] > self.window:
             combined = combined[:, -self.window:]
         self.cache = combined.detach()
         return _masked_mean(combined, attention_mask)
+
+    def _advance(self, hidden_states: torch.Tensor) -> torch.Tensor:
+        """The window moved on by the new states and its mean, in one pass (moc_window_pool)."""
+        old, h = self.cache, hidden_states
+        B, n_old, d = old.shape
+        n_new = h.shape[1]
+        n = min(n_old + n_new, self.window)
+        out = torch.empty(B, n, d, device=h.device, dtype=h.dtype)
+        ws_bytes = L.query("moc_router_pool_workspace", B, n, d)
+        pooled = torch.empty(B * d + ws_bytes // 4, device=h.device, dtype=torch.float32)
+        call("moc_window_pool", ptr(old), old.stride(0), n_old, ptr(h), h.stride(0), n_new, L.dtype_code(h.dtype), B, n, d,
+             ptr(out), ptr(pooled), pooled.data_ptr() + 4 * B * d, ws_bytes, stream_ptr(h.device))
+        self.cache = out
+        return pooled[:B * d].view(B, d)
 
     @torch.no_grad()
     def prefill(self, hidden_states: torch.Tensor, attention_mask: Optional[torch.Tensor] = None) -> DecodeRouting:
@@ -248,6 +308,17 @@ def decode_attention(q: torch.Tensor, cache: MemoryDecodeCache, routing: DecodeR
     return out
 
 
+def _step_native(x, wq, wo, H: int, cache: MemoryDecodeCache, routing: DecodeRouting) -> bool:
+    """Whether moc_decode_step takes the step (bf16 throughout, few rows; with the per-kernel timing armed
+    the kernels run as separate entry points).  A re-routed step of 16 sequences: 172 to 182 us with a call
+    per kernel, most of it host time, 91 with three calls."""
+    return (cache.dtype == torch.bfloat16 and wo.dtype == torch.bfloat16 and 0 < x.shape[0] == routing.B
+            and ops._few_rows(x, wq) and wo.is_cuda and H % 2 == 0 and wq.shape == (64 * H, x.shape[1])
+            and wo.shape[0] % 16 == 0 and wo.shape[1] == 64 * H and cache.k_tiles.is_cuda and H % cache.HK == 0
+            and x.data_ptr() % 16 == 0 and wq.data_ptr() % 16 == 0 and wo.data_ptr() % 16 == 0
+            and L.KERNEL_EVENTS is None)
+
+
 def memory_decode_step(memory_attn, hidden: torch.Tensor, cache: MemoryDecodeCache,
                        routing: DecodeRouting) -> torch.Tensor:
     """One decode step of a memory sublayer: hidden (B, 1, d) -> (B, 1, d) (before the residual)."""
@@ -255,7 +326,19 @@ def memory_decode_step(memory_attn, hidden: torch.Tensor, cache: MemoryDecodeCac
     H = memory_attn.num_heads
     with torch.no_grad():
         wq, wo = memory_attn.q_proj.weight, memory_attn.o_proj.weight
-        q = ops.linear(hidden.reshape(B, -1).to(wq.dtype), wq).view(B, H, memory_attn.head_dim)
+        x = hidden.reshape(B, -1).to(wq.dtype)
+        if _step_native(x, wq, wo, H, cache, routing):
+            x, wq, wo = x.contiguous(), wq.contiguous(), wo.contiguous()
+            pl, NS, N = routing.plan, routing.NS, wo.shape[0]
+            nbytes = L.query("moc_decode_step_workspace", B, H, NS)
+            ws = torch.empty(nbytes, device=x.device, dtype=torch.uint8)
+            out = torch.empty(B, 1, N, device=x.device, dtype=x.dtype)
+            call("moc_decode_step", ptr(x), B, x.shape[1], ptr(wq), H, ptr(cache.k_tiles), ptr(cache.v_tiles), cache.HK,
+                 cache.T, ptr(pl.uniq), ptr(pl.n_uniq), ptr(pl.csr_off), ptr(pl.csr_edge), ptr(pl.edge_u),
+                 routing.max_units, ptr(routing.omega), NS, 0.125, ptr(wo), N, ptr(ws), nbytes, ptr(out),
+                 ptr(routing.row_tab), stream_ptr(x.device))
+            return out
+        q = ops.linear(x, wq).view(B, H, memory_attn.head_dim)
         a = decode_attention(q, cache, routing)
         return ops.linear(a.reshape(B, 1, -1).to(wo.dtype), wo)
 
