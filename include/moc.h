@@ -728,6 +728,17 @@ int moc_decode_step(const void* x, int64_t B, int64_t d, const void* wq, int H, 
                     const int32_t* csr_edge, const int32_t* edge_u, int64_t max_u, const float* omega, int NS,
                     float scale, const void* wo, int64_t N, void* workspace, size_t workspace_bytes, void* out,
                     const int32_t* row_tab, hipStream_t stream);
+/* moc_decode_step of n independent layers of one shape (9 <= NS <= 68 slots, B * H <= 16,384), one launch per
+ * kernel and eight layers; workspace_bytes: moc_decode_step_workspace, for each layer's own workspace. */
+typedef struct {
+  const void *x, *wq, *k_tiles, *v_tiles, *wo;
+  const int32_t *uniq, *n_uniq, *csr_off, *csr_edge, *edge_u, *row_tab;
+  const float* omega;
+  void *workspace, *out;
+  int64_t max_u;
+} moc_decode_layer;
+int moc_decode_step_group(const moc_decode_layer* layers, int n, int64_t B, int64_t d, int H, int HK, int T, int NS,
+                          float scale, int64_t N, size_t workspace_bytes, hipStream_t stream);
 
 #ifdef __cplusplus
 }

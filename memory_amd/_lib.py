@@ -52,6 +52,7 @@ _SIGS = {
                                   _I, _F, _I, _P, _P, _P, _P, _P, _P, _SZ, _P, _P]),
     "moc_seq_layer_bwd_ex": (_I, [_P, _P, _P, _I, _P, _I64, _I64, _I64, _I, _I, _I64, _I, _I, _F, _I, _P, _P, _P, _P,
                                   _SZ, _P, _P, _P, _P, _I64, _P, _P, _P, _P, _I, _P, _P, _SZ, _P, _P, _P]),
+    "moc_decode_step_group": (_I, [_P, _I, _I64, _I64, _I, _I, _I, _I, _F, _I64, _SZ, _P]),
     "moc_window_pool": (_I, [_P, _I64, _I64, _P, _I64, _I64, _I, _I64, _I64, _I64, _P, _P, _P, _SZ, _P]),
     "moc_decode_route": (_I, [_P, _I64, _I64, _P, _I, _P, _I64, _I, _I, _F, _P, _P, _P, _P, _P, _P, _SZ, _P, _P, _P,
                               _P, _P, _I64, _P, _P]),

@@ -20,6 +20,8 @@
 // instead of after them, and its q rows go out together with its K / V tiles.
 #include "moc_common.h"
 
+#include <algorithm>
+
 using namespace moc;
 
 namespace {
@@ -131,6 +133,39 @@ int moc_decode_step(const void* x, int64_t B, int64_t d, const void* wq, int H, 
                                   H, 0, ws + y.a, (float*)(ws + y.lse), stream))
     return rc;
   return moc_linear_rows(ws + y.a, B, (int64_t)H * 64, wo, N, MOC_BF16, out, stream);
+}
+
+int moc_decode_step_group(const moc_decode_layer* layers, int n, int64_t B, int64_t d, int H, int HK, int T, int NS,
+                          float scale, int64_t N, size_t workspace_bytes, hipStream_t stream) {
+  MOC_REQUIRE(layers && n > 0, MOC_ERR_ARG, "moc_decode_step_group: no layers");
+  MOC_REQUIRE(T == 64 && B > 0 && H > 0 && HK > 0 && H % HK == 0 && NS > 8 && NS <= 68 && B * H <= 16384,
+              MOC_ERR_UNSUPPORTED, "moc_decode_step_group: B=%lld H=%d HK=%d T=%d NS=%d", (long long)B, H, HK, T, NS);
+  const StepLayout y(B, H, NS);
+  MOC_REQUIRE(workspace_bytes >= y.bytes, MOC_ERR_ARG, "moc_decode_step_group: workspace %zu < %zu bytes",
+              workspace_bytes, y.bytes);
+  for (int i = 0; i < n; ++i) {
+    const moc_decode_layer& l = layers[i];
+    MOC_REQUIRE(l.x && l.wq && l.k_tiles && l.v_tiles && l.wo && l.uniq && l.n_uniq && l.csr_off && l.csr_edge && l.edge_u &&
+                    l.omega && l.workspace && l.out && l.max_u >= 0 && l.max_u < (1 << 24) &&
+                    (((uintptr_t)l.x | (uintptr_t)l.wq | (uintptr_t)l.wo | (uintptr_t)l.workspace) & 15) == 0,
+                MOC_ERR_ARG, "moc_decode_step_group: layer %d: null or unaligned pointer", i);
+  }
+  for (int i0 = 0; i0 < n; i0 += kDecodeGroup) {
+    const int m = std::min(kDecodeGroup, n - i0);
+    DecodeGroup grp{};
+    for (int i = 0; i < m; ++i) {
+      const moc_decode_layer& l = layers[i0 + i];
+      char* ws = (char*)l.workspace;
+      grp.l[i] = DecodeLayer{(const bf16*)l.x, (const bf16*)l.wq, (const bf16*)l.k_tiles, (const bf16*)l.v_tiles,
+                             (const bf16*)l.wo, l.uniq, l.n_uniq, l.csr_off, l.csr_edge, l.edge_u, l.row_tab, l.omega,
+                             (bf16*)(ws + y.q), (bf16*)(ws + y.o_part), (bf16*)(ws + y.a), (bf16*)l.out,
+                             (float*)(ws + y.lse_part), (float*)(ws + y.lse), l.max_u};
+    }
+    if (int rc = decode_linear_group(grp, m, false, B, d, (int64_t)H * 64, stream)) return rc;
+    if (int rc = decode_attend_group(grp, m, B, H, HK, NS, scale, stream)) return rc;
+    if (int rc = decode_linear_group(grp, m, true, B, (int64_t)H * 64, N, stream)) return rc;
+  }
+  return MOC_OK;
 }
 
 }  // extern "C"

@@ -371,6 +371,28 @@ bool mid_linear_takes(int64_t M, int N, int K);
 int mid_linear(const void* x, int64_t ldx, int64_t M, const void* w, int N, int K, void* y, int64_t ldy,
                const void* res, int64_t ldr, hipStream_t stream);
 
+// One layer's operands of a grouped decode step (moc_decode_step_group): the kernels of up to
+// kDecodeGroup layers run as one launch each, the layer on the grid.  Bound by launch latency and the
+// kernels' own round trips at few sequences, by HBM at many; four layers of 1 / 4 / 16 / 64 sequences
+// at 65 of 4,097 chapters, a replay with a chain of kernels per layer -> grouped: 77 -> 34, 101 -> 54,
+// 205 -> 155, 441 -> 405 us.  (The layers as parallel branches of the graph: 124, 138, 199, 451 us.)
+constexpr int kDecodeGroup = 8;
+struct DecodeLayer {
+  const bf16 *x, *wq, *k, *v, *wo;
+  const int32_t *uniq, *n_uniq, *csr_off, *csr_edge, *edge_u, *row_tab;
+  const float* omega;
+  bf16 *q, *o_part, *a, *out;
+  float *lse_part, *lse;
+  int64_t max_u;
+};
+struct DecodeGroup {
+  DecodeLayer l[kDecodeGroup];
+};
+int decode_linear_group(const DecodeGroup& grp, int layers, bool out, int64_t M, int64_t K, int64_t N,
+                        hipStream_t stream);
+int decode_attend_group(const DecodeGroup& grp, int layers, int64_t B, int H, int HK, int NS, float scale,
+                        hipStream_t stream);
+
 // moc_gemm_f32 of any size it can index, with c += op(a) op(b) when `add` is set (gemm_f32.hip).
 int gemm_f32(int ta, int tb, int64_t M, int64_t N, int64_t K, const float* a, int64_t lda, const float* b, int64_t ldb,
              float* c, int64_t ldc, int add, hipStream_t stream);

@@ -19,9 +19,8 @@ constexpr int kSlRows = 16 * kSlTiles;
 constexpr int kSlChunks = 6;      // 32-wide K chunks a wave holds in registers at once
 
 template <typename TO>
-__global__ __launch_bounds__(64 * kSlWaves) void small_linear_kernel(const bf16* __restrict__ x, int M, int K,
-                                                                    const bf16* __restrict__ W, int N,
-                                                                    TO* __restrict__ y) {
+__device__ __forceinline__ void small_linear_tile(const bf16* __restrict__ x, int M, int K, const bf16* __restrict__ W,
+                                                  int N, TO* __restrict__ y) {
   __shared__ f32x4 red[kSlWaves][kSlTiles][64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int g = lane >> 4, c16 = lane & 15;
@@ -69,6 +68,24 @@ __global__ __launch_bounds__(64 * kSlWaves) void small_linear_kernel(const bf16*
     const int m = m0 + 16 * mt + 4 * g + e;
     if (m < M) y[(size_t)m * N + n0 + c16] = from_f<TO>(s[e]);
   }
+}
+
+template <typename TO>
+__global__ __launch_bounds__(64 * kSlWaves) void small_linear_kernel(const bf16* __restrict__ x, int M, int K,
+                                                                    const bf16* __restrict__ W, int N,
+                                                                    TO* __restrict__ y) {
+  small_linear_tile<TO>(x, M, K, W, N, y);
+}
+
+// The projections of several layers' decode steps in one launch (blockIdx.z = layer): q = x wq^T, or
+// out = a wo^T with OUT.
+template <bool OUT>
+__global__ __launch_bounds__(64 * kSlWaves) void decode_linear_group_kernel(DecodeGroup grp, int M, int K, int N) {
+  const DecodeLayer& l = grp.l[blockIdx.z];
+  if constexpr (OUT)
+    small_linear_tile<bf16>(l.a, M, K, l.wo, N, l.out);
+  else
+    small_linear_tile<bf16>(l.x, M, K, l.wq, N, l.q);
 }
 
 // The same idea for a few hundred rows (a prompt's q_proj / o_proj, few rows per training step): a
@@ -180,6 +197,20 @@ int mid_linear(const void* x, int64_t ldx, int64_t M, const void* w, int N, int 
 }  // namespace moc
 
 using namespace moc;
+
+int moc::decode_linear_group(const DecodeGroup& grp, int layers, bool out, int64_t M, int64_t K, int64_t N,
+                             hipStream_t stream) {
+  MOC_REQUIRE(M > 0 && M <= 256 && K > 0 && N > 0 && K % (32 * kSlWaves) == 0 && N % 16 == 0 && K <= 65536 && N <= 65536,
+              MOC_ERR_UNSUPPORTED, "decode_linear_group: M=%lld (at most 256 rows), K=%lld, N=%lld", (long long)M,
+              (long long)K, (long long)N);
+  const dim3 grid((unsigned)(N / 16), (unsigned)((M + kSlRows - 1) / kSlRows), (unsigned)layers);
+  if (out)
+    hipLaunchKernelGGL(decode_linear_group_kernel<true>, grid, dim3(64 * kSlWaves), 0, stream, grp, (int)M, (int)K, (int)N);
+  else
+    hipLaunchKernelGGL(decode_linear_group_kernel<false>, grid, dim3(64 * kSlWaves), 0, stream, grp, (int)M, (int)K,
+                       (int)N);
+  return check_launch("decode_linear_group_kernel");
+}
 
 extern "C" {
 

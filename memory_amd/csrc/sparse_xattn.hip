@@ -330,7 +330,7 @@ __global__ __launch_bounds__(64 * kCombWaves) void sparse_combine_kernel(const T
 constexpr int kCombSmallPerGroup = 17;
 
 template <typename T>
-__global__ __launch_bounds__(64 * kCombWaves) void sparse_combine_small_kernel(
+__device__ __forceinline__ void sparse_combine_small_row(
     const T* __restrict__ o_part, const float* __restrict__ lse_part, const int32_t* __restrict__ edge_u,
     const float* __restrict__ w, int mode, int S, int rpe, int64_t ntok, int HQ, int hq_off, T* __restrict__ out,
     float* __restrict__ lse_joint) {
@@ -396,6 +396,20 @@ __global__ __launch_bounds__(64 * kCombWaves) void sparse_combine_small_kernel(
     if (lane == 0) lse_joint[row] = den > 0.f ? M + log2f(den) : INFINITY;
   }
   sp_row_store(out + ((int64_t)tok * HQ + hq_off + r) * kSpDh, acc, inv, lane);
+}
+
+template <typename T>
+__global__ __launch_bounds__(64 * kCombWaves) void sparse_combine_small_kernel(
+    const T* __restrict__ o_part, const float* __restrict__ lse_part, const int32_t* __restrict__ edge_u,
+    const float* __restrict__ w, int mode, int S, int rpe, int64_t ntok, int HQ, int hq_off, T* __restrict__ out,
+    float* __restrict__ lse_joint) {
+  sparse_combine_small_row<T>(o_part, lse_part, edge_u, w, mode, S, rpe, ntok, HQ, hq_off, out, lse_joint);
+}
+
+// The joint combine of several layers' decode steps (blockIdx.y = layer).
+__global__ __launch_bounds__(64 * kCombWaves) void decode_combine_group_kernel(DecodeGroup grp, int NS, int H, int64_t B) {
+  const DecodeLayer& l = grp.l[blockIdx.y];
+  sparse_combine_small_row<bf16>(l.o_part, l.lse_part, l.edge_u, nullptr, 1, NS, H, B, H, 0, l.a, l.lse);
 }
 
 // The combine for at most kCombFew slots: a row of 64 dims is LPR lanes of 16 bytes each, and those
@@ -953,7 +967,7 @@ __device__ __forceinline__ void unit_dma16(__amdgpu_buffer_rsrc_t r, uint32_t vo
 // fragments straight into registers, and the first 16-row block's edge ids before both, so its
 // q loads go out while the tiles are in flight.  Rows are taken 16 at a time (a decode unit has
 // one or two).
-__global__ __launch_bounds__(64 * kUnitWaves) void sparse_fwd_unit_kernel(
+__device__ __forceinline__ void sparse_fwd_unit(
     const bf16* __restrict__ q, int HQ, const bf16* __restrict__ k, const bf16* __restrict__ v, int64_t cs,
     int64_t hs, int64_t rs, int HK, const int32_t* __restrict__ uniq, const int32_t* __restrict__ n_uniq,
     const int32_t* __restrict__ csr_off, const int32_t* __restrict__ csr_edge, int64_t max_u, int S, int hk0,
@@ -1066,6 +1080,26 @@ __global__ __launch_bounds__(64 * kUnitWaves) void sparse_fwd_unit_kernel(
       if (g == 0) lse_part[erow] = m + log2f(l);
     }
   }
+}
+
+__global__ __launch_bounds__(64 * kUnitWaves) void sparse_fwd_unit_kernel(
+    const bf16* __restrict__ q, int HQ, const bf16* __restrict__ k, const bf16* __restrict__ v, int64_t cs,
+    int64_t hs, int64_t rs, int HK, const int32_t* __restrict__ uniq, const int32_t* __restrict__ n_uniq,
+    const int32_t* __restrict__ csr_off, const int32_t* __restrict__ csr_edge, int64_t max_u, int S, int hk0,
+    int nhk, int hq_off, int rpe, float scale_log2, bf16* __restrict__ o_part, float* __restrict__ lse_part,
+    const float* __restrict__ omega, const int32_t* __restrict__ row_tab, int kvdiv) {
+  sparse_fwd_unit(q, HQ, k, v, cs, hs, rs, HK, uniq, n_uniq, csr_off, csr_edge, max_u, S, hk0, nhk, hq_off, rpe, scale_log2,
+                  o_part, lse_part, omega, row_tab, kvdiv);
+}
+
+// The units of several layers' decode steps (blockIdx.y = layer, each with its own plan and tiles).  One
+// layer of one sequence is 195 workgroups of a few microseconds' latency, mostly idle CUs: four layers
+// in one launch take 12.1 us, one alone 6.3.
+__global__ __launch_bounds__(64 * kUnitWaves) void decode_unit_group_kernel(DecodeGroup grp, int H, int HK, int NS,
+                                                                            float scale_log2) {
+  const DecodeLayer& l = grp.l[blockIdx.y];
+  sparse_fwd_unit(l.q, H, l.k, l.v, (int64_t)HK * 4096, 4096, 64, HK, l.uniq, l.n_uniq, l.csr_off, l.csr_edge, l.max_u, NS, 0,
+                  HK, 0, H, scale_log2, l.o_part, l.lse_part, l.omega, l.row_tab, 1);
 }
 
 // Backward of one unit on a workgroup of two waves, wave w owning keys 32 w .. 32 w + 31
@@ -1512,6 +1546,27 @@ int moc::sparse_fwd_launch(int dtype, const void* q, int HQ, const void* k, cons
     return check_launch("sparse_fwd_kernel");
   }
   return set_error(MOC_ERR_UNSUPPORTED, "%s: dtype %d", who, dtype);
+}
+
+int moc::decode_attend_group(const DecodeGroup& grp, int layers, int64_t B, int H, int HK, int NS, float scale,
+                             hipStream_t stream) {
+  MOC_REQUIRE(H > 0 && HK > 0 && H % HK == 0 && NS > 0 && NS <= 4 * kCombSmallPerGroup && B > 0 && B * H <= 16384,
+              MOC_ERR_UNSUPPORTED, "decode_attend_group: B=%lld H=%d HK=%d NS=%d", (long long)B, H, HK, NS);
+  int64_t units = 0;
+  for (int i = 0; i < layers; ++i) {
+    const DecodeLayer& l = grp.l[i];
+    MOC_REQUIRE(unit_kv_aligned(l.q, l.k, l.v, 4096, 4096, 64) && (((uintptr_t)l.o_part | (uintptr_t)l.a) & 15) == 0,
+                MOC_ERR_ARG, "decode_attend_group: 16-byte aligned q / k / v / o_part / a");
+    units = max(units, l.max_u * HK);
+  }
+  if (units > 0) {
+    hipLaunchKernelGGL(decode_unit_group_kernel, dim3((unsigned)((units + kUnitWaves - 1) / kUnitWaves), (unsigned)layers),
+                       dim3(64 * kUnitWaves), 0, stream, grp, H, HK, NS, scale * 1.4426950408889634f);
+    if (int rc = check_launch("decode_unit_group_kernel")) return rc;
+  }
+  hipLaunchKernelGGL(decode_combine_group_kernel, dim3((unsigned)((B * H + kCombWaves - 1) / kCombWaves), (unsigned)layers),
+                     dim3(64 * kCombWaves), 0, stream, grp, NS, H, B);
+  return check_launch("decode_combine_group_kernel");
 }
 
 int moc::sparse_bwd_launch(int dtype, const void* q, const void* dout, int64_t ntok, int HQ, const void* k,

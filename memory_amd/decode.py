@@ -12,6 +12,7 @@ sequence's slots -> o_proj.  Inference only (no autograd).
 
 from __future__ import annotations
 
+import ctypes
 from typing import Optional
 
 import torch
@@ -343,10 +344,54 @@ def memory_decode_step(memory_attn, hidden: torch.Tensor, cache: MemoryDecodeCac
         return ops.linear(a.reshape(B, 1, -1).to(wo.dtype), wo)
 
 
+class _Layer(ctypes.Structure):
+    """moc_decode_layer."""
+    _fields_ = [(n, ctypes.c_void_p) for n in ("x", "wq", "k_tiles", "v_tiles", "wo", "uniq", "n_uniq", "csr_off",
+                                               "csr_edge", "edge_u", "row_tab", "omega", "workspace", "out")]
+    _fields_.append(("max_u", ctypes.c_int64))
+
+
+def _group_native(layers, inputs) -> bool:
+    """Whether the layers' steps run as one group (moc_decode_step_group): several, each on the one-call
+    step, of one shape, with the slot counts its combine kernel takes."""
+    shapes = set()
+    for (attn, cache, routing), h in zip(layers, inputs):
+        wq, wo, H = attn.q_proj.weight, attn.o_proj.weight, attn.num_heads
+        if h.dtype != wq.dtype or not (h.is_contiguous() and wq.is_contiguous() and wo.is_contiguous()):
+            return False
+        x = h.reshape(h.shape[0], -1)
+        if not _step_native(x, wq, wo, H, cache, routing) or cache.T != 64 or x.device != inputs[0].device:
+            return False
+        shapes.add((x.shape, H, cache.HK, routing.NS, wo.shape))
+    return len(layers) > 1 and len(shapes) == 1 and 8 < routing.NS <= 68 and routing.B * H <= 16384
+
+
+def _decode_steps(layers, inputs):
+    """memory_decode_step of every layer of a group, one launch per kernel for all of them."""
+    with torch.no_grad():
+        x = inputs[0]
+        B, dev = x.shape[0], x.device
+        attn, cache, routing = layers[0]
+        H, NS, N = attn.num_heads, routing.NS, attn.o_proj.weight.shape[0]
+        nbytes = L.query("moc_decode_step_workspace", B, H, NS)
+        ws = torch.empty(len(layers), nbytes, device=dev, dtype=torch.uint8)
+        outs = [torch.empty(B, 1, N, device=dev, dtype=x.dtype) for _ in layers]
+        args = (_Layer * len(layers))()
+        for i, ((attn, c, r), h) in enumerate(zip(layers, inputs)):
+            p = r.plan
+            args[i] = _Layer(ptr(h), ptr(attn.q_proj.weight), ptr(c.k_tiles), ptr(c.v_tiles), ptr(attn.o_proj.weight),
+                             ptr(p.uniq), ptr(p.n_uniq), ptr(p.csr_off), ptr(p.csr_edge), ptr(p.edge_u), ptr(r.row_tab),
+                             ptr(r.omega), ws[i].data_ptr(), ptr(outs[i]), r.max_units)
+        call("moc_decode_step_group", ctypes.addressof(args), len(layers), B, x.numel() // B, H, cache.HK, cache.T, NS,
+             0.125, N, nbytes, stream_ptr(dev))
+        return outs
+
+
 class DecodeStepGraph:
     """The per-token decode of several memory sublayers captured once as a HIP graph
     (torch.cuda.CUDAGraph) and replayed for every generated token: one graph launch replaces
-    the ~4 kernel launches per layer, and their inter-launch gaps.
+    the ~4 kernel launches per layer, and their inter-launch gaps.  Layers of one shape are captured
+    together, one launch per kernel for all of them (every layer's input is given at once).
 
     ``layers`` is a list of (memory_attn, cache, routing); ``inputs`` the per-layer hidden
     states (B, 1, d) used for the capture (their shapes and dtypes are fixed).  ``run(inputs)``
@@ -370,6 +415,8 @@ class DecodeStepGraph:
             self.static_out = self._body()
 
     def _body(self):
+        if _group_native(self.layers, self.static_in):
+            return _decode_steps(self.layers, self.static_in)
         return [memory_decode_step(attn, x, cache, routing)
                 for (attn, cache, routing), x in zip(self.layers, self.static_in)]
 
@@ -377,8 +424,11 @@ class DecodeStepGraph:
         """Replay with ``inputs`` (copied into the captured input buffers unless they are those
         buffers: a serving loop that writes each token's hidden states into ``static_in``
         directly replays with no copies)."""
-        for buf, x in zip(self.static_in, inputs):
-            if x.data_ptr() != buf.data_ptr():
+        new = [(buf, x) for buf, x in zip(self.static_in, inputs) if x.data_ptr() != buf.data_ptr()]
+        if len(new) > 1 and all(x.shape == buf.shape and x.dtype == buf.dtype and x.device == buf.device for buf, x in new):
+            torch._foreach_copy_([buf for buf, _ in new], [x for _, x in new])
+        else:
+            for buf, x in new:
                 buf.copy_(x)
         self.graph.replay()
         return self.static_out

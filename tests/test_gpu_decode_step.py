@@ -100,3 +100,48 @@ def test_step_equals_separate_calls(gpu_device, monkeypatch, B, d, H, HK, C, S, 
     for a, b in zip(*runs):
         for x, y in zip(a, b):
             assert x.shape == y.shape and x.dtype == y.dtype and torch.equal(x, y)
+
+
+@pytest.mark.parametrize("n,B,H,HK,C,k,grouped", [(2, 1, 4, 4, 90, 64, True), (9, 3, 4, 2, 40, 8, True),
+                                                  (3, 17, 12, 12, 120, 67, True), (2, 2, 4, 4, 40, 7, False),
+                                                  (2, 2, 4, 4, 90, 68, False), (1, 2, 4, 4, 40, 20, False)])
+def test_graph_groups_layers(gpu_device, monkeypatch, n, B, H, HK, C, k, grouped):
+    """Layers of one shape captured as one launch per kernel: every replay equals the layers' own steps;
+    other slot counts, single layers and layers of different shapes keep a chain each."""
+    from memory_amd import decode
+    from memory_amd.memory_attention import MemoryCrossAttention
+    dev = gpu_device
+    d = 64 * H
+    g = gen(n * 100 + k)
+    layers = []
+    for i in range(n):
+        attn = MemoryCrossAttention(d, H, HK, wo_init_zero=False).to(dev, BF)
+        bank = torch.randn(C * 64, d, generator=g).to(dev, BF)
+        cache = decode.MemoryDecodeCache(bank, attn.k_proj.weight, attn.v_proj.weight, num_chapters=C,
+                                         tokens_per_chapter=64, num_kv_heads=HK)
+        idx = torch.stack([torch.randperm(C, generator=g)[:k + 1] for _ in range(B)])
+        if i == 1:
+            idx[:] = idx[0]                 # one set of chapters for every sequence: fewer units
+        w = torch.rand(B, k + 1, generator=g) + 0.1
+        layers.append((attn, cache, decode.DecodeRouting(idx.to(dev), w.to(dev), C, sync=i != 0)))
+    called = []
+    real = decode.call
+    monkeypatch.setattr(decode, "call", lambda name, *a: (called.append(name), real(name, *a))[1])
+    xs = [torch.randn(B, 1, d, generator=g).to(dev, BF) for _ in range(n)]
+    graph = decode.DecodeStepGraph(layers, xs)
+    assert ("moc_decode_step_group" in called) == grouped
+    for rep in range(3):
+        inputs = [torch.randn(B, 1, d, generator=g).to(dev, BF) for _ in range(n)]
+        outs = [o.clone() for o in graph.run(inputs)]
+        junk = torch.randn(1000, device=dev).sum()
+        torch.cuda.synchronize()
+        for i, ((a, c, r), x) in enumerate(zip(layers, inputs)):
+            assert torch.equal(outs[i], decode.memory_decode_step(a, x, c, r)), (rep, i)
+        graph.static_in[0].copy_(inputs[-1])      # inputs written straight into the captured buffers
+        outs = graph.run(graph.static_in)
+        assert torch.equal(outs[0], decode.memory_decode_step(layers[0][0], inputs[-1], *layers[0][1:]))
+    if grouped:
+        other = MemoryCrossAttention(d, H, 1, wo_init_zero=False).to(dev, BF)
+        cache = decode.MemoryDecodeCache(bank, other.k_proj.weight, other.v_proj.weight, num_chapters=C,
+                                         tokens_per_chapter=64, num_kv_heads=1)
+        assert not decode._group_native(layers + [(other, cache, layers[0][2])], xs + xs[:1])
