@@ -234,7 +234,7 @@ struct SeqLayout {
 // The float32 layer (moc_seq_layer_f32_*): the reference's small configurations, where a step is some
 // thirty launches of 2 to 20 us each and the host issuing them one autograd function at a time was what it
 // waited for (692 us of host time for 199 us of kernels at 2 x 128 tokens, d = 256; in one call each way
-// 295 us).  One stream: nothing here is long enough to be worth an event.
+// 194 us).  One stream: nothing here is long enough to be worth an event.
 struct SeqF32Layout {
   int64_t B, L, d, C, E, max_u;
   int NS, KV, Lp;

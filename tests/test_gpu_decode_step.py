@@ -145,3 +145,12 @@ def test_graph_groups_layers(gpu_device, monkeypatch, n, B, H, HK, C, k, grouped
         cache = decode.MemoryDecodeCache(bank, other.k_proj.weight, other.v_proj.weight, num_chapters=C,
                                          tokens_per_chapter=64, num_kv_heads=1)
         assert not decode._group_native(layers + [(other, cache, layers[0][2])], xs + xs[:1])
+
+
+def test_stream_ptr(gpu_device):
+    from memory_amd._lib import stream_ptr
+    side = torch.cuda.Stream()
+    for st in (torch.cuda.current_stream(), side):
+        with torch.cuda.stream(st):
+            for dev in (None, torch.device("cuda"), torch.device("cuda", torch.cuda.current_device())):
+                assert stream_ptr(dev) == st.cuda_stream
