@@ -150,8 +150,8 @@ def cpu_model() -> str:
 PROBE_BYTES = 256 << 20
 # entry point -> device kernel whose HBM traffic the counter passes measured
 # entry point / native-layer stage -> the device kernel its roofline figures are about
-TRAFFIC_KERNELS = {"moc_xattn_bwd_dkv": "xattn_bwd_dkv_kernel<bf16>", "moc_xattn_fwd": "xattn_fwd_kernel<bf16>",
-                   "moc_xattn_bwd_dq": "xattn_bwd_dq_kernel<bf16>", "moc_kv_project": "kv_project_wide_kernel",
+TRAFFIC_KERNELS = {"moc_xattn_bwd_dkv": "xattn_bwd_dkv_kernel<bf16>", "moc_xattn_fwd": "xattn_fwd_kernel<bf16,0>",
+                   "moc_xattn_bwd_dq": "xattn_bwd_dq_kernel<bf16,0>", "moc_kv_project": "kv_project_wide_kernel",
                    "moc_decode_partial": "sparse_fwd_unit_kernel", "moc_sparse_bwd": "sparse_bwd_unit_kernel",
                    "moc_bank_adamw": "bank_adamw_kernel"}
 
