@@ -194,13 +194,14 @@ __global__ __launch_bounds__(256) void plan_place_kernel(const int32_t* __restri
   }
 }
 
-// Whole plan in one workgroup for small batches (E <= 4,096 edges, C <= 8,192): the histogram, both
+// Whole plan in one workgroup for small batches (E <= 8,192 edges, C <= 8,192): the histogram, both
 // scans and the stable placement run out of LDS, so the plan costs one launch instead of four (the
 // sequence-level path has B * (S + k) edges, 520 at the paper shape; re-routed decode of 16 sequences
-// 1,040).  Same outputs as the general path.  P edges per thread, placed 1,024 at a time.  Latency-bound
-// (one workgroup's barriers and LDS round trips): 5.4 us for 1,040 edges of 4,097 chapters, where the
-// four launches take 32.1.  The limit is what one workgroup's LDS holds beside 8,192 chapters' counts.
-constexpr int kPlanSmallP = 4;
+// 1,040, a prompt of 301 tokens routed one by one 4,816).  Same outputs as the general path.  P edges per
+// thread, placed 1,024 at a time.  Latency-bound (one workgroup's barriers and LDS round trips), four
+// launches -> one at 4,097 chapters: 1,040 edges 27.6 -> 5.5-7.3 us, 4,816 29.2 -> 11.9, 8,192 29.5 ->
+// 14.4.  The limit is what one workgroup's LDS holds beside 8,192 chapters' counts.
+constexpr int kPlanSmallP = 8;
 constexpr int kPlanSmallE = 1024 * kPlanSmallP;
 constexpr int kPlanSmallC = 8192;
 
@@ -269,7 +270,9 @@ __global__ __launch_bounds__(1024) void plan_small_kernel(const int32_t* __restr
   __syncthreads();
   // placement into the chapter's segment in arrival order, then the stable order: an edge's slot is
   // the segment start plus the edges of earlier blocks of 1,024 plus those of its own block with a
-  // smaller id
+  // smaller id, counted one by one, or, when a chapter has many of a block (every sequence on one
+  // chapter; with more than one block), from the edge's rank among its wave's and the waves' counts
+  // taken in order (4,096 edges of one chapter: 180 us counted, 31 so, 207 in the four launches)
 #pragma unroll
   for (int p = 0; p < P; ++p) {
     const int e = 1024 * p + tid;
@@ -282,14 +285,32 @@ __global__ __launch_bounds__(1024) void plan_small_kernel(const int32_t* __restr
     }
     if (ok) tmp[cnt[c] + atomicAdd(&fill[c], 1)] = e;
     __syncthreads();
+    const int n = ok ? fill[c] : 0;
+    int before = n0;
+    if (P > 1 && __syncthreads_or(n - n0 > 64)) {
+      int rank = 0, same = 0;   // among the wave's edges of the chapter: those before this one, all
+      for (int l = 0; l < 64; ++l) {
+        const bool eq = __shfl(c, l, 64) == c;
+        rank += eq && l < lane;
+        same += eq;
+      }
+      if (ok) fill[c] = n0;
+      for (int w = 0; w < 16; ++w) {
+        __syncthreads();
+        if (wave == w && ok) {
+          const int base = fill[c];
+          before = base + rank;
+          if (rank == 0) fill[c] = base + same;
+        }
+      }
+      __syncthreads();
+    } else if (ok) {
+      const int s0 = cnt[c];
+      for (int j = n0; j < n; ++j) before += tmp[s0 + j] < e;
+    }
     if (e < E) {
       edge_u[e] = ok ? uid[c] : -1;
-      if (ok) {
-        const int s0 = cnt[c], n = fill[c];
-        int before = n0;
-        for (int j = n0; j < n; ++j) before += tmp[s0 + j] < e;
-        csr_edge[s0 + before] = e;
-      }
+      if (ok) csr_edge[cnt[c] + before] = e;
     }
   }
 }
@@ -334,6 +355,9 @@ int plan_launch(const int32_t* chap, int64_t E, int64_t C, void* workspace, int3
     const size_t lds = 3 * (size_t)C * sizeof(int32_t);
     if (E <= 1024)
       hipLaunchKernelGGL(plan_small_kernel<1>, dim3(1), dim3(1024), lds, stream, chap, E, C, uniq, n_uniq, edge_u,
+                         csr_off, csr_edge);
+    else if (E <= 4096)
+      hipLaunchKernelGGL(plan_small_kernel<4>, dim3(1), dim3(1024), lds, stream, chap, E, C, uniq, n_uniq, edge_u,
                          csr_off, csr_edge);
     else
       hipLaunchKernelGGL(plan_small_kernel<kPlanSmallP>, dim3(1), dim3(1024), lds, stream, chap, E, C, uniq, n_uniq,

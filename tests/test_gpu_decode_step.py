@@ -12,13 +12,15 @@ BF = torch.bfloat16
 
 
 @pytest.mark.parametrize("E,C", [(1023, 700), (1024, 33), (1025, 1), (2048, 8192), (2049, 300), (4095, 4097), (4096, 8),
-                                 (4097, 50)])
+                                 (4097, 50), (8191, 8192), (8192, 900), (8193, 60)])
 def test_small_plan(gpu_device, E, C):
     from memory_amd import ops
     ids = torch.randint(0, C, (E,), generator=gen(E + C), dtype=torch.int32)
     ids[::7] = -1
     ids[3::11] = C
     ids[E // 2:E // 2 + 40] = C // 2
+    if E % 1024 != 1:
+        ids[E // 3:E - 5:2] = C // 3      # one chapter with most of several blocks
     a = ids.numpy()
     ok = (a >= 0) & (a < C)
     uniq = np.unique(a[ok])
