@@ -146,6 +146,34 @@ __global__ __launch_bounds__(kFwdThreads) void xattn_fwd_kernel(
     }
   };
 
+  // S^T[kb][qb]: rows = keys 16*kb + 4*g + e, column = query c16 of block qb
+  auto scores = [&](const char* Ks, f32x4 (&st)[4][2]) {
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+      for (int qb = 0; qb < 2; ++qb) st[kb][qb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb) {
+        F8 a = Tile::frag(Ks, 16 * kb + c16, 32 * ks + 8 * g);
+#pragma unroll
+        for (int qb = 0; qb < 2; ++qb) mma(st[kb][qb], a, qf[qb][ks]);
+      }
+    }
+  };
+  // a row's maximum over the chapter (three-input max chains)
+  auto row_max = [&](const f32x4 (&st)[4][2], int qb) {
+    float mx = max3f(st[0][qb][0], st[0][qb][1], st[0][qb][2]);
+    mx = max3f(mx, st[0][qb][3], st[1][qb][0]);
+    mx = max3f(mx, st[1][qb][1], st[1][qb][2]);
+    mx = max3f(mx, st[1][qb][3], st[2][qb][0]);
+    mx = max3f(mx, st[2][qb][1], st[2][qb][2]);
+    mx = max3f(mx, st[2][qb][3], st[3][qb][0]);
+    mx = max3f(mx, st[3][qb][1], st[3][qb][2]);
+    return quad_max_pl(fmax_fast(mx, st[3][qb][3]));
+  };
+
   int u_cur = su[s_begin];
   if (u_cur >= 0) {
     fetch(u_cur, s_begin & 1);
@@ -154,11 +182,39 @@ __global__ __launch_bounds__(kFwdThreads) void xattn_fwd_kernel(
       vio.store(sV[s_begin & 1], tid);
     }
   }
+  // A later split starts from the maximum over the row's first used chapter, as the unsplit loop does:
+  // bf16 rounds P~ = 2^(logit - m) to 8 bits, and where a chapter's P~ falls in their binade, hence each
+  // one's rounding, goes with m.  With one m the splits round every P~ as the unsplit kernel (until a
+  // maximum grows by more than kRescaleSlack) and differ from it by f32 sums only; each with its own
+  // first maximum, single prompts came out with up to 1.03 times its error.
+  int s_first = s_begin;
+  if constexpr (SPLIT && kDma) {
+    s_first = 0;
+    while (s_first < s_begin && su[s_first] < 0) ++s_first;
+    s_first = __builtin_amdgcn_readfirstlane(s_first);   // the DMA's offset is a scalar operand
+    if (s_first < s_begin) {
+      const uint32_t so = tile_off(su[s_first]);
+      fwd_dma16(kb.r, dma_v0, sK[(s_begin & 1) ^ 1] + 2048 * wave, so);
+      fwd_dma16(kb.r, dma_v0 + 8 * row_bytes, sK[(s_begin & 1) ^ 1] + 2048 * wave + 1024, so);
+    }
+  }
   // Q fragments must have landed before the loop on every path (also when slot 0
   // is skipped); otherwise the wait for them inside the loop can't be told apart
   // from the prefetch and becomes a full vmcnt(0) ahead of the first MFMA.
   vm_wait_all();
   __syncthreads();
+  if constexpr (SPLIT && kDma) {
+    if (s_first < s_begin) {
+      f32x4 st[4][2];
+      scores(sK[(s_begin & 1) ^ 1], st);
+#pragma unroll
+      for (int qb = 0; qb < 2; ++qb) {
+        const float cm = row_max(st, qb) * (om[s_first] * scale_log2);
+        m[qb] = cm > m[qb] + kRescaleSlack ? cm : m[qb];
+      }
+      __syncthreads();   // the loop's first fetch overwrites this tile
+    }
+  }
 
   for (int s = s_begin; s < s_end; ++s) {
     const int buf = s & 1;
@@ -170,40 +226,19 @@ __global__ __launch_bounds__(kFwdThreads) void xattn_fwd_kernel(
       const float c = w * scale_log2;
       const char* Ks = sK[buf];
       const char* Vs = sV[buf];
-      // S^T[kb][qb]: rows = keys 16*kb + 4*g + e, column = query c16 of block qb
       f32x4 st[4][2];
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb)
-#pragma unroll
-        for (int qb = 0; qb < 2; ++qb) st[kb][qb] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks) {
-#pragma unroll
-        for (int kb = 0; kb < 4; ++kb) {
-          F8 a = Tile::frag(Ks, 16 * kb + c16, 32 * ks + 8 * g);
-#pragma unroll
-          for (int qb = 0; qb < 2; ++qb) mma(st[kb][qb], a, qf[qb][ks]);
-        }
-      }
+      scores(Ks, st);
       // the previous chapter's row sums (their MFMA has long completed): folded in before any
       // rescale, in units of the reference max they were taken against
 #pragma unroll
       for (int qb = 0; qb < 2; ++qb) lsum[qb] += pend_ls[qb] * pend_rw;
       pend_rw = 0.f;
-      // chapter max per row (three-input max chains), lazy update of the reference max
+      // chapter max per row, lazy update of the reference max
       float cm[2];
       bool grow = false;
 #pragma unroll
       for (int qb = 0; qb < 2; ++qb) {
-        float mx = max3f(st[0][qb][0], st[0][qb][1], st[0][qb][2]);
-        mx = max3f(mx, st[0][qb][3], st[1][qb][0]);
-        mx = max3f(mx, st[1][qb][1], st[1][qb][2]);
-        mx = max3f(mx, st[1][qb][3], st[2][qb][0]);
-        mx = max3f(mx, st[2][qb][1], st[2][qb][2]);
-        mx = max3f(mx, st[2][qb][3], st[3][qb][0]);
-        mx = max3f(mx, st[3][qb][1], st[3][qb][2]);
-        mx = fmax_fast(mx, st[3][qb][3]);
-        cm[qb] = quad_max_pl(mx) * c;  // c >= 0 (router weights are non-negative)
+        cm[qb] = row_max(st, qb) * c;  // c >= 0 (router weights are non-negative)
         grow |= cm[qb] > m[qb] + kRescaleSlack;
       }
       if (__any(grow)) {
