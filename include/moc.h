@@ -673,6 +673,11 @@ int moc_sparse_packed_bwd(int dtype, const void* q, const void* dout, int64_t nt
                           const int32_t* csr_off, const int32_t* csr_edge, int64_t max_u, int S, int mode,
                           const float* lse_row, float* delta_row, const float* w, float scale, void* dk, void* dv,
                           void* dq_part, float* dlog, void* workspace, size_t workspace_bytes, hipStream_t stream);
+/* Joint modes 2 / 3: dlog [E][rpe] with the error of delta taken out.  The gradients of the log weights of a
+ * row's valid slots add up to zero; what they add up to is shared out by the slots' probabilities
+ * w 2^lse_part / 2^lse_joint.  In place, before moc_sparse_dw. */
+int moc_sparse_dlog_center(float* dlog, const float* lse_part, const float* lse_joint, const float* w,
+                           const int32_t* edge_u, int mode, int S, int rpe, int64_t ntok, hipStream_t stream);
 /* Zeros the (chapter, kv head) blocks of dK / dV (element (t, dh) at c*cs + hk*hs + t*rs + dh,
  * heads hk0 .. hk0+nhk-1, C chapters) whose chapter is not among the plan's uniq[0 .. n_uniq):
  * moc_sparse_bwd writes every block it touches whole, so this replaces zero-initialising the

@@ -133,6 +133,7 @@ _SIGS = {
     "moc_sparse_packed_bwd_workspace": (_SZ, [_I, _I64, _I, _I, _I, _I64, _F]),
     "moc_sparse_packed_bwd": (_I, [_I, _P, _P, _I64, _I, _P, _P, _I64, _I64, _I, _I, _P, _P, _P, _P, _I64, _I, _I, _P,
                                    _P, _P, _F, _P, _P, _P, _P, _P, _SZ, _P]),
+    "moc_sparse_dlog_center": (_I, [_P, _P, _P, _P, _P, _I, _I, _I, _I64, _P]),
     "moc_sparse_zero_untouched": (_I, [_I, _P, _P, _I64, _I64, _I64, _I64, _I, _I, _P, _P, _I64, _P, _P]),
     "moc_decode_partial": (_I, [_I, _P, _I64, _I, _P, _P, _I, _I, _I, _P, _P, _P, _P, _I64, _P, _I, _F, _P, _P, _P,
                                 _P]),

@@ -146,34 +146,58 @@ __global__ __launch_bounds__(256) void sparse_rows_fwd_kernel(
       mma(st[kb], kf[kb][0], qf[0]);
       mma(st[kb], kf[kb][1], qf[1]);
     }
+    // 64 keys at a time, each with its own maximum: bf16 rounds P = 2^(s - max) to 8 bits, exactly for
+    // the maximum's own key alone, so one maximum over 128 keys put 128-key units at 1.018 times the
+    // error of 64-key ones (outputs, 8 blocks of 128; 1.001 so, the one rounding of a partial row in
+    // place of two).  The halves are scaled to each other in f32: 590 -> 598 us for the call above,
+    // forward and backward.  (Row sums of the rounded P on the matrix cores: 613 us, and dK / dV
+    // 1.0006 times as far off.)
     if (KT > 64 && un.nk < KT) {   // a half last block: its missing keys take no part
 #pragma unroll
       for (int kb = 4; kb < NKB; ++kb) st[kb] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
     }
-    float mx = st[0][0];
-#pragma unroll
-    for (int kb = 0; kb < NKB; ++kb)
-#pragma unroll
-      for (int x = 0; x < 4; ++x) mx = fmax_fast(mx, st[kb][x]);
-    const float m = quad_max(mx) * scale_log2;   // scale > 0 (host check)
-    float ps = 0.f;
-    bf16x8 pf[KT / 32];
-#pragma unroll
-    for (int kb = 0; kb < NKB; ++kb)
-#pragma unroll
-      for (int x = 0; x < 4; ++x) {
-        const float p = sr_exp2(st[kb][x] * scale_log2 - m);
-        ps += p;
-        pf[kb >> 1][4 * (kb & 1) + x] = (bf16)p;
-      }
-    const float l = quad_sum(ps);
+    float m = -INFINITY, l = 0.f;
     f32x4 o[4];
 #pragma unroll
-    for (int db = 0; db < 4; ++db) o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int h = 0; h < KT / 64; ++h) {
+      float mx = st[4 * h][0];
 #pragma unroll
-    for (int ks = 0; ks < KT / 32; ++ks)
+      for (int kb = 4 * h; kb < 4 * h + 4; ++kb)
 #pragma unroll
-      for (int db = 0; db < 4; ++db) mma(o[db], tr_frag_mk<Tile>(sV, 32 * ks, 16 * db, lane), pf[ks]);
+        for (int x = 0; x < 4; ++x) mx = fmax_fast(mx, st[kb][x]);
+      const float mh = quad_max(mx) * scale_log2;   // scale > 0 (host check)
+      const float ref = mh > -INFINITY || KT == 64 ? mh : 0.f;   // a half of -inf scores adds nothing
+      float ps = 0.f;
+      bf16x8 pf[2];
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          const float p = sr_exp2(st[4 * h + kb][x] * scale_log2 - ref);
+          ps += p;
+          pf[kb >> 1][4 * (kb & 1) + x] = (bf16)p;
+        }
+      const float lh = quad_sum(ps);
+      f32x4 oh[4];
+#pragma unroll
+      for (int db = 0; db < 4; ++db) oh[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int db = 0; db < 4; ++db) mma(oh[db], tr_frag_mk<Tile>(sV, 64 * h + 32 * ks, 16 * db, lane), pf[ks]);
+      if (h == 0) {
+        m = mh;
+        l = lh;
+#pragma unroll
+        for (int db = 0; db < 4; ++db) o[db] = oh[db];
+      } else {
+        const float mn = fmaxf(m, mh), fa = sr_exp2(m - mn), fb = sr_exp2(mh - mn);
+        m = mn;
+        l = l * fa + lh * fb;
+#pragma unroll
+        for (int db = 0; db < 4; ++db) o[db] = o[db] * fa + oh[db] * fb;
+      }
+    }
     // dims 16 db + 4 g .. + 3 of two db in one lane -> dims 16 db + 8 (g / 2) .. + 7 of one: the
     // odd 16-lane groups' db = 2 j against the even groups' db = 2 j + 1
     const float inv = 1.f / l;
@@ -600,6 +624,30 @@ __global__ __launch_bounds__(256) void sparse_pack_ids_kernel(const I* __restric
   out[i] = c >= 0 && c < nblk ? (int32_t)((b * nblk + c) * HK + hk) : -1;
 }
 
+// dlog[e, r] -= P_e sum_e' dlog[e', r] over the valid slots of a (token, row), P_e = w_e 2^lse_e / 2^lse_joint:
+// the joint softmax's log-weight gradients P_e (dP_e - D) add up to zero, and what they add up to is the
+// error of D = dO . out, whose out is rounded to bf16.  That error was all of dw's (1.13e-3 in bf16 over 8
+// blocks of 128 keys, a token with one valid block moved by 0.8 where the largest dw is 27; 3e-7 now), and
+// 128-key units' roundings of out put it at 1.02 to 1.05 times that of 64-key ones.  Thread = (token, row).
+__global__ __launch_bounds__(256) void sparse_dlog_center_kernel(float* __restrict__ dlog,
+                                                                 const float* __restrict__ lse_part,
+                                                                 const float* __restrict__ lse_joint,
+                                                                 const float* __restrict__ w,
+                                                                 const int32_t* __restrict__ edge_u, int mode, int S,
+                                                                 int rpe, int64_t rows) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= rows) return;
+  const int64_t tok = i / rpe, r = i - tok * rpe;
+  float sum = 0.f;
+  for (int s = 0; s < S; ++s)
+    if (edge_u[tok * S + s] >= 0) sum += dlog[(tok * S + s) * rpe + r];
+  const float lj = lse_joint[i];
+  for (int s = 0; s < S; ++s) {
+    const int64_t e = tok * S + s, at = e * rpe + r;
+    if (edge_u[e] >= 0) dlog[at] -= sr_exp2(lse_part[at] + sr_logw(mode, w[e]) - lj) * sum;
+  }
+}
+
 }  // namespace moc
 
 using namespace moc;
@@ -782,6 +830,18 @@ int moc_sparse_packed_bwd(int dtype, const void* q, const void* dout, int64_t nt
   if (KT == 64) SR_RED(64); else SR_RED(128);
 #undef SR_RED
   return check_launch("sparse_rows_reduce_kernel");
+}
+
+int moc_sparse_dlog_center(float* dlog, const float* lse_part, const float* lse_joint, const float* w,
+                           const int32_t* edge_u, int mode, int S, int rpe, int64_t ntok, hipStream_t stream) {
+  MOC_REQUIRE(dlog && lse_part && lse_joint && w && edge_u, MOC_ERR_ARG, "moc_sparse_dlog_center: null pointer");
+  MOC_REQUIRE((mode == 2 || mode == 3) && S > 0 && rpe > 0 && ntok >= 0 && ntok * rpe < ((int64_t)1 << 38), MOC_ERR_ARG,
+              "moc_sparse_dlog_center: mode %d, S=%d, %d rows of %lld tokens", mode, S, rpe, (long long)ntok);
+  if (ntok == 0) return MOC_OK;
+  const int64_t rows = ntok * rpe;
+  hipLaunchKernelGGL(sparse_dlog_center_kernel, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, stream, dlog, lse_part,
+                     lse_joint, w, edge_u, mode, S, rpe, rows);
+  return check_launch("sparse_dlog_center_kernel");
 }
 
 }  // extern "C"

@@ -270,13 +270,14 @@ class _PackedFSA(torch.autograd.Function):
         lse_joint = None if mode == 0 else torch.empty(ntok * G, device=dev, dtype=torch.float32)
         call("moc_sparse_combine", dt, ptr(o_part), ptr(lse_part), ptr(plan.edge_u), ptr(wf), mode, S, G, ntok, G, 0,
              ptr(out), ptr(lse_joint), st)
-        ctx.save_for_backward(q, k, v, out, wf, lse_part if mode == 0 else lse_joint)
+        center = lse_part if kt == 128 and mode in (2, 3) and ctx.needs_input_grad[3] else None
+        ctx.save_for_backward(q, k, v, out, wf, lse_part if mode == 0 else lse_joint, center)
         ctx.plan, ctx.cfg = plan, (mode, scale, kt, S, None if w is None else w.dim(), None if w is None else w.dtype)
         return out
 
     @staticmethod
     def backward(ctx, dout):
-        q, k, v, out, wf, lrow = ctx.saved_tensors
+        q, k, v, out, wf, lrow, center = ctx.saved_tensors
         mode, scale, kt, S, wdim, wdt = ctx.cfg
         plan = ctx.plan
         B, Tq, HQ, D = q.shape
@@ -303,6 +304,9 @@ class _PackedFSA(torch.autograd.Function):
         call("moc_sparse_dq_combine", dt, ptr(dq_part), ptr(plan.edge_u), S, G, ntok, G, 0, ptr(dq), st)
         dw = None
         if mode != 1:
+            if center is not None:
+                call("moc_sparse_dlog_center", ptr(dlog), ptr(center), ptr(lrow), ptr(wf), ptr(plan.edge_u), mode, S, G,
+                     ntok, st)
             dw = torch.empty(B, Tq, HK, S, device=dev, dtype=torch.float32)
             call("moc_sparse_dw", ptr(drow if mode == 0 else dlog), ptr(wf), ptr(plan.edge_u), mode, G, ntok * S,
                  ptr(dw), st)

@@ -118,3 +118,76 @@ def test_packed_scale_signs(gpu_device, scale):
     seg = SA._FSAFunction.apply(q, k, v, None, (idx.unsqueeze(-1) * 2 + torch.arange(2, device=dev)).flatten(-2).int(), 1,
                                 scale)
     assert_parity(out, seg, torch.bfloat16, f"scale {scale}")
+
+
+@pytest.mark.parametrize("S,Tk", [(8, 2048), (3, 1088)])
+def test_128_key_units_round_as_64_key_ones(gpu_device, S, Tk):
+    """Outputs of 128-key units are no further from float64 than those of the same blocks as 64-key units
+    (the segments): one maximum, and so one exact P, per 64 keys.  The ratio of the two errors over N =
+    65,536 rows is a ratio of mean squares of at least 4 N independent terms (the roundings of a row's P
+    and partial rows): 1 within 4 sqrt(2 / 4 N) / 2 = 0.0055; one maximum per 128 keys puts it at 1.018."""
+    from memory_amd import sparse_attention as SA
+    dev = gpu_device
+    g = gen(S)
+    Tq, HQ = 4096, 16
+    q, k, v = (torch.randn(1, n, h, 64, generator=g).to(dev, torch.bfloat16) for n, h in ((Tq, HQ), (Tk, 1), (Tk, 1)))
+    idx = torch.rand(1, Tq, 1, -(-Tk // 128), generator=g).argsort(-1)[..., :S]
+    assert SA._packed_block(q, k, v, None, idx.to(dev), 1, 0.125, 128) == 128
+    out = SA.FSA_topk_sparse_attention_bthd(q, k, v, idx.to(dev, torch.int32), 128, disable_causal_mask=True)
+    sub = (idx.unsqueeze(-1) * 2 + torch.arange(2)).flatten(-2).to(dev, torch.int32)
+    seg = SA._FSAFunction.apply(q, k, v, None, sub, 1, 0.125)
+    ref = torch.cat([_reference(q[:, a:a + 256].double().cpu(), k.double().cpu(), v.double().cpu(), idx[:, a:a + 256], None,
+                                1, 128, 0.125) for a in range(0, Tq, 256)], 1)
+    err, base = ((t.double().cpu() - ref).norm().item() for t in (out, seg))
+    print(f"S={S} Tk={Tk}: error ratio {err / base:.4f}", flush=True)
+    assert err <= 1.0055 * base
+
+
+@pytest.mark.parametrize("mode", [2, 3])
+def test_128_key_units_block_weight_gradient(gpu_device, mode):
+    """The block weights' gradient of 128-key units is free of the output's bf16 rounding: products of exact
+    bf16 operands and float32 sums over 128 keys of 64 dims, P and lse to a few units of 2^-23, divided by
+    the weight: below 1e-5 of the largest value here (2^-23 times the ~30 for the cancelling sum of a
+    token's slots), against 1e-2 with the error of dO . out left in."""
+    from memory_amd import sparse_attention as SA
+    dev = gpu_device
+    g = gen(90 + mode)
+    Tq, HQ, Tk, S = 400, 8, 448, 3
+    q, dO = (torch.randn(1, Tq, HQ, 64, generator=g).bfloat16() for _ in range(2))
+    k, v = (torch.randn(1, Tk, 2, 64, generator=g).bfloat16() for _ in range(2))
+    idx = torch.rand(1, Tq, 2, 4, generator=g).argsort(-1)[..., :S]
+    idx[:, ::5, :, 0] = -1
+    idx[:, ::10, :, 1] = 4                        # one valid block: no gradient at all
+    idx[:, 7] = -1                                # none
+    w = torch.softmax(torch.randn(1, Tq, 2, S, generator=g), -1)
+    if mode == 2:
+        w[:, 11, :, 0] = 0.0
+    rw = w.double().requires_grad_(True)
+    ref = _reference(q.double(), k.double(), v.double(), idx, rw, mode, 128, 0.125)
+    (ref * dO.double()).sum().backward()
+    fn = (SA.FSA_topk_sparse_attention_weighted_joint_bias_bthd if mode == 3 else
+          lambda a, b, c, i, x, n, **kw: SA.FSA_topk_sparse_attention_bthd(a, b, c, i, n, block_weights_bths=x, **kw))
+    tw = w.to(dev).requires_grad_(True)
+    assert SA._packed_block(q.to(dev), k.to(dev), v.to(dev), tw, idx.to(dev), mode, 0.125, 128) == 128
+    fn(q.to(dev), k.to(dev), v.to(dev), idx.to(dev, torch.int32), tw, 128, disable_causal_mask=True).backward(dO.to(dev))
+    got, want = tw.grad.double().cpu(), rw.grad
+    if mode == 2:                                 # the gradient at a weight of zero is the clamp's: none here
+        got, want = (torch.where(w > 0, t, 0.0) for t in (got, want))
+    assert ((got - want).abs().max() / want.abs().max()).item() <= 1e-5
+
+
+def test_128_key_unit_with_a_half_of_infinite_scores(gpu_device):
+    """Keys whose scores are -inf (here a whole half of a block) take no part, as in a softmax over the
+    block."""
+    from memory_amd import sparse_attention as SA
+    dev = gpu_device
+    g = gen(5)
+    q = (torch.rand(1, 200, 4, 64, generator=g) + 0.1).to(dev, torch.bfloat16)
+    k, v = (torch.randn(1, 256, 1, 64, generator=g).to(dev, torch.bfloat16) for _ in range(2))
+    k[:, 64:128, :, 0] = -float("inf")
+    k[:, 128:192, :, 0] = -float("inf")
+    idx = torch.zeros(1, 200, 1, 2, dtype=torch.int32, device=dev)
+    idx[..., 1] = 1
+    out = SA.FSA_topk_sparse_attention_bthd(q, k, v, idx, 128, disable_causal_mask=True)
+    s = torch.einsum("thd,jd->thj", q[0].double(), k[0, :, 0].double().nan_to_num(neginf=-1e300)) * 0.125
+    assert_parity(out[0], torch.softmax(s, -1) @ v[0, :, 0].double(), torch.bfloat16, "out")
