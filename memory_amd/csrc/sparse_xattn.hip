@@ -442,6 +442,26 @@ __device__ __forceinline__ void sp_chunk_store(T* __restrict__ row, const float 
   *reinterpret_cast<typename SpRow16<T>::V*>(row + SpRow16<T>::EPL * ch) = o;
 }
 
+// float32: acc = sum_i a_i v_i in the order of the one-wave-per-row kernels above (lane group i % NG takes
+// slots i and i + NG, the groups pairwise): the same bits, where a running sum put float32 outputs and dQ
+// at up to 1.004 times their error.  a_i = 0 marks a slot that is not to be read.  (bf16 rows carry
+// roundings of 2^-9 in which the order of float32 sums does not show: a running sum, 64.4 us for 262,144
+// rows, 68 pairwise.)
+__device__ __forceinline__ void sp_few_sum(const f32x4 (&v)[kCombFew], const float (&a)[kCombFew], float (&acc)[4]) {
+  constexpr int NG = SpRow16<float>::NG;
+  static_assert(kCombFew == 8 && NG == 4, "pairwise order");
+#pragma unroll
+  for (int x = 0; x < 4; ++x) {
+    float p[NG];
+#pragma unroll
+    for (int i = 0; i < kCombFew; ++i) {
+      const float t = a[i] != 0.f ? v[i][x] : 0.f;
+      p[i % NG] = __builtin_fmaf(a[i], t, i < NG ? 0.f : p[i % NG]);   // (no a v + a' v' in one rounding)
+    }
+    acc[x] = (p[0] + p[1]) + (p[2] + p[3]);
+  }
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void sparse_combine_few_kernel(
     const T* __restrict__ o_part, const float* __restrict__ lse_part, const int32_t* __restrict__ edge_u,
@@ -473,15 +493,23 @@ __global__ __launch_bounds__(256) void sparse_combine_few_kernel(
 #pragma unroll
   for (int i = 0; i < kCombFew; ++i) M = fmaxf(M, lg[i]);
   float den = 0.f, acc[R::EPL];
+  if constexpr (sizeof(T) == 4) {
+    float a[kCombFew];
 #pragma unroll
-  for (int x = 0; x < R::EPL; ++x) acc[x] = 0.f;
+    for (int i = 0; i < kCombFew; ++i) a[i] = !ok[i] ? 0.f : mode == 0 ? lg[i] : M > -INFINITY ? exp2f(lg[i] - M) : 0.f;
+    den = ((a[0] + a[4]) + (a[2] + a[6])) + ((a[1] + a[5]) + (a[3] + a[7]));
+    sp_few_sum(v, a, acc);
+  } else {
 #pragma unroll
-  for (int i = 0; i < kCombFew; ++i) {
-    const float a = !ok[i] ? 0.f : mode == 0 ? lg[i] : M > -INFINITY ? exp2f(lg[i] - M) : 0.f;
-    den += a;
-    if (a != 0.f) {
+    for (int x = 0; x < R::EPL; ++x) acc[x] = 0.f;
 #pragma unroll
-      for (int x = 0; x < R::EPL; ++x) acc[x] += a * (float)v[i][x];
+    for (int i = 0; i < kCombFew; ++i) {
+      const float a = !ok[i] ? 0.f : mode == 0 ? lg[i] : M > -INFINITY ? exp2f(lg[i] - M) : 0.f;
+      den += a;
+      if (a != 0.f) {
+#pragma unroll
+        for (int x = 0; x < R::EPL; ++x) acc[x] += a * (float)v[i][x];
+      }
     }
   }
   float inv = 1.f;
@@ -881,14 +909,21 @@ __global__ __launch_bounds__(256) void sparse_dq_combine_few_kernel(const T* __r
     eu[i] = in ? edge_u[e] : -1;
   }
   float acc[R::EPL];
+  if constexpr (sizeof(T) == 4) {
+    float a[kCombFew];
 #pragma unroll
-  for (int x = 0; x < R::EPL; ++x) acc[x] = 0.f;
+    for (int i = 0; i < kCombFew; ++i) a[i] = eu[i] >= 0 ? 1.f : 0.f;
+    sp_few_sum(v, a, acc);
+  } else {
 #pragma unroll
-  for (int i = 0; i < kCombFew; ++i)
-    if (eu[i] >= 0) {
+    for (int x = 0; x < R::EPL; ++x) acc[x] = 0.f;
 #pragma unroll
-      for (int x = 0; x < R::EPL; ++x) acc[x] += (float)v[i][x];
-    }
+    for (int i = 0; i < kCombFew; ++i)
+      if (eu[i] >= 0) {
+#pragma unroll
+        for (int x = 0; x < R::EPL; ++x) acc[x] += (float)v[i][x];
+      }
+  }
   sp_chunk_store(dq + (tok * HQ + hq_off + r) * kSpDh, acc, 1.f, ch);
 }
 

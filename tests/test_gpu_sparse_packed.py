@@ -191,3 +191,45 @@ def test_128_key_unit_with_a_half_of_infinite_scores(gpu_device):
     out = SA.FSA_topk_sparse_attention_bthd(q, k, v, idx, 128, disable_causal_mask=True)
     s = torch.einsum("thd,jd->thj", q[0].double(), k[0, :, 0].double().nan_to_num(neginf=-1e300)) * 0.125
     assert_parity(out[0], torch.softmax(s, -1) @ v[0, :, 0].double(), torch.bfloat16, "out")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("mode", [0, 1, 2, 3])
+@pytest.mark.parametrize("S", [1, 4, 5, 7, 8])
+def test_few_slot_combine_order(gpu_device, dtype, mode, S):
+    """The combines for at most 8 slots against the one-wave-per-row kernels, which take the same rows with
+    skipped slots up to 9: float32 adds in their order, to the same bits, and bf16 is apart by the order of
+    float32 sums (8 roundings of 2^-24: 2^-20 of the largest value, and in log2 for lse) and then one
+    rounding of its own (a step of at most 2^-7 of the value)."""
+    from memory_amd import _lib as lib
+    dev = gpu_device
+    g = gen(10 * S + mode)
+    ntok, rpe, S9 = 301, 3, 9
+    dt, st = lib.dtype_code(dtype), torch.cuda.current_stream().cuda_stream
+    part = torch.randn(ntok, S9, rpe, 64, generator=g).to(dtype)
+    lse = torch.randn(ntok, S9, rpe, generator=g) * 3
+    w = torch.rand(ntok, S9, generator=g)
+    edge = torch.zeros(ntok, S9, dtype=torch.int32)
+    edge[:, S:] = -1
+    edge[::5, 0] = -1
+    edge[7] = -1
+    part[edge.eq(-1).unsqueeze(-1).expand(ntok, S9, rpe)] = float("nan")     # never written by the kernels
+
+    def run(n):
+        p, l, ww, e = (t[:, :n].contiguous().to(dev) for t in (part, lse, w, edge))
+        out, dq = (torch.empty(ntok, rpe, 64, device=dev, dtype=dtype) for _ in range(2))
+        lj = torch.empty(ntok, rpe, device=dev)
+        lib.call("moc_sparse_combine", dt, p.data_ptr(), l.data_ptr(), e.data_ptr(), None if mode == 1 else ww.data_ptr(),
+                 mode, n, rpe, ntok, rpe, 0, out.data_ptr(), None if mode == 0 else lj.data_ptr(), st)
+        lib.call("moc_sparse_dq_combine", dt, p.data_ptr(), e.data_ptr(), n, rpe, ntok, rpe, 0, dq.data_ptr(), st)
+        return [out, dq] + ([] if mode == 0 else [lj])
+
+    for a, b in zip(run(S), run(S9)):
+        assert not torch.isnan(a).any()
+        if dtype == torch.float32:
+            assert torch.equal(a, b)
+            continue
+        a, b, step = a.double(), b.double(), 2.0 ** -7 if a.dtype == dtype else 0.0
+        a, b = (torch.where(torch.isinf(t), 1e9, t) for t in (a, b))
+        ok = torch.where(b < 1e9, b, 0.0).abs().max()
+        assert bool(((a - b).abs() <= step * b.abs() + 2.0 ** -20 * ok).all())
