@@ -18,6 +18,25 @@ from . import _lib as L
 from ._lib import call, ptr, stream_ptr
 
 
+def recorded_backward(fn, inputs, needs, grad_outputs):
+    """Gradients of fn(*inputs) for an autograd function's backward that is itself recorded (create_graph):
+    fn runs again on aliases of the inputs (so that a dependence of one input on another, outside of fn, is
+    left to the caller's graph) and is differentiated with its own operations on the graph.  ``needs``: which
+    inputs' gradients are wanted; None for the others and for inputs fn does not depend on."""
+    alias = [t if t is None else t.view_as(t) for t in inputs]
+    outputs = fn(*alias)
+    outputs = outputs if isinstance(outputs, tuple) else (outputs,)
+    pairs = [(o, g) for o, g in zip(outputs, grad_outputs) if g is not None and o.requires_grad]
+    wanted = [i for i, n in enumerate(needs) if n]
+    grads = [None] * len(inputs)
+    if pairs and wanted:
+        got = torch.autograd.grad([o for o, _ in pairs], [alias[i] for i in wanted], [g for _, g in pairs],
+                                  create_graph=True, allow_unused=True)
+        for i, g in zip(wanted, got):
+            grads[i] = g
+    return grads
+
+
 # --------------------------------------------------------------------------- router
 
 class _RouterPool(torch.autograd.Function):
@@ -223,6 +242,11 @@ def norm_code(norm_type: Optional[str]) -> int:
     if norm_type not in _NORM:
         raise ValueError(f"Unsupported norm_type: {norm_type}")
     return _NORM[norm_type]
+
+
+def norm_name(code: int) -> Optional[str]:
+    """The norm_type of a norm_code."""
+    return next(n for n, c in _NORM.items() if c == code)
 
 
 def row_stats(bank: torch.Tensor, plan: ChapterPlan, T: int, norm: int, eps: float):

@@ -287,7 +287,22 @@ def supported_f32(h, bank, wr, br, wq, wk, wv, wo, *, num_chapters: int, tokens_
                       ops.norm_code(norm_type)) is not None
 
 
+def _f32_per_op(h, bank, wr, br, wq, wk, wv, wo, *, coef, cfg):
+    """(out, logits) of the layer through the per-op autograd functions."""
+    C, T, S, k, scale, H, HK, norm, eps, _train = cfg
+    B, Lq, d = h.shape
+    logits = ops.router_linear(ops.router_pool(h, coef), wr, br)
+    idx_star, omega = ops.prepend_shared(*ops.router_topk(logits, k, S), S, scale)
+    q = ops.linear(h, wq).view(B, Lq, H, d // H)
+    a = ops.routed_attention(q, bank, wk, wv, omega, idx_star, num_chapters=C, tokens_per_chapter=T,
+                             norm_type=ops.norm_name(norm), eps=eps, num_kv_heads=HK)
+    return ops.linear(a.reshape(B, Lq, d), wo), logits
+
+
 class _SeqF32Layer(torch.autograd.Function):
+    """The float32 layer in one host call each way.  A recorded backward (create_graph) goes through the
+    per-op functions instead, whose products of the projections are recorded."""
+
     @staticmethod
     def forward(ctx, h, bank, wr, br, wq, wk, wv, wo, coef, cfg):
         C, T, S, k, scale, H, HK, norm, eps, train = cfg
@@ -307,13 +322,17 @@ class _SeqF32Layer(torch.autograd.Function):
         ctx.cfg = cfg
         ctx.set_materialize_grads(False)
         if train:
-            ctx.save_for_backward(h, bank, wr, wq, wk, wv, wo, cf, logits, idx, omega, saved)
+            ctx.save_for_backward(h, bank, wr, br, wq, wk, wv, wo, cf, logits, idx, omega, saved)
         ctx.mark_non_differentiable(idx, idx_star, omega)
         return out, logits, idx, idx_star, omega
 
     @staticmethod
     def backward(ctx, dout, dlogits, _didx, _didx_star, _domega):
-        h, bank, wr, wq, wk, wv, wo, cf, logits, idx, omega, saved = ctx.saved_tensors
+        h, bank, wr, br, wq, wk, wv, wo, cf, logits, idx, omega, saved = ctx.saved_tensors
+        if torch.is_grad_enabled():     # create_graph: the backward is itself differentiated
+            grads = ops.recorded_backward(functools.partial(_f32_per_op, coef=cf, cfg=ctx.cfg),
+                                          (h, bank, wr, br, wq, wk, wv, wo), ctx.needs_input_grad[:8], (dout, dlogits))
+            return (*grads, None, None)
         C, T, S, k, scale, H, HK, norm, eps, _train = ctx.cfg
         need_h, need_bank, need_wr, need_br, need_wq, need_wk, need_wv, need_wo = ctx.needs_input_grad[:8]
         dev = h.device

@@ -132,3 +132,62 @@ def test_f32_layer_stays_per_op(gpu_device, monkeypatch):
     layer.fused = False
     sum(layer(y, bank)[1].values()).backward()
     _same(x.grad, y.grad, "losses alone")
+
+
+@pytest.mark.parametrize("norm", ["none", "rms"])
+def test_f32_layer_recorded_backward(gpu_device, norm):
+    """A penalty on o_proj's weight gradient (create_graph), alone and added to another loss, against float64
+    autograd: the gradient is a recorded product of the attention's output, whose own derivative is the
+    attention's backward.  Gradients to 1e-4 of their largest value: two float32 chains of sums of up to 330
+    keys (2^-24 each, square-root growth below 1e-5) and the penalty's squares."""
+    import oracle as O
+    from memory_amd import seq_layer
+    dev = gpu_device
+    B, L, d, H, C, S, k = 2, 40, 128, 2, 9, 1, 4
+    layer = _layer(dev, d, H, H, C, S, k, norm)
+    g = gen(77)
+    h, up = torch.randn(B, L, d, generator=g), torch.randn(B, L, d, generator=g)
+    bank = torch.randn(C * 64, d, generator=g)
+    attn, r = layer.memory_attn, layer.router.router
+    params = [r.weight, r.bias, attn.q_proj.weight, attn.k_proj.weight, attn.v_proj.weight, attn.o_proj.weight]
+    leaves = [t.detach().double().cpu().requires_grad_() for t in (h, bank, *params)]
+    ref = O.sequence_memory_layer(*leaves, H=H, HK=H, C=C, T=64, S=S, top_k=k, routed_scale=2.5, normalize=norm != "none")
+    hd, bd = h.to(dev).requires_grad_(), bank.to(dev).requires_grad_()
+    assert seq_layer.supported_f32(hd, bd, *params, num_chapters=C, tokens_per_chapter=64, num_shared=S, top_k=k,
+                                   num_heads=H, num_kv_heads=H)
+    out = layer(hd, bd, return_losses=False)[0]
+    got_leaves = [hd, bd, *params]
+    for extra in (0.0, 0.5):
+        def penalty(out, up, wo):
+            gw, = torch.autograd.grad((out * up).sum(), wo, create_graph=True)
+            return (gw ** 2).sum() * 0.01 + extra * (out ** 2).sum()
+
+        want = torch.autograd.grad(penalty(ref, up.double(), leaves[-1]), leaves, retain_graph=True, allow_unused=True)
+        got = torch.autograd.grad(penalty(out, up.to(dev), params[-1]), got_leaves, retain_graph=True, allow_unused=True)
+        for n, a, b in zip(("h", "bank", "wr", "br", "wq", "wk", "wv", "wo"), got, want):
+            if n == "wo" and extra == 0.0:      # the weight's gradient does not depend on the weight
+                assert a is None or a.abs().max().item() <= 1e-6
+                continue
+            err = ((a.double().cpu() - b).abs().max() / b.abs().max()).item()
+            assert err <= 1e-4, (extra, n, err)
+
+
+def test_f32_layer_recorded_gradients_are_the_gradients(gpu_device):
+    """create_graph changes no first-order gradient, frozen inputs keep none, and one input may depend on
+    another."""
+    dev = gpu_device
+    layer = _layer(dev, 128, 2, 1, 9, 1, 3, "layernorm")
+    g = gen(6)
+    h = torch.randn(2, 33, 128, generator=g).to(dev)
+    bank = (torch.randn(9 * 64, 128, generator=g) * 0.1).to(dev)
+    layer.memory_attn.k_proj.weight.requires_grad_(False)
+
+    def grads(create_graph):
+        x = h.clone().requires_grad_()
+        b = (bank + x.mean() * 0.1)
+        out, losses = layer(x, b)
+        leaves = [x] + [p for p in layer.parameters() if p.requires_grad]
+        return torch.autograd.grad((out ** 2).sum() + sum(losses.values()), leaves, create_graph=create_graph)
+
+    for a, b in zip(grads(True), grads(False)):
+        _same(a, b, "gradient")
