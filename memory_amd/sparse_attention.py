@@ -241,10 +241,13 @@ class _PackedFSA(torch.autograd.Function):
     entry points): every (token, kv head) is a token of G query rows, every (batch, block of kt
     keys, kv head) an id of one plan, so all heads share each launch.
 
-    idx (B, Tq, >= HK, S) int32 / int64 block ids of kt keys; w (B, Tq, HK, S), (B, Tq, S) or None."""
+    idx (B, Tq, >= HK, S) int32 / int64 block ids of kt keys; w (B, Tq, HK, S), (B, Tq, S) or None.
+    A recorded backward (create_graph) of the per-block mixture over 128-key blocks goes through one joint
+    call per slot (_mixture), whose weighted sum is recorded."""
 
     @staticmethod
     def forward(ctx, q, k, v, w, idx, mode, scale, kt):
+        given = (q, k, v, w, idx) if mode == 0 and kt == 128 else (None,) * 5
         B, Tq, HQ, D = q.shape
         Bk, Tk, HK = k.shape[:3]
         G, S = HQ // HK, idx.shape[-1]
@@ -271,14 +274,24 @@ class _PackedFSA(torch.autograd.Function):
         call("moc_sparse_combine", dt, ptr(o_part), ptr(lse_part), ptr(plan.edge_u), ptr(wf), mode, S, G, ntok, G, 0,
              ptr(out), ptr(lse_joint), st)
         center = lse_part if kt == 128 and mode in (2, 3) and ctx.needs_input_grad[3] else None
-        ctx.save_for_backward(q, k, v, out, wf, lse_part if mode == 0 else lse_joint, center)
+        ctx.save_for_backward(q, k, v, out, wf, lse_part if mode == 0 else lse_joint, center, *given)
         ctx.plan, ctx.cfg = plan, (mode, scale, kt, S, None if w is None else w.dim(), None if w is None else w.dtype)
         return out
 
     @staticmethod
     def backward(ctx, dout):
-        q, k, v, out, wf, lrow, center = ctx.saved_tensors
+        q, k, v, out, wf, lrow, center, *given = ctx.saved_tensors
         mode, scale, kt, S, wdim, wdt = ctx.cfg
+        if given[0] is not None and torch.is_grad_enabled():
+            *given, idx = given
+            group = q.shape[2] // k.shape[2]
+
+            def mixture(q, k, v, w):
+                per_query_head = w.repeat_interleave(group, 2) if w.dim() == 4 else w
+                return _mixture(q, k, v, per_query_head, idx, scale, kt)
+
+            grads = ops.recorded_backward(mixture, given, ctx.needs_input_grad[:4], (dout,))
+            return (*grads, None, None, None, None)
         plan = ctx.plan
         B, Tq, HQ, D = q.shape
         Bk, Tk, HK = k.shape[:3]
@@ -468,14 +481,19 @@ def FSA_topk_sparse_attention_weighted_bthd(q_bthd, k_bthd, v_bthd, block_indice
         return out.to(q_bthd.dtype).reshape(q_bthd.shape)
     if m == 1 or _packed_block(q_bthd, k_bthd, v_bthd, w, idx, 0, scale, block_size):
         return _fsa(q_bthd, k_bthd, v_bthd, w, idx, 0, scale, block_size)
+    return _mixture(q_bthd, k_bthd, v_bthd, w, idx, scale, block_size)
+
+
+def _mixture(q, k, v, w, idx, scale: float, block_size: int):
+    """sum_s w_s softmax(q K_s^T) V_s with one joint call per slot."""
     out = None
     for sl in range(idx.shape[-1]):
-        o = _fsa(q_bthd, k_bthd, v_bthd, None, idx[..., sl:sl + 1], 1, scale, block_size)
+        o = _fsa(q, k, v, None, idx[..., sl:sl + 1], 1, scale, block_size)
         ws = w[..., sl]
         ws = ws.unsqueeze(-1).unsqueeze(-1) if ws.dim() == 2 else ws.unsqueeze(-1)   # (B, T[, H]) -> broadcast
         term = o.float() * ws.float()
         out = term if out is None else out + term
-    return out.to(q_bthd.dtype)
+    return out.to(q.dtype)
 
 
 def FSA_topk_sparse_attention_weighted_joint_bias_bthd(q_bthd, k_bthd, v_bthd, block_indices_bths,

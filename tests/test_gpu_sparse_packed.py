@@ -233,3 +233,32 @@ def test_few_slot_combine_order(gpu_device, dtype, mode, S):
         a, b = (torch.where(torch.isinf(t), 1e9, t) for t in (a, b))
         ok = torch.where(b < 1e9, b, 0.0).abs().max()
         assert bool(((a - b).abs() <= step * b.abs() + 2.0 ** -20 * ok).all())
+
+
+@pytest.mark.parametrize("HK,per_head", [(1, False), (2, True)])
+def test_mixture_recorded_backward(gpu_device, HK, per_head):
+    """A penalty on the block weights' gradient (create_graph) at 128-key blocks: the weights' gradient is a
+    recorded product of the slots' outputs, whose own derivative is the attention's backward; against float64
+    autograd, bf16 gate."""
+    from memory_amd import sparse_attention as SA
+    dev = gpu_device
+    g = gen(40 + HK)
+    B, Tq, HQ, Tk, S = 1, 130, 4, 512, 3
+    q, dO = (torch.randn(B, Tq, HQ, 64, generator=g).bfloat16() for _ in range(2))
+    k, v = (torch.randn(B, Tk, HK, 64, generator=g).bfloat16() for _ in range(2))
+    idx = torch.rand(B, Tq, HK, 4, generator=g).argsort(-1)[..., :S]
+    w = torch.rand(B, Tq, HK, S, generator=g) if per_head else torch.rand(B, Tq, S, generator=g)
+    t = [x.to(dev).requires_grad_() for x in (q, k, v, w)]
+    r = [x.double().requires_grad_() for x in (q, k, v, w)]
+    assert SA._packed_block(*t[:3], t[3], idx.to(dev), 0, 0.125, 128) == 128
+    out = SA.FSA_topk_sparse_attention_weighted_bthd(*t[:3], idx.to(dev, torch.int32), t[3], 128, disable_causal_mask=True)
+    ref = _reference(*r[:3], idx, r[3], 0, 128, 0.125)
+    first = torch.autograd.grad(out, t, dO.to(dev), retain_graph=True)
+    recorded = torch.autograd.grad(out, t, dO.to(dev), create_graph=True)
+    for n, a, b in zip("qkvw", recorded, first):
+        assert_parity(a, b, torch.bfloat16, f"d{n} recorded")
+    gw, = torch.autograd.grad((ref * dO.double()).sum(), r[3], create_graph=True)
+    want = torch.autograd.grad((gw ** 2).sum() * 0.01, r[:3])
+    got = torch.autograd.grad((recorded[3].float() ** 2).sum() * 0.01, t[:3])
+    for n, a, b in zip("qkv", got, want):
+        assert_parity(a, b, torch.bfloat16, f"penalty d{n}")
