@@ -262,3 +262,36 @@ def test_mixture_recorded_backward(gpu_device, HK, per_head):
     got = torch.autograd.grad((recorded[3].float() ** 2).sum() * 0.01, t[:3])
     for n, a, b in zip("qkv", got, want):
         assert_parity(a, b, torch.bfloat16, f"penalty d{n}")
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+def test_packed_float32_at_any_offset(gpu_device, mode):
+    """Contiguous float32 views one element into a buffer (4-byte boundary), upstream gradient too, give what
+    aligned operands give; bf16 ones are refused, as the segments refuse them."""
+    from memory_amd import sparse_attention as SA
+    dev = gpu_device
+    g = gen(60 + mode)
+    B, Tq, HQ, HK, Tk, S = 2, 37, 4, 2, 320, 2
+    q, dO = (torch.randn(B, Tq, HQ, 64, generator=g) for _ in range(2))
+    k, v = (torch.randn(B, Tk, HK, 64, generator=g) for _ in range(2))
+    idx = torch.rand(B, Tq, HK, 5, generator=g).argsort(-1)[..., :S].to(dev, torch.int32)
+    w = torch.rand(B, Tq, S, generator=g).to(dev)
+
+    def run(place, dtype=torch.float32):
+        t = [place(x.to(dev, dtype)).requires_grad_() for x in (q, k, v)]
+        if mode == 0:
+            out = SA.FSA_topk_sparse_attention_weighted_bthd(*t, idx, w, 64, disable_causal_mask=True)
+        else:
+            out = SA.FSA_topk_sparse_attention_bthd(*t, idx, 64, disable_causal_mask=True)
+        out.backward(place(dO.to(dev, dtype)))
+        return [out.detach()] + [x.grad for x in t]
+
+    def off(x):
+        flat = torch.empty(x.numel() + 1, device=dev, dtype=x.dtype)
+        flat[1:] = x.reshape(-1)
+        return flat[1:].view(x.shape)
+
+    for a, b in zip(run(off), run(lambda x: x)):
+        assert torch.equal(a, b)
+    with pytest.raises(ValueError, match="aligned"):
+        run(off, torch.bfloat16)
