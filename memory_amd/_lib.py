@@ -280,7 +280,10 @@ def query(name: str, *args):
 
 def stream_ptr(device: torch.device | None = None) -> int:
     """The current stream of `device` as the entry points take it, without building a Stream object per
-    launch (1.9 us of host time against 0.1; a layer's step makes up to some forty launches)."""
+    launch (1.9 us of host time against 0.1; a layer's step makes up to some forty launches).  A device
+    of another type is refused: the caller's pointers are host memory then."""
+    if device is not None and device.type != "cuda":
+        raise ValueError(f"expected a ROCm (cuda) device, got {device}: memory_amd has no CPU fallback")
     index = None if device is None else device.index
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 

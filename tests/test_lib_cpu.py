@@ -84,3 +84,15 @@ def test_seq_layer_stage_names(libpath):
     assert _lib.lib().moc_seq_layer_stage_name(len(names)) is None
     with pytest.raises(ValueError):
         _lib.seq_stage_timing(["no_such_stage"], 4)
+
+
+def test_cpu_tensors_are_refused_before_a_launch():
+    """Host pointers never reach a kernel: a launch's stream is that of a ROCm device, or the call is refused
+    (rows_linear has no other look at where its operands are)."""
+    import torch
+    from memory_amd import ops
+    with pytest.raises(ValueError, match="cpu"):
+        _lib.stream_ptr(torch.device("cpu"))
+    x, w = torch.zeros(4, 256, dtype=torch.bfloat16), torch.zeros(256, 256, dtype=torch.bfloat16)
+    with pytest.raises(ValueError, match="cpu"):
+        ops.rows_linear(x, w)
