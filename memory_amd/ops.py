@@ -362,7 +362,7 @@ def matmul2d(a: torch.Tensor, b: torch.Tensor, ta: bool = False, tb: bool = Fals
     """op(a) op(b) of 2-D tensors (ta / tb: transposed).  Small float32 products run on
     moc_gemm_f32; everything else on the library, autocast and a backward that is itself recorded
     (create_graph) included."""
-    if (a.dtype == torch.float32 and b.dtype == torch.float32 and a.is_cuda and b.is_cuda
+    if (a.dtype == torch.float32 and b.dtype == torch.float32 and a.is_cuda and a.device == b.device
             and not torch.is_autocast_enabled()
             and not (torch.is_grad_enabled() and (a.requires_grad or b.requires_grad))):
         K, M = a.shape if ta else a.shape[::-1]

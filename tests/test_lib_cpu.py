@@ -96,3 +96,20 @@ def test_cpu_tensors_are_refused_before_a_launch():
     x, w = torch.zeros(4, 256, dtype=torch.bfloat16), torch.zeros(256, 256, dtype=torch.bfloat16)
     with pytest.raises(ValueError, match="cpu"):
         ops.rows_linear(x, w)
+
+
+def test_products_across_devices_go_to_the_library(monkeypatch):
+    """Operands on two GPUs are the library's to refuse, never a kernel's pointers (stand-ins: no GPU here)."""
+    import types
+    import torch
+    from memory_amd import ops
+
+    def operand(index):
+        t = types.SimpleNamespace(dtype=torch.float32, is_cuda=True, device=torch.device("cuda", index), shape=(8, 8),
+                                  requires_grad=False, is_contiguous=lambda: True, data_ptr=lambda: 0)
+        t.t = lambda: t
+        return t
+
+    monkeypatch.setattr(ops, "call", lambda *a: pytest.fail("a kernel was called"))
+    monkeypatch.setattr(torch, "matmul", lambda a, b: "library")
+    assert ops.matmul2d(operand(0), operand(1)) == "library"
