@@ -134,11 +134,17 @@ def split_rows(x: torch.Tensor, n: int):
     return _SplitRows.apply(x, n)
 
 
-def _has_hooks(m: nn.Module) -> bool:
-    """Whether calling `m` would run anything beside its class's own forward."""
-    return bool(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
-                or "forward" in m.__dict__ or type(m) is not MemoryCrossAttention
-                or torch.nn.modules.module._has_any_global_hook())
+_ATTENTION_METHODS = frozenset(n for n, f in vars(MemoryCrossAttention).items() if callable(f))
+_ROUTER_METHODS = frozenset(n for n, f in vars(ChapterRouter).items() if callable(f))
+
+
+def _plain_modules(attn: nn.Module, router: nn.Module) -> bool:
+    """Whether calling `attn` and routing with `router` run their classes' own code and nothing beside it (no
+    subclass, no method replaced on the instance, no hooks)."""
+    return (type(attn) is MemoryCrossAttention and type(router) is ChapterRouter
+            and not (attn._forward_hooks or attn._forward_pre_hooks or attn._backward_hooks or attn._backward_pre_hooks)
+            and _ATTENTION_METHODS.isdisjoint(attn.__dict__) and _ROUTER_METHODS.isdisjoint(router.__dict__)
+            and not torch.nn.modules.module._has_any_global_hook())
 
 
 class RoutedMemoryLayer(nn.Module):
@@ -201,8 +207,8 @@ class RoutedMemoryLayer(nn.Module):
         norm_type = self.norm_type if normalize else None
         router = self.router.router
         if hidden_states.dtype == torch.float32:
-            # hooks on the attention module run where it is called
-            if _has_hooks(attn) or not seq_layer.supported_f32(
+            # hooks on the attention module run where it is called, a router of the caller's own is asked
+            if not _plain_modules(attn, self.router) or not seq_layer.supported_f32(
                     hidden_states, bank, router.weight, router.bias, attn.q_proj.weight, attn.k_proj.weight,
                     attn.v_proj.weight, attn.o_proj.weight, num_chapters=C, tokens_per_chapter=self.tokens_per_chapter,
                     num_shared=S, top_k=k, num_heads=attn.num_heads, num_kv_heads=attn.num_kv_heads,

@@ -191,3 +191,42 @@ def test_f32_layer_recorded_gradients_are_the_gradients(gpu_device):
 
     for a, b in zip(grads(True), grads(False)):
         _same(a, b, "gradient")
+
+
+def test_f32_layer_asks_the_callers_router(gpu_device):
+    """A router subclass, and router or attention methods replaced on the instance, are used as the per-op
+    path uses them."""
+    from memory_amd.router import ChapterRouter
+    dev = gpu_device
+    g = gen(8)
+    h, bank = torch.randn(2, 40, 128, generator=g).to(dev), (torch.randn(9 * 64, 128, generator=g) * 0.1).to(dev)
+
+    class Noisy(ChapterRouter):
+        def sequence_logits(self, *a, **kw):
+            return -super().sequence_logits(*a, **kw)
+
+    def results(change):
+        layer = _layer(dev, 128, 2, 2, 9, 1, 3, "none")
+        plain = layer(h, bank)[0]
+        change(layer)
+        a = layer(h, bank)[0]
+        layer.fused = False
+        return plain, a, layer(h, bank)[0]
+
+    def subclass(layer):
+        other = Noisy(128, 9, 3).to(dev)
+        other.load_state_dict(layer.router.state_dict())
+        layer.router = other
+
+    def replaced(layer):
+        real = layer.router.sequence_logits
+        layer.router.sequence_logits = lambda *a, **kw: -real(*a, **kw)
+
+    def queries(layer):
+        real = layer.memory_attn._queries
+        layer.memory_attn._queries = lambda *a, **kw: real(*a, **kw) * 2
+
+    for change in (subclass, replaced, queries):
+        plain, a, per_op = results(change)
+        _same(a, per_op, change.__name__)
+        assert not torch.allclose(a, plain, rtol=1e-3)
