@@ -358,6 +358,9 @@ int moc_seq_layer_bwd_ex(const void* h, const void* bank, const void* wr, int wr
  * moc_seq_layer_fwd_ex / _bwd_ex with float32 tensors; dwkv [2*HK*64][d]. */
 int moc_seq_layer_f32_sizes(int64_t B, int64_t L, int64_t d, int H, int HK, int64_t C, int S, int k, int norm,
                             size_t* saved, size_t* scratch);
+/* Whether a training step of these sizes is to run in one call (1) or has reductions long enough to be the
+ * library's (0): a forward alone always may. */
+int moc_seq_layer_f32_trains(int64_t B, int64_t L, int64_t C, int S, int k);
 int moc_seq_layer_f32_fwd(const float* h, const float* bank, const void* wr, int wr_dtype, const float* br,
                           const float* wq, const float* wk, const float* wv, const float* wo, const float* coef,
                           int64_t B, int64_t L, int64_t d, int H, int HK, int64_t C, int S, int k, float routed_scale,

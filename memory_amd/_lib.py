@@ -60,6 +60,7 @@ _SIGS = {
     "moc_decode_step": (_I, [_P, _I64, _I64, _P, _I, _P, _P, _I, _I, _P, _P, _P, _P, _P, _I64, _P, _I, _F, _P, _I64, _P,
                              _SZ, _P, _P, _P]),
     "moc_seq_layer_f32_sizes": (_I, [_I64, _I64, _I64, _I, _I, _I64, _I, _I, _I, _P, _P]),
+    "moc_seq_layer_f32_trains": (_I, [_I64, _I64, _I64, _I, _I]),
     "moc_seq_layer_f32_fwd": (_I, [_P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I, _I, _I64, _I, _I, _F,
                                    _I, _F, _P, _P, _P, _P, _P, _P, _SZ, _P]),
     "moc_seq_layer_f32_bwd": (_I, [_P, _P, _P, _I, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I, _I, _I64, _I, _I, _F, _I,

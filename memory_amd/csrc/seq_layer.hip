@@ -26,6 +26,7 @@
 // event completes costs ~15 us of wake-up besides the wait itself, so the side streams are given
 // work that ends before the main stream reaches the join.
 // Calls on one device must come from one host thread at a time (the events are per device).
+#include <algorithm>
 #include <mutex>
 
 #include "moc_common.h"
@@ -67,10 +68,18 @@ int seq_events(hipEvent_t** out) {
 
 // Multiply-adds of one d x d projection of the tokens plus one K or V projection of the rows up to which
 // the float32 layer runs as one host call on moc_gemm_f32.  A training step against the per-op functions,
-// which need 600 to 850 us of host time at any size: 295 against 693 us at 2 x 128 tokens of d = 256 with
-// 10 chapters (2.7e7), 501 against 853 at 8 x 512 with 56 (5.0e8), 746 against 830 at 8 x 1,024 with 40
-// (7.0e8); past the line the library's larger tiles win, 1,021 against 829 at 8 x 1,024 with 128 (1.1e9).
+// which need 570 to 870 us of host time at any size: 285 against 620-693 us at 2 x 128 tokens of d = 256
+// with 10 chapters (2.7e7), 442 against 571 at 8 x 64 with 129 (5.7e8), 746 against 830 at 8 x 1,024 with
+// 40 (7.0e8); past the line the library's larger tiles win, 1,021 against 829 at 8 x 1,024 with 128
+// (1.1e9).  Forwards alone: 84-162 against 190-350 us below the line (d = 64 to 1,024, 16 to 32,768
+// tokens; 222 against 255 at 131,072 tokens of d = 64), 241 / 220 where both are per-op at 8.7e8.
 constexpr int64_t kSeqF32Work = (int64_t)3 << 28;
+// Tokens, and bank rows, of a training step: the weight gradients reduce over them in one workgroup per 32
+// x 64 outputs, about 0.03 us a token and 0.02 us a row whatever d is.  One call / per-op: 8,192 tokens
+// 534 / 696 us (d = 64), 565 / 801 (128), 667 / 796 (256); 10,983 tokens 819 / 805 (256); 16,384 tokens
+// 909 / 820 (128); 32,768 tokens 1,432 / 857 (64), 1,570 / 846 (128); 8,256 rows 442 / 571 (256); 32,832
+// rows 1,036 / 686 (128).
+constexpr int64_t kSeqF32Reduce = 8192;
 
 inline size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
 
@@ -234,7 +243,7 @@ struct SeqLayout {
 // The float32 layer (moc_seq_layer_f32_*): the reference's small configurations, where a step is some
 // thirty launches of 2 to 20 us each and the host issuing them one autograd function at a time was what it
 // waited for (692 us of host time for 199 us of kernels at 2 x 128 tokens, d = 256; in one call each way
-// 194 us).  One stream: nothing here is long enough to be worth an event.
+// 285 us).  One stream: nothing here is long enough to be worth an event.
 struct SeqF32Layout {
   int64_t B, L, d, C, E, max_u;
   int NS, KV, Lp;
@@ -611,6 +620,10 @@ int moc_seq_layer_f32_sizes(int64_t B, int64_t L, int64_t d, int H, int HK, int6
   *saved = y.saved_bytes;
   *scratch = y.scratch_bytes;
   return MOC_OK;
+}
+
+int moc_seq_layer_f32_trains(int64_t B, int64_t L, int64_t C, int S, int k) {
+  return B * L <= kSeqF32Reduce && std::min(B * (S + k), C) * 64 <= kSeqF32Reduce;
 }
 
 int moc_seq_layer_f32_fwd(const float* h, const float* bank, const void* wr, int wr_dtype, const float* br,

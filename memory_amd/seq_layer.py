@@ -256,6 +256,16 @@ class _SeqRoutedLayer(torch.autograd.Function):
         return dh, dbank, dwr, dbr, dwq, dwk, dwv, dwo, None, None
 
 
+def _trains(*tensors) -> bool:
+    """Whether a backward may follow a call on these tensors (grad mode is off inside a function's forward)."""
+    return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
+
+
+@functools.lru_cache(maxsize=256)
+def _f32_trains(B, Lq, C, S, k) -> bool:
+    return bool(L.query("moc_seq_layer_f32_trains", B, Lq, C, S, k))
+
+
 @functools.lru_cache(maxsize=256)
 def _f32_sizes(B, Lq, d, H, HK, C, S, k, norm):
     """(saved, scratch) buffer bytes of the native float32 layer, or None for shapes outside it."""
@@ -283,6 +293,9 @@ def supported_f32(h, bank, wr, br, wq, wk, wv, wo, *, num_chapters: int, tokens_
         if t is not None and (t.device != h.device or not t.is_contiguous() or t.data_ptr() % 16
                               or (t is not wr and t.dtype != f32)):
             return False
+    if (_trains(h, bank, wr, br, wq, wk, wv, wo)
+            and not _f32_trains(h.shape[0], h.shape[1], num_chapters, num_shared, top_k)):
+        return False
     return _f32_sizes(h.shape[0], h.shape[1], d, num_heads, num_kv_heads, num_chapters, num_shared, top_k,
                       ops.norm_code(norm_type)) is not None
 
@@ -399,9 +412,7 @@ def seq_routed_layer(h, bank, wr, br, wq, wk, wv, wo, *, num_chapters: int, toke
                      num_shared: int, top_k: int, routed_scale: float, num_heads: int, num_kv_heads: int,
                      norm_type: Optional[str] = None, eps: float = 1e-6, coef: Optional[torch.Tensor] = None):
     """(out (B, L, d), logits f32 (B, C), idx int32 (B, k), idx_star int32 (B, S+k), omega f32 (B, S+k))."""
-    # grad mode is read here: it is off inside the function's forward
-    train = torch.is_grad_enabled() and any(t is not None and t.requires_grad
-                                            for t in (h, bank, wr, br, wq, wk, wv, wo))
+    train = _trains(h, bank, wr, br, wq, wk, wv, wo)
     cfg = (int(num_chapters), int(tokens_per_chapter), int(num_shared), int(top_k), float(routed_scale),
            int(num_heads), int(num_kv_heads), ops.norm_code(norm_type), float(eps), train)
     layer = _SeqF32Layer if h.dtype == torch.float32 else _SeqRoutedLayer

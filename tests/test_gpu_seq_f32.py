@@ -230,3 +230,28 @@ def test_f32_layer_asks_the_callers_router(gpu_device):
         plain, a, per_op = results(change)
         _same(a, per_op, change.__name__)
         assert not torch.allclose(a, plain, rtol=1e-3)
+
+
+@pytest.mark.parametrize("B,L,C,k,one_call", [(1, 8192, 5, 2, True), (1, 8193, 5, 2, False), (43, 3, 128, 2, True),
+                                              (44, 3, 129, 2, False)])
+def test_f32_training_step_long_reductions(gpu_device, monkeypatch, B, L, C, k, one_call):
+    """Training steps whose weight gradients reduce over more than 8,192 tokens or bank rows keep the per-op
+    functions, their forwards alone do not; both give the same."""
+    from memory_amd import seq_layer
+    dev = gpu_device
+    layer = _layer(dev, 64, 1, 1, C, 1, k, "none")
+    g = gen(B + L)
+    h, up = torch.randn(B, L, 64, generator=g).to(dev), torch.randn(B, L, 64, generator=g).to(dev)
+    bank = (torch.randn(C * 64, 64, generator=g) * 0.1).to(dev)
+    called = []
+    real = seq_layer.call
+    monkeypatch.setattr(seq_layer, "call", lambda name, *a: (called.append(name), real(name, *a))[1])
+    got = _step(layer, h, bank, up, True)
+    assert called == (["moc_seq_layer_f32_fwd", "moc_seq_layer_f32_bwd"] if one_call else [])
+    called.clear()
+    with torch.no_grad():
+        _same(layer(h, bank, return_losses=False)[0], got[0], "forward alone")
+    assert called == ["moc_seq_layer_f32_fwd"]
+    want = _step(layer, h, bank, up, False)
+    for n in want[2]:
+        _same(got[2][n], want[2][n], n)
