@@ -22,8 +22,6 @@
 // K and V blocks (both [key][dim]) are double-buffered in
 // LDS; the V^T operand is read from the V tile with the transposing LDS read, whose lane
 // order is the key order of the P~^T fragments.
-#include <math.h>
-
 #include "moc_common.h"
 
 namespace moc {
@@ -448,26 +446,34 @@ __global__ __launch_bounds__(256) void xattn_weights_kernel(
 
 using namespace moc;
 
-// The loop over the slots is a serial chain, ~1.15 us (bf16; f32 ~6) a slot at low occupancy, and a
-// launch has one workgroup per (sequence, head, 128 queries), a "tile"; three fit a CU.  Splitting the
-// slots n ways costs a merge launch (~5 us) and its f32 partial rows (~0.016 us per tile and split,
-// written and read): n at the minimum of chain + partial rows, while n tiles fit the chip, and only
-// where the sum is smaller.  Measured (forward; dQ is alike), 65 slots: 48 tiles 76 -> 27 us, 96 tiles
-// 76 -> 35, 192 tiles 78 -> 54, 288 tiles 96 -> 81, 384 tiles 98 -> 86; 17 slots: 32 tiles 23 -> 17,
-// 384 tiles 32 -> 39 (not split); the plain minimum chain length (one slot a split) was slower
-// everywhere (48 tiles 42 us).
+// The loop over the slots is a serial chain, and a launch has one workgroup per (sequence, head, 128
+// queries), a "tile".  A slot takes the longer the more workgroups a CU holds at once, at most three: bf16
+// ~1.15 / 1.45 / 2.1 us; f32 ~6 us each, as if one after another (its registers fill a CU).  Splitting the
+// slots n ways costs a merge launch (~5 us, ~0.2 a split) and f32 partial rows (~0.016 us per tile
+// and split, written and read).  n is the one of least sum; 1, not split, has the chain alone.  Measured,
+// unsplit -> split, forward / dQ, us:
+//   bf16 65 slots:  48 tiles 72 -> 29 / 65 -> 25, 192 tiles 73 -> 52 / 66 -> 50, 384 tiles 95 -> 78 / 93 -> 84
+//        64 slots: 128 tiles 71 -> 41 / 64 -> 40, 256 tiles 71 -> 62 / 65 -> 62
+//        33 slots:  64 tiles 38 -> 23 / 35 -> 19, 256 tiles at three splits 39 -> 44 / 36 -> 42 (not split)
+//        17 slots:  48 tiles 22 -> 17 / 20 -> 14;  9 slots: 24 tiles 13 -> 13 / 13 -> 11
+//   f32  65 slots:  48 tiles 341 -> 84 / 441 -> 99, 192 tiles 342 -> 256 / 442 -> 357, 384 tiles 608 -> 488 /
+//        881 -> 694; 64 slots: 256 tiles at three splits 337 -> 328 / 437 -> 462 (not split)
 int moc::xattn_splits(int dtype, int64_t B, int64_t L, int H, int NS) {
   const int64_t tiles = B * H * ((L + 127) / 128);
   if (tiles <= 0 || NS <= 1) return 1;
-  const double slot = dtype == MOC_F32 ? 6.0 : 1.15, tile = 0.016;
-  int64_t n = kXattnWgs / tiles;
-  const int64_t best = (int64_t)(sqrt(slot * NS / (tile * (double)tiles)) + 0.5);
-  if (n > best) n = best;
-  if (n > NS) n = NS;
-  if (n < 2) return 1;
-  const int64_t per = (NS + n - 1) / n;
-  n = (NS + per - 1) / per;
-  return slot * (double)(NS - per) > 5.0 + tile * (double)(n * tiles) ? (int)n : 1;
+  auto chain = [&](int64_t n) {
+    const int64_t per_cu = (tiles * n + 255) / 256;
+    const double slot = dtype == MOC_F32 ? 6.0 * per_cu : per_cu == 1 ? 1.15 : per_cu == 2 ? 1.45 : 2.1;
+    return slot * (double)((NS + n - 1) / n);
+  };
+  int64_t best = 1;
+  double least = chain(1);
+  for (int64_t n = 2; n <= NS && n * tiles <= kXattnWgs; ++n) {
+    const double cost = 5.0 + 0.2 * (double)n + chain(n) + 0.016 * (double)(n * tiles);
+    if (cost < least) least = cost, best = n;
+  }
+  const int64_t per = (NS + best - 1) / best;
+  return (int)((NS + per - 1) / per);
 }
 
 extern "C" {
