@@ -204,6 +204,10 @@ __global__ __launch_bounds__(256) void plan_place_kernel(const int32_t* __restri
 constexpr int kPlanSmallP = 8;
 constexpr int kPlanSmallE = 1024 * kPlanSmallP;
 constexpr int kPlanSmallC = 8192;
+// At most 64 chapters crowd every block of 1,024 edges, which one workgroup ranks block after block, about
+// 6 us each: up to here it is level with the four launches (9 chapters: 4,096 edges 39.3 -> 26.3 us, 6,000
+// edges 40.6 -> 38.8, 8,192 edges 41.1 -> 49.6; 33 chapters: 22.8 -> 14.8, 23.5 -> 22.6, 23.7 -> 27.9).
+constexpr int kPlanCrowdedC = 64, kPlanCrowdedE = 6144;
 
 __device__ __forceinline__ int wave_incl_scan(int v) {
   const int lane = threadIdx.x & 63;
@@ -351,7 +355,7 @@ size_t plan_workspace_bytes(int64_t E, int64_t C) {
 // The plan's kernels on a given workspace (every word of it is written before it is read).
 int plan_launch(const int32_t* chap, int64_t E, int64_t C, void* workspace, int32_t* uniq, int32_t* n_uniq,
                 int32_t* edge_u, int32_t* csr_off, int32_t* csr_edge, hipStream_t stream) {
-  if (E <= kPlanSmallE && C <= kPlanSmallC) {
+  if (E <= (C <= kPlanCrowdedC ? kPlanCrowdedE : kPlanSmallE) && C <= kPlanSmallC) {
     const size_t lds = 3 * (size_t)C * sizeof(int32_t);
     if (E <= 1024)
       hipLaunchKernelGGL(plan_small_kernel<1>, dim3(1), dim3(1024), lds, stream, chap, E, C, uniq, n_uniq, edge_u,

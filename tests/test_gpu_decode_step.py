@@ -12,7 +12,7 @@ BF = torch.bfloat16
 
 
 @pytest.mark.parametrize("E,C", [(1023, 700), (1024, 33), (1025, 1), (2048, 8192), (2049, 300), (4095, 4097), (4096, 8),
-                                 (4097, 50), (8191, 8192), (8192, 900), (8193, 60)])
+                                 (4097, 50), (8191, 8192), (8192, 900), (8193, 60), (6144, 64), (6145, 64), (8192, 65)])
 def test_small_plan(gpu_device, E, C):
     from memory_amd import ops
     ids = torch.randint(0, C, (E,), generator=gen(E + C), dtype=torch.int32)
