@@ -51,3 +51,29 @@ def test_few_chapter_projection(gpu_device, nsel, C, N, K, gather):
     x = bank if gather else bank[rows]
     y = ops.chapter_project(x.to(dev), plan, w.to(dev), gather=gather)
     assert_parity(y[: nsel * 64], bank[rows].double() @ w.double().t(), torch.bfloat16, "projection")
+
+
+@pytest.mark.parametrize("nsel,C,N,K", [(1, 7, 768, 512), (85, 90, 768, 256), (170, 180, 768, 256), (171, 180, 768, 256),
+                                         (84, 90, 1536, 512), (86, 90, 1536, 512), (9, 12, 512, 256)])
+@pytest.mark.parametrize("bank_rows", [True, False])
+def test_few_chapter_input_gradient(gpu_device, nsel, C, N, K, bank_rows):
+    """moc_chapter_dx on both sides of its line between 128 x 256 and 256 x 384 tiles ((chapters + 1) / 2 *
+    N / 256 against 256 workgroups): 170 chapters are the last of the narrow side at N = 768, 84 at 1,536."""
+    from memory_amd import ops
+    dev = gpu_device
+    g = gen(nsel + N)
+    ids = torch.randperm(C, generator=g)[:nsel].to(torch.int32)
+    plan = ops.chapter_plan(ids.to(dev), C)
+    dkv = torch.randn(nsel * 64, K, generator=g).bfloat16()          # one edge per chapter, in edge order
+    wt = (torch.randn(N, K, generator=g) * 0.05).bfloat16()          # [Wk; Wv]^T
+    want = dkv.double() @ wt.double().t()                            # edge order
+    out = torch.full(((C if bank_rows else nsel) * 64, N), float("nan"), device=dev, dtype=torch.bfloat16)
+    ops.chapter_dx(dkv.to(dev), dkv.to(dev), plan.uniq, plan.n_uniq, plan.max_u, plan.csr_off, plan.csr_edge, wt.to(dev),
+                   out, bank_rows=bank_rows)
+    place = ids.long() if bank_rows else ids.long().argsort().argsort()
+    rows = (place.unsqueeze(-1) * 64 + torch.arange(64)).reshape(-1)
+    assert_parity(out.cpu()[rows], want, torch.bfloat16, "dx")
+    if bank_rows:
+        rest = torch.ones(C, dtype=torch.bool)
+        rest[ids.long()] = False
+        assert bool(torch.isnan(out.cpu().view(C, -1)[rest]).all())

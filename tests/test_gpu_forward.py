@@ -181,12 +181,13 @@ def test_chapter_plan_skips_out_of_range(dev):
     assert plan.csr_edge.cpu().tolist()[:6] == [0, 6, 1, 4, 2, 7]
 
 
-def test_chapter_plan_general_path_skips_out_of_range(dev):
-    """More than 1,024 edges (the multi-block path): ids outside [0, C) are skipped, the rest
-    planned as the stable (chapter, edge) order."""
+@pytest.mark.parametrize("rows", [100, 400])
+def test_chapter_plan_general_path_skips_out_of_range(dev, rows):
+    """3,000 edges (one workgroup, blocks of 1,024) and 12,000 (more than 8,192: the multi-block path): ids
+    outside [0, C) are skipped, the rest planned as the stable (chapter, edge) order."""
     g = np.random.default_rng(7)
     C = 50
-    chap = g.integers(-3, C + 3, size=(100, 30)).astype(np.int32)
+    chap = g.integers(-3, C + 3, size=(rows, 30)).astype(np.int32)
     plan = _ops().chapter_plan(torch.from_numpy(chap).to(dev), C)
     flat = chap.reshape(-1)
     ok = (flat >= 0) & (flat < C)

@@ -50,7 +50,7 @@ def _layer(dev, dtype, Wr, br, Wq, Wk, Wv, Wo, normalize, strategy="sequence", w
     return layer
 
 
-@pytest.mark.parametrize("dtype,fused", [(torch.float32, "per-op"), (torch.bfloat16, "native"),
+@pytest.mark.parametrize("dtype,fused", [(torch.float32, "per-op"), (torch.float32, "native"), (torch.bfloat16, "native"),
                                          (torch.bfloat16, "python"), (torch.bfloat16, "per-op")])
 @pytest.mark.parametrize("normalize,strategy,window", [(False, "sequence", None), (True, "sequence", None),
                                                        (False, "sequence-rolling", 16)])
@@ -58,8 +58,12 @@ def _layer(dev, dtype, Wr, br, Wq, Wk, Wv, Wo, normalize, strategy="sequence", w
 def test_config1_layer_forward_backward(gpu_device, monkeypatch, dtype, fused, normalize, strategy, window, Lq):
     """bf16 runs the whole-layer autograd function (memory_amd.seq_layer) with its native
     schedule (moc_seq_layer_fwd_ex / _bwd_ex, a normalised bank included) and
-    with the Python-scheduled one, and the per-op functions; fp32 always takes the per-op path."""
+    with the Python-scheduled one, and the per-op functions; fp32 of these sizes runs as one host call each
+    way (moc_seq_layer_f32_fwd / _bwd) and as the per-op functions."""
     from memory_amd import seq_layer
+    called = []
+    real = seq_layer.call
+    monkeypatch.setattr(seq_layer, "call", lambda name, *a: (called.append(name), real(name, *a))[1])
     print(f"config1 layer dtype={dtype} fused={fused} normalize={normalize} strategy={strategy} L={Lq}", flush=True)
     monkeypatch.setattr(seq_layer, "NATIVE", fused == "native")
     dev = gpu_device
@@ -76,6 +80,9 @@ def test_config1_layer_forward_backward(gpu_device, monkeypatch, dtype, fused, n
     out, _ = layer(hg, bg, return_losses=False)
     dO = torch.randn(out.shape, generator=torch.Generator().manual_seed(1))
     (out.float() * dO.to(dev)).sum().backward()
+    kind = {torch.float32: "moc_seq_layer_f32_{}", torch.bfloat16: "moc_seq_layer_{}_ex"}[dtype]
+    assert [n for n in called if n.startswith("moc_seq_layer")] == \
+        ([kind.format("fwd"), kind.format("bwd")] if fused == "native" else [])
 
     leaves = [t.double().clone().requires_grad_(True) for t in (h, bank, Wr, br, Wq, Wk, Wv, Wo)]
     if dtype != torch.float32:   # reference sees the same rounded activations / weights

@@ -1,7 +1,7 @@
 """moc_chapter_plan_noalloc (the plan on the library's fixed device scratch array, no
-allocation) against moc_chapter_plan with a caller workspace: two calls in a row, the second on a
-smaller input, both large enough for the multi-kernel path that uses the workspace; outputs are
-integer and must be identical.  A plan larger than the scratch array is refused on the host."""
+allocation) against moc_chapter_plan with a caller workspace: calls in a row on smaller inputs, the
+first two large enough for the multi-kernel path that uses the workspace (more than 8,192 edges), the
+third on the one-workgroup path that does not; outputs are integer and must be identical.  A plan larger than the scratch array is refused on the host."""
 
 import pytest
 import torch
@@ -31,7 +31,7 @@ def test_noalloc_plan_matches_workspace_plan(gpu_device):
     from memory_amd import _lib as L
     L.lib()
     g = torch.Generator().manual_seed(0)
-    for E, C in ((200_000, 4097), (5_000, 1000)):          # the second call smaller than the first
+    for E, C in ((200_000, 4097), (20_000, 1000), (5_000, 1000)):      # each call smaller than the one before
         print(f"noalloc plan E={E} C={C}", flush=True)
         chap = torch.randint(-3, C + 3, (E,), generator=g, dtype=torch.int32)   # a few skipped edges
         chap_d = chap.to(gpu_device)
