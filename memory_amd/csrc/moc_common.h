@@ -336,6 +336,25 @@ __device__ __forceinline__ float quad_sum(float v) {
   v += __shfl_xor(v, 32, 64);
   return v;
 }
+// max over the lanes {l, l^16, l^32, l^48} (the four row groups of a 16x16 accumulator column)
+// with the gfx950 row-swap permutes.  v_permlane16_swap_b32 a, b swaps the odd 16-lane rows of
+// a with the even rows of b (v_permlane32_swap_b32: the upper 32 lanes of a with the lower 32 of
+// b); from two copies of v it leaves v's partner-row values in one of the copies.
+__device__ __forceinline__ float quad_max_pl(float v) {
+  float a = v, b = v;
+  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+  float c = fmax_fast(a, b), d = c;
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(c), "+v"(d));
+  return fmax_fast(c, d);
+}
+// the sum alike (the same bits as quad_sum)
+__device__ __forceinline__ float quad_sum_pl(float v) {
+  float a = v, b = v;
+  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+  float c = a + b, d = c;
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(c), "+v"(d));
+  return c + d;
+}
 
 inline int dtype_size(int dt) { return dt == MOC_F32 ? 4 : (dt == MOC_BF16 ? 2 : 0); }
 

@@ -17,7 +17,7 @@
 //
 // Measured at 16,384 tokens, 16 query heads on one kv head, 8 blocks of 128 among 512 per sequence
 // (1,024 units of ~2,048 rows; 206 GFLOP forward + backward), against the 64-key units before:
-// forward 289 -> 145 us, backward 531 -> 290 us, the combines 324 -> 145 us.  What bounds them now:
+// forward 289 -> 153 us, backward 531 -> 310 us, the combines 324 -> 145 us.  What bounds them now:
 // the forward the partial rows and gathered q rows (537 MB, 3.7 TB/s) beside its softmax VALU work;
 // the backward MFMA + VALU issue (~180 us) and the transposing LDS reads (~170 us), partly
 // overlapped at two waves per SIMD.  32-row blocks took 410 us against 339 (two barriers per 32
@@ -149,9 +149,9 @@ __global__ __launch_bounds__(256) void sparse_rows_fwd_kernel(
     // 64 keys at a time, each with its own maximum: bf16 rounds P = 2^(s - max) to 8 bits, exactly for
     // the maximum's own key alone, so one maximum over 128 keys put 128-key units at 1.018 times the
     // error of 64-key ones (outputs, 8 blocks of 128; 1.001 so, the one rounding of a partial row in
-    // place of two).  The halves are scaled to each other in f32: 590 -> 598 us for the call above,
-    // forward and backward.  (Row sums of the rounded P on the matrix cores: 613 us, and dK / dV
-    // 1.0006 times as far off.)
+    // place of two).  The halves are scaled to each other in f32.  Cross-lane maxima and sums go by row
+    // swaps: the kernel 150 -> 161 us with the second maximum, 153 with them in place of LDS permutes.
+    // (Row sums of the rounded P on the matrix cores: 15 us more, and dK / dV 1.0006 times as far off.)
     if (KT > 64 && un.nk < KT) {   // a half last block: its missing keys take no part
 #pragma unroll
       for (int kb = 4; kb < NKB; ++kb) st[kb] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
@@ -165,7 +165,7 @@ __global__ __launch_bounds__(256) void sparse_rows_fwd_kernel(
       for (int kb = 4 * h; kb < 4 * h + 4; ++kb)
 #pragma unroll
         for (int x = 0; x < 4; ++x) mx = fmax_fast(mx, st[kb][x]);
-      const float mh = quad_max(mx) * scale_log2;   // scale > 0 (host check)
+      const float mh = quad_max_pl(mx) * scale_log2;   // scale > 0 (host check)
       const float ref = mh > -INFINITY || KT == 64 ? mh : 0.f;   // a half of -inf scores adds nothing
       float ps = 0.f;
       bf16x8 pf[2];
@@ -177,7 +177,7 @@ __global__ __launch_bounds__(256) void sparse_rows_fwd_kernel(
           ps += p;
           pf[kb >> 1][4 * (kb & 1) + x] = (bf16)p;
         }
-      const float lh = quad_sum(ps);
+      const float lh = quad_sum_pl(ps);
       f32x4 oh[4];
 #pragma unroll
       for (int db = 0; db < 4; ++db) oh[db] = f32x4{0.f, 0.f, 0.f, 0.f};

@@ -37,17 +37,6 @@ constexpr float kRescaleSlack = 8.f;
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ float max3f(float a, float b, float c) { return fmax_fast(fmax_fast(a, b), c); }
-// max over the lanes {l, l^16, l^32, l^48} (the four row groups of a 16x16 accumulator column)
-// with the gfx950 row-swap permutes.  v_permlane16_swap_b32 a, b swaps the odd 16-lane rows of
-// a with the even rows of b (v_permlane32_swap_b32: the upper 32 lanes of a with the lower 32 of
-// b); from two copies of v it leaves v's partner-row values in one of the copies.
-__device__ __forceinline__ float quad_max_pl(float v) {
-  float a = v, b = v;
-  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
-  float c = fmax_fast(a, b), d = c;
-  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(c), "+v"(d));
-  return fmax_fast(c, d);
-}
 
 // One 16-byte-per-lane LDS DMA (buffer_load_dwordx4 ... lds): lane l's 16 bytes at voff + soff
 // of the buffer land at LDS address m0 + 16 l.  The wait on these loads is an explicit vmcnt(0).
