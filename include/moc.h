@@ -656,7 +656,8 @@ int moc_sparse_dw(const float* src, const float* w, const int32_t* edge_u, int m
  * workgroups (f32 partials in the workspace, summed in a fixed order). */
 /* KT for these arguments (ntok = ntok'; S slots of block_size keys; mode as moc_sparse_combine), or
  * 0 when the packed form does not apply (too many ids for the plan or rows for its indices; a
- * per-block softmax over other blocks than 64 and 128 keys). */
+ * per-block softmax over other blocks than 64 and 128 keys; partial rows past 16 GiB where a head, or a
+ * slot, at a time holds less). */
 int moc_sparse_packed_block(int dtype, int64_t ntok, int G, int64_t S, int64_t Bk, int64_t Tk, int HK, int block_size,
                             int mode, float scale);
 /* out i32 [ntok * HK * S]: plan ids of idx [ntok][heads][S] (4- or 8-byte ids, heads >= HK); -1

@@ -18,7 +18,7 @@
 // Measured at 16,384 tokens, 16 query heads on one kv head, 8 blocks of 128 among 512 per sequence
 // (1,024 units of ~2,048 rows; 206 GFLOP forward + backward), against the 64-key units before:
 // forward 289 -> 153 us, backward 531 -> 310 us, the combines 324 -> 145 us.  What bounds them now:
-// the forward the partial rows and gathered q rows (537 MB, 3.7 TB/s) beside its softmax VALU work;
+// the forward the partial rows and gathered q rows (537 MB, 3.5 TB/s) beside its softmax VALU work;
 // the backward MFMA + VALU issue (~180 us) and the transposing LDS reads (~170 us), partly
 // overlapped at two waves per SIMD.  32-row blocks took 410 us against 339 (two barriers per 32
 // rows), division by run-time S and G 50 us more; leaving the dQ row stores in flight over the wait for the
@@ -676,6 +676,10 @@ constexpr int64_t kSrMinRows = 48;
 // A 128-key block as one unit instead of two 64-key ones wins from fewer rows on: 16 rows
 // 189 / 205 us, 48 rows 122 / 136 (G = 1) and 252 / 322 (G = 4), 1,024 rows 170 / 316 (G = 16).
 constexpr int64_t kSrMinRows128 = 16;
+// Bytes of partial rows up to which all kv heads (and, per-block mixture, all slots) run at once: per-head
+// segments hold one head's at a time, which a call of a million tokens with 64 slots on 16 kv heads needs
+// (8 GiB a head, 128 GiB packed, in the forward and again in the backward).
+constexpr int64_t kSrPartBytes = (int64_t)16 << 30;
 bool sr_many_rows(int64_t rows, int64_t max_u, int64_t least) { return max_u > 0 && rows >= least * max_u; }
 bool sr_use_rows(int dtype, int KT, int64_t rows, int64_t max_u, float scale) {
   return dtype == MOC_BF16 && (KT == 128 || (scale > 0.f && sr_many_rows(rows, max_u, kSrMinRows)));
@@ -729,7 +733,9 @@ int moc_sparse_packed_block(int dtype, int64_t ntok, int G, int64_t S, int64_t B
   const int m = block_size / 64;
   auto fits = [&](int kt) {
     const int64_t ids = Bk * ((Tk + kt - 1) / kt) * HK, edges = ntok * S * (block_size / kt);
-    return ids <= kSrMaxIds && edges * G < ((int64_t)1 << 31) && ntok * G * 256 < ((int64_t)1 << 32) - 16;
+    const int64_t bytes = edges * G * kSrDh * (dtype == MOC_F32 ? 4 : 2);
+    return ids <= kSrMaxIds && edges * G < ((int64_t)1 << 31) && ntok * G * 256 < ((int64_t)1 << 32) - 16 &&
+           (bytes <= kSrPartBytes || (HK == 1 && mode != 0));   // (one head, joint: its segment holds them too)
   };
   // A block's own softmax (mode 0) spans one unit at 128 keys and is otherwise the caller's one
   // call per slot; a joint softmax over 128-key units halves the partial rows, at a unit's cost in

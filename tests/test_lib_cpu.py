@@ -123,3 +123,15 @@ def test_slots_are_split_where_that_is_faster(libpath, dtype, B, L, H, NS, split
     """One workgroup per CU already, and as many again do not run beside it at its speed: 256 tiles of 33 slots
     in bf16, or of 64 in float32, were slower split (44 against 39 us, dQ 462 against 437)."""
     assert (_lib.query("moc_xattn_split_workspace", dtype, B, L, H, NS) > 0) == split
+
+
+@pytest.mark.parametrize("ntok,G,S,HK,block,mode,want", [
+    (1 << 20, 1, 64, 16, 64, 1, 64),       # 8 GiB of partial rows for all heads
+    (1 << 21, 1, 65, 16, 64, 1, 0),        # past 16 GiB: a head at a time
+    ((1 << 20) - 1, 16, 10, 1, 64, 1, 64), # one head: its segment holds as much
+    (1 << 18, 16, 33, 1, 128, 0, 0),       # the per-block mixture: a slot at a time
+    (1 << 18, 16, 32, 1, 128, 0, 128),
+])
+def test_packed_partial_rows_are_bounded(libpath, ntok, G, S, HK, block, mode, want):
+    """All kv heads at once while their partial rows (bf16, 128 bytes each) fit 16 GiB."""
+    assert _lib.query("moc_sparse_packed_block", _lib.MOC_BF16, ntok, G, S, 1, 8192 // HK, HK, block, mode, 0.125) == want
