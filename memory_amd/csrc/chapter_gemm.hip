@@ -864,8 +864,14 @@ int cg_check(const char* who, int64_t ldx, int N, int K, int64_t max_u, int64_t 
 }
 
 // Few chapters (a prompt's own, a dense memory): 128-row x 256-feature tiles, two k-stages ahead, where
-// they fit one round of the grid.  A round of them is half as long as one of the wide tiles (65 chapters,
-// 1,536 features, K = 768: 198 tiles in 20 us against 66 tiles of 256 x 384 in 33 us).
+// they fit one round of the grid.  A round of them is about half as long as one of the wide tiles, so just
+// past the line, at two rounds, the wide ones are level.  Projection, narrow / wide, us:
+//   1,536 features, K = 768: 1 chapter 13.4 / 24.9, 65 (198 tiles) 18.0 / 31.4;   K = 256: 65 10.0 / 17.0
+//     768 features, K = 768: 17 14.3 / 28.0, 129 (195 tiles) 17.4 / 30.4;         K = 1,536: 129 28.8 / 50.7
+//     512 features, K = 512: 171 12.8 / 17.3, 257 (258 tiles, past it) 21.8 (dX) / 18.9;  K = 2,048: 171 34 / 47
+//   2,048 features, K = 1,024: 17 19.5 / 26.7, 65 (264 tiles, past it) 36.4 (dX) / 29.8
+// (the wide kernel of N % 384 != 0 is 256 x 256; dX at such N has no wide form and keeps the narrow one).
+// dX at N % 384 == 0 is alike: 1,536 x 768, 65 chapters 17.9 / 31.2.
 bool cg_narrow(int64_t max_u, int N) { return (max_u + 1) / 2 * (N / 256) <= cg_grid(); }
 
 // workgroups per output tile of the weight gradients: fill `budget` CUs (256: the chip), but give

@@ -135,6 +135,9 @@ int moc_decode_step(const void* x, int64_t B, int64_t d, const void* wq, int H, 
   return moc_linear_rows(ws + y.a, B, (int64_t)H * 64, wo, N, MOC_BF16, out, stream);
 }
 
+// 9 to 68 slots and 16,384 rows are what the one combine kernel with a grouped form takes
+// (sparse_combine_small_kernel): fewer slots and more rows have combines of their own, which would need one
+// too, and run a chain of kernels per layer.
 int moc_decode_step_group(const moc_decode_layer* layers, int n, int64_t B, int64_t d, int H, int HK, int T, int NS,
                           float scale, int64_t N, size_t workspace_bytes, hipStream_t stream) {
   MOC_REQUIRE(layers && n > 0, MOC_ERR_ARG, "moc_decode_step_group: no layers");

@@ -117,9 +117,10 @@ extern "C" {
 
 int moc_gemm_f32_takes(int ta, int tb, int64_t M, int64_t N, int64_t K) {
   // us here / hipBLASLt (graph replays, forward / input-gradient / weight-gradient form alike): 256^3
-  // 6.5 / 63, 640 x 512 x 256 6.5 / 6.3, 768 x 256 x 512 10 / 6.5, 512 x 1024 x 1024 18 / 12, 256 x 256 x
-  // 2048 29 / 9; a library call also costs ~20 us more on the host, which is what a step of such sizes
-  // waits for.
+  // 6.5 / 63, 640 x 512 x 256 7 / 6.3, 512 x 512 x 256 6.6 / 5.6, 8,192 x 64 x 64 5 / 4.5, 320 x 256 x 512
+  // 10 / 6.5, 64 x 64 x 512 10 / 10.7, 512 x 1024 x 1024 18 / 12, 256 x 256 x 2048 29 / 9.  From the host a
+  // call of either is longer than that, 8 us here against 19 to 20 of the library, which is what a step of
+  // such sizes waits for: calls back to back take 8 to 11 us here and 19 to 20 there at every one of them.
   constexpr int64_t kMaxWork = 100000000, kMaxK = 512;
   if (M <= 0 || N <= 0 || K <= 0 || N % 4 != 0 || M > (1 << 20) || N > (1 << 20) || K > (1 << 20)) return 0;
   if ((!ta || tb) && K % 8 != 0) return 0;   // an operand with a contiguous reduction is read 8 at a time

@@ -380,8 +380,9 @@ class _Linear(torch.autograd.Function):
     """y = x W^T (bias-free nn.Linear of the memory layer's q_proj / o_proj,
     memory_transformer/memory_attention.py:140-143, :241 and :456).  The weight gradient
     dW = dy^T x runs on the split-row MFMA kernel (the token dimension is long and the output
-    small); forward and dx stay on hipBLASLt (at 8,192 x 768 x 768 it beats the chapter GEMM,
-    whose 192 tiles fill one round of the chip), few rows on the few-row kernel."""
+    small); bf16 forward and dx stay on hipBLASLt (at 8,192 x 768 x 768 it beats the chapter GEMM,
+    whose 192 tiles fill one round of the chip), few rows on the few-row kernel; float32 products of
+    small sizes run on moc_gemm_f32 (matmul2d), larger ones on the library."""
 
     @staticmethod
     def forward(ctx, x, w):

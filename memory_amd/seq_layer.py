@@ -32,7 +32,8 @@ requires a gradient) leaves out what only the backward reads, and its buffer is 
 
 The float32 layer at the reference's small sizes runs as one host call each way on one stream
 (moc_seq_layer_f32_fwd / _bwd): its launches take a few microseconds each and the step is what the
-host needs to issue them.
+host needs to issue them.  Training steps that reduce over many tokens or bank rows, and backwards that
+are themselves recorded, go through the per-op functions.
 """
 
 from __future__ import annotations
