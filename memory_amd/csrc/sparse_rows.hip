@@ -151,7 +151,8 @@ __global__ __launch_bounds__(256) void sparse_rows_fwd_kernel(
     // error of 64-key ones (outputs, 8 blocks of 128; 1.001 so, the one rounding of a partial row in
     // place of two).  The halves are scaled to each other in f32.  Cross-lane maxima and sums go by row
     // swaps: the kernel 150 -> 161 us with the second maximum, 153 with them in place of LDS permutes.
-    // (Row sums of the rounded P on the matrix cores: 15 us more, and dK / dV 1.0006 times as far off.)
+    // (Row sums of the rounded P: for the partial rows alone 0.998 of that error, but 169 us, by dot products
+    // or on the matrix cores; in lse as well dK / dV come out 1.0006 times as far off.)
     if (KT > 64 && un.nk < KT) {   // a half last block: its missing keys take no part
 #pragma unroll
       for (int kb = 4; kb < NKB; ++kb) st[kb] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
